@@ -213,7 +213,7 @@ inline std::vector<int> radix_plan4(int L) {
     int a, b;
     std::vector<int> big;
     factor_or_fail(L, a, b, big);
-    const int first = a >= 5 ? 4 : 2;
+    const int first = a >= 4 ? 4 : 2;
     a -= first == 4 ? 2 : 1;
     const int last = a >= 2 ? 4 : 2;
     a -= last == 4 ? 2 : 1;
