@@ -403,6 +403,146 @@ void gspo_run_fused(qdx_prop *p, R *psi, const R *psi0, long first, long nsteps,
     }
 }
 
+// --- short 1D lines: dense kinetic operator (qdx_dense.hip) ------------------
+
+// qdx_ctx_set_line_points 4 or 8 asks for the line-transform kernels
+bool dense_on(const qdx_prop *p) { return p->dense && p->ctx->line_ppt == 0; }
+
+// The circulant matrix t(i - j) = 1/N sum_k f(T_k) cos(2 pi k (i - j) / N) of
+// f(T) for every state (T_k = T_{N-k}, f real), as the dense kernels read it:
+// per state and parity (t(d) +- t(d + N/2)) / 2 for d < N.  Summed in
+// extended precision; a state without a kinetic term has f(0).
+std::vector<double> circulant_tables(const std::vector<std::vector<double>> &Tk, int N,
+                                     const std::function<long double(double)> &f) {
+    std::vector<long double> cs(N), w(N / 2 + 1), t(N);
+    for (int q = 0; q < N; ++q) cs[q] = cosl(2.0L * 3.14159265358979323846264338327950288L * q / N);
+    std::vector<double> tab;
+    for (const std::vector<double> &T : Tk) {
+        for (int k = 0; k <= N / 2; ++k) w[k] = f(T[k]) * (k == 0 || k == N / 2 ? 1.0L : 2.0L) / N;
+        for (int d = 0; d <= N / 2; ++d) {
+            long double a = 0;
+            for (int k = 0, q = 0; k <= N / 2; ++k) {
+                a += w[k] * cs[q];
+                q += d;
+                if (q >= N) q -= N;
+            }
+            t[d] = a;
+            if (d > 0) t[N - d] = a;
+        }
+        for (int par = 0; par < 2; ++par)
+            for (int d = 0; d < N; ++d) {
+                const long double u = t[(d + N / 2) % N];
+                tab.push_back((double)(0.5L * (par ? t[d] - u : t[d] + u)));
+            }
+    }
+    return tab;
+}
+
+// the per-state kinetic tables T_k of a 1D operator
+std::vector<std::vector<double>> kinetic_values(const qdx_ham *op) {
+    const int N = op->grid.N[0];
+    std::vector<std::vector<double>> T(op->S, std::vector<double>(N, 0.0));
+    for (int s = 0; s < op->S; ++s)
+        if (op->dev.h64.tk[s][0])
+            HIPCHK(hipMemcpy(T[s].data(), op->dev.h64.tk[s][0], N * sizeof(double), hipMemcpyDeviceToHost));
+    return T;
+}
+
+// host arrays that copies in flight on a stream still read
+struct StreamKeep {
+    hipStream_t s;
+    std::vector<std::vector<double>> v;
+    ~StreamKeep() {
+        if (!v.empty()) (void)hipStreamSynchronize(s);
+    }
+};
+
+// Steps first .. first + nsteps - 1 of a propagation that keeps to dense
+// lines.  obs (nullable): observables before each step, 4 S doubles per step;
+// orders (nullable): H applications per step (device arrays).  The host
+// arrays of fields go to `keep`.
+// When the clock leaves the field, the steps before run and the error is
+// raised then, as step by step.
+void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
+               StreamKeep &keep) {
+    qdx_ctx *ctx = p->ctx;
+    const int S = p->S, N = p->grid.N[0];
+    const bool cheby = p->kind == qdx_prop::CHEBY;
+    XGroupDev<double> pre, post;
+    qdx_ham *fop = nullptr;   // the operator whose field changes with the clock
+    bool coupled = false;
+    if (!cheby) {
+        const auto seq = gspo_sequence(p);
+        size_t kpos = 0;
+        for (size_t i = 0; i < seq.size(); ++i) {
+            if (seq[i].kinetic) kpos = i;
+            else if (seq[i].op->time_dependent()) fop = seq[i].op;
+        }
+        pre.n = post.n = 0;
+        for (size_t i = 0; i < kpos; ++i) pre.op[pre.n++] = xsplit<double>(p, seq[i].op, seq[i].tau, first);
+        for (size_t i = kpos + 1; i < seq.size(); ++i) post.op[post.n++] = xsplit<double>(p, seq[i].op, seq[i].tau, first);
+        for (int i = 0; i < pre.n; ++i) coupled = coupled || pre.op[i].coupled;
+    } else if (p->ham->time_dependent()) {
+        fop = p->ham;
+    }
+    const int nf = cheby ? S * S : 1;   // field values per step
+    // a launch runs at most 2^16 orders (2^14 split-operator steps): tens of
+    // milliseconds
+    const long most = cheby ? std::max(1L, 65536L / std::max(p->k_launch, 1)) : 16384L;
+    for (long i = 0; i < nsteps;) {
+        long n = std::min(most, nsteps - i);
+        DenseRun a;
+        a.N = N;
+        a.psi0 = psi0;
+        a.obs = obs ? obs + (size_t)i * 4 * S : nullptr;
+        a.orders = orders ? orders + i : nullptr;
+        std::function<void()> late;   // raises the error of the step after the last valid one
+        if (fop) {
+            std::vector<double> f;
+            HamDev<double> h;
+            for (long k = 0; k < n; ++k) {
+                try {
+                    fop->set_fields(h, first + i + k);
+                } catch (const QdxError &e) {
+                    if (k == 0) throw;
+                    const QdxError err = e;
+                    late = [err] { throw err; };
+                    n = k;
+                    break;
+                }
+                for (int c = 0; c < nf; ++c) f.push_back(h.Edip[cheby ? c / S : 0][cheby ? c % S : 0]);
+            }
+            if (n == 1) {
+                std::copy(f.begin(), f.end(), a.field0);
+            } else {
+                if (p->dfields.bytes < f.size() * sizeof(double)) {
+                    HIPCHK(hipStreamSynchronize(ctx->stream));
+                    p->dfields.alloc((size_t)std::min(most, nsteps) * nf * sizeof(double));
+                }
+                keep.v.push_back(std::move(f));
+                HIPCHK(hipMemcpyAsync(p->dfields.p, keep.v.back().data(), keep.v.back().size() * sizeof(double),
+                                      hipMemcpyHostToDevice, ctx->stream));
+                a.fields = p->dfields.as<double>();
+            }
+        }
+        a.nsteps = (int)n;
+        if (cheby) {
+            KTimer t(ctx, QDX_K_CHEBY_ROW);
+            launch_dense_cheby(ctx->stream, S, p->ham->dev.h64, a, p->dtab.as<double>(), p->coefd.as<double>(),
+                               p->k_launch, p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec, p->imag,
+                               psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
+            p->last_nb = 1;
+            p->nb_init = 1;
+        } else {
+            KTimer t(ctx, QDX_K_GSPO_ROW);
+            launch_dense_gspo(ctx->stream, S, pre, post, a, p->dtab.as<double>(), p->dtab.as<double>() + 2 * S * N,
+                              fop != nullptr, coupled, psi->ptr());
+        }
+        if (late) late();
+        i += n;
+    }
+}
+
 // |norm0 - accnorm| / norm0 of the last executed order of the last step
 // (imaginary time: |accnorm - accnorm of the order before| / the latter),
 // from the partial sums the kernels stored
@@ -433,13 +573,19 @@ void arnoldi_step(qdx_prop *p, qdx_wf *psi, long step);
 
 void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step);
 
+// FP32 split-operator propagation holds psi in FP32 between the steps (the
+// dense line kernels keep complex128)
+bool psi_in_fp32(const qdx_prop *p) {
+    return p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK && !dense_on(p);
+}
+
 // OPropagator::Backward() in real time (exponent +i dt, with the operators
 // conjugated, OPropagator.h:82-100): exp(+i H* dt) psi = conj(exp(-i H dt)
 // conj(psi)), the forward step between two conjugations (exact: conjugation
 // commutes with every rounding of the forward step)
 void prop_step(qdx_prop *p, qdx_wf *psi, long step) {
     if (!p->backward) return prop_step_forward(p, psi, step);
-    const bool g32 = p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK;
+    const bool g32 = psi_in_fp32(p);
     void *d = g32 ? static_cast<void *>(p->psi32.as<float>()) : static_cast<void *>(psi->ptr());
     const long n = (long)p->S * psi->n();
     launch_conj(p->ctx->stream, d, n, g32);
@@ -454,6 +600,11 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step) {
     }
     if (p->kind == qdx_prop::ARNOLDI) {
         arnoldi_step(p, psi, step);
+        return;
+    }
+    if (dense_on(p)) {
+        StreamKeep keep{p->ctx->stream, {}};   // one step copies no fields
+        dense_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep);
         return;
     }
     if (p->kind == qdx_prop::CHEBY) {
@@ -1082,10 +1233,18 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
         p->line_step = !imag && p->grid.nd == 1 && p->S == 1 &&
                        p->grid.N[0] <= (precision == QDX_FP32_BULK ? kMaxLine : 2048) &&
                        line_lds <= 160 * 1024;
-        if (p->line_step) {
+        p->dense = p->grid.nd == 1 && dense_blocks(p->grid.N[0], p->S, false) > 0;
+        if (p->dense) {
+            const std::vector<double> t = circulant_tables(kinetic_values(h), p->grid.N[0],
+                                                           [](double T) { return (long double)T; });
+            p->dtab.alloc(t.size() * sizeof(double));
+            HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+        }
+        if (p->line_step || p->dense) {
             // the same products as the per-order scalars of cheby_step
             const std::complex<double> ph =
-                std::exp(std::complex<double>(0, -1) * dt * std::complex<double>(p->cp.offset, p->cp.offset_i));
+                imag ? std::complex<double>(std::exp(-dt * p->cp.offset), 0.0)
+                     : std::exp(std::complex<double>(0, -1) * dt * std::complex<double>(p->cp.offset, p->cp.offset_i));
             std::vector<double> c(2 * (size_t)std::max(p->k_launch, 1));
             for (int k = 0; k < p->k_launch; ++k) {
                 const std::complex<double> v = p->cp.coeff[k] * ph;
@@ -1189,6 +1348,25 @@ static void gspo_create_impl(qdx_ham *const *ops, int32_t nops, double dt, int32
         if (p->grid.nd > 1) p->X.alloc(nbytes);
         if (precision == QDX_FP32_BULK) p->psi32.alloc(nbytes);
         p->partials.alloc(kMaxPartials * sizeof(double));
+        // short 1D lines in real time whose sequence holds one kinetic
+        // operator (the first) and at most one field: the dense kernel
+        int nkin = 0, nfield = 0, nx = 0;
+        for (qdx_ham *o : p->ops) {
+            if (o->terms[0].kind == T_KIN) ++nkin;
+            else ++nx;
+            if (o->time_dependent()) ++nfield;
+        }
+        p->dense = !imag && p->grid.nd == 1 && nkin == 1 && p->ops[0]->terms[0].kind == T_KIN && nx <= kMaxXOps &&
+                   nfield <= 1 && dense_blocks(p->grid.N[0], p->S, true) > 0;
+        if (p->dense) {
+            const auto T = kinetic_values(p->ops[0]);
+            const int N = p->grid.N[0];
+            std::vector<double> t = circulant_tables(T, N, [&](double v) { return cosl((long double)dt * v); });
+            const std::vector<double> ti = circulant_tables(T, N, [&](double v) { return -sinl((long double)dt * v); });
+            t.insert(t.end(), ti.begin(), ti.end());
+            p->dtab.alloc(t.size() * sizeof(double));
+            HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+        }
         ctx_acquire(p->ctx);
         *out = p.release();
     }
@@ -1207,10 +1385,10 @@ int qdx_prop_apply(qdx_prop *p, qdx_wf *psi, int64_t step, qdx_step_stats *stats
         if (!p) fail(QDX_ERR_PARAM, "propagator is NULL");
         check_prop_wf(p, psi);
         hipStream_t s = p->ctx->stream;
-        if (p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK)
-            launch_convert_c128_to_c64(s, psi->ptr(), p->psi32.as<float>(), (long)p->S * psi->n());
+        const bool g32 = psi_in_fp32(p);
+        if (g32) launch_convert_c128_to_c64(s, psi->ptr(), p->psi32.as<float>(), (long)p->S * psi->n());
         prop_step(p, psi, step);
-        if (p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK)
+        if (g32)
             launch_convert_c64_to_c128(s, p->psi32.as<float>(), psi->ptr(), (long)p->S * psi->n());
         if (stats) {
             if (p->kind == qdx_prop::CHEBY) {
@@ -1251,7 +1429,7 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
         hipStream_t s = p->ctx->stream;
         const int S = p->S;
         const long n = psi->n();
-        const bool g32 = p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK;
+        const bool g32 = psi_in_fp32(p);
         // device observables: per step, per state (re, im) of <psi|psi> and <psi|psi0>
         const size_t per_step = 4 * S;
         p->obs.alloc(std::max<size_t>(1, (size_t)nsteps * per_step + nsteps) * sizeof(double));
@@ -1288,7 +1466,12 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
                 gspo_run_fused<double>(p, ps, p0, first_step, nsteps, want ? obs : nullptr, per_step);
             }
         }
-        for (int64_t i = 0; i < (fused ? 0 : nsteps); ++i) {
+        const bool dense = dense_on(p) && !p->backward;
+        StreamKeep keep{s, {}};
+        if (dense)
+            dense_run(p, psi, first_step, nsteps, autocorr ? psi0->ptr() : nullptr, norm2 || autocorr ? obs : nullptr,
+                      p->kind == qdx_prop::CHEBY ? orders : nullptr, keep);
+        for (int64_t i = 0; i < (fused || dense ? 0 : nsteps); ++i) {
             double *o = obs + i * per_step;
             if (norm2) {
                 if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi32.as<float>(), n, S, part, o);

@@ -964,6 +964,11 @@ struct qdx_prop {
     // the phased coefficients coeff[k] exp(-i offset dt) on the device
     bool line_step = false;
     DevBuf coefd;
+    // short 1D lines (any states): whole runs in one block with the kinetic
+    // operator as a dense circulant matrix (qdx_dense.hip); dtab holds its
+    // tables (GSPO: real part, then imaginary part)
+    bool dense = false;
+    DevBuf dtab, dfields;
     int last_nb = 0, nb_init = 0;   // partial counts of the last Chebyshev step
     // SIL (Lanczos vectors and a buffer as device wave functions; `imag`
     // above selects imaginary time)

@@ -183,6 +183,17 @@ struct XGroupDev {
     XSplitDev<R> op[kMaxXOps];
 };
 
+// A run of steps on a 1D line by the dense kernels (qdx_dense.hip)
+struct DenseRun {
+    int N = 0;
+    int nsteps = 0;
+    const double *fields = nullptr;   // per step the S x S values -E(t) scale (GSPO: one value)
+    double field0[kMaxStates * kMaxStates] = {};   // the same for every step when fields is null
+    const double *psi0 = nullptr;     // autocorrelation partner (complex128)
+    double *obs = nullptr;            // observables before each step, 4 S doubles per step
+    int *orders = nullptr;            // H applications per step
+};
+
 // Events attached to the dispatch packet of the next kernel launch (set by the
 // host's profiling timer, consumed and cleared by that launch).
 struct LaunchTiming {
@@ -261,6 +272,18 @@ struct Launch {
     static void line_fft(hipStream_t s, const GridDev &g, int S, int dim, const LinePlan &p, const double *src,
                          R *X);
 };
+
+// Whole runs of a short 1D line in one block with T as a dense circulant
+// matrix (qdx_dense.hip).  dense_blocks: 0 when the line does not fit.  tab:
+// per state and parity the N values (t(d) +- t(d + N/2)) / 2 of the matrix
+// t(i - j) (GSPO: of exp(-i tau T), real and imaginary part)
+int dense_blocks(int N, int S, bool gspo);
+void launch_dense_cheby(hipStream_t s, int S, const HamDev<double> &h, const DenseRun &a, const double *tab,
+                        const double *coef, int order, double offset, double offset_i, double inv_scaling, double prec,
+                        bool imag, double *psi, ChebyCtl *ctl, double *partials);
+void launch_dense_gspo(hipStream_t s, int S, const XGroupDev<double> &pre, const XGroupDev<double> &post,
+                       const DenseRun &a, const double *tabr, const double *tabi, bool mu, bool coupled,
+                       double *psi);
 
 // precision-independent helpers
 void launch_convert_c128_to_c64(hipStream_t s, const double *src, float *dst, long n);
