@@ -20,44 +20,11 @@
 // all that follows (multiplies with the surfaces, recurrence, psi) is done
 // there, the other component one lane away.  One barrier per order publishes
 // the new term and the partial sums of the break test together.
+#include "qdx_gridfft.hpp"
 #include "qdx_kernels_common.hpp"
 #include "qdx_xsplit.hpp"
 
 namespace qdx {
-
-// the barrier of these kernels orders LDS only (no wait for global stores)
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// value of another lane by a DPP control word
-template <int CTRL>
-__device__ __forceinline__ double dpp(double x) {
-    const int lo = __double2loint(x), hi = __double2hiint(x);
-    return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, false),
-                            __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, false));
-}
-constexpr int kXor1 = 0xB1;          // quad_perm [1, 0, 3, 2]
-constexpr int kXor2 = 0x4E;          // quad_perm [2, 3, 0, 1]
-constexpr int kXor7 = 0x141;         // row_half_mirror
-constexpr int kXor15 = 0x140;        // row_mirror
-constexpr int kXor8 = 0x128;         // row_ror:8
-
-// sum over the wave, in every lane: 16-lane rows by DPP, then the four rows
-__device__ __forceinline__ double dense_wave_sum(double v) {
-    v += dpp<kXor1>(v);
-    v += dpp<kXor2>(v);
-    v += dpp<kXor7>(v);
-    v += dpp<kXor15>(v);
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    double t = 0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-        t += __hiloint2double(__builtin_amdgcn_readlane(hi, 16 * r), __builtin_amdgcn_readlane(lo, 16 * r));
-    return t;
-}
 
 // position of a thread and the pieces of LDS it uses
 template <int NB>
@@ -144,9 +111,9 @@ struct DenseLine {
 // sum |psi|^2 and sum conj(psi) psi0; red: 3 doubles per wave
 __device__ __forceinline__ void dense_obs_put(double ps, double p0, int comp, int wave, double *red) {
     const double p0x = dpp<kXor1>(p0);
-    const double n2 = dense_wave_sum(ps * ps);
-    const double ar = dense_wave_sum(ps * p0);
-    const double ai = dense_wave_sum(comp ? -ps * p0x : ps * p0x);
+    const double n2 = dpp_wave_sum(ps * ps);
+    const double ar = dpp_wave_sum(ps * p0);
+    const double ai = dpp_wave_sum(comp ? -ps * p0x : ps * p0x);
     if ((threadIdx.x & 63) == 0) {
         red[3 * wave] = n2;
         red[3 * wave + 1] = ar;
@@ -266,7 +233,7 @@ __global__ void __launch_bounds__(128 * NB * S) k_dense_cheby(HamDev<double> h, 
             }
             ps += ckr * pk - sgn * cki * dpp<kXor1>(pk);
             if (k >= 2 && (prec > 0 || k == order - 1)) {
-                const double s = dense_wave_sum(ps * ps);
+                const double s = dpp_wave_sum(ps * ps);
                 if (lane == 0) red[buf][B.wave] = s;
             }
             lds_barrier();

@@ -1,0 +1,634 @@
+// gfx950 persistent kernels of 2D grids that fit the chip's registers: whole
+// Chebyshev runs in one cooperative launch.
+//
+// A 2D grid of up to 2^19 points and states is bound by latency when every
+// order is two launches (row kernel and column pass): each of them reads its
+// operands back from memory, fills the chip with only two waves per SIMD and
+// drains (512 x 512 points, two states: 36 us per order in FP64, 25 in FP32;
+// here 19.5 and 14, of which the two filters take 9 and the two exchanges of
+// 8.4 MB 7).  Here every block keeps its rows of psi, phi_{k-1}, phi_{k-2} and of
+// the surfaces in registers over all orders and steps; only the kinetic part
+// along dimension 1 travels: phi_{k-1} to the owners of the columns, its
+// filtered lines back to the owners of the rows.
+//
+// Block b owns rows [b rb, (b + 1) rb) of every state and the columns
+// [b cw, (b + 1) cw) of every state; lanes run over the lines first (row: l =
+// r S + st, column: l = c S + st), then over the points of a line.  The two
+// exchange buffers hold one chunk of S rb cw values per (row block, column
+// block) pair, column-block major for phi (A) and row-block major for the way
+// back (B), so that both sides move whole chunks.
+//
+// Order of an iteration: store phi to A, filter the own rows along dimension 0
+// (hides the exchange), signaling on the way, wait for all row blocks, load the own
+// columns, filter, store to B, signal, wait for all column blocks, load,
+// epilogue.  Chunks move with agent-scope (sc1) stores and loads, which go
+// past the XCDs' private L2s: no cache write-back or invalidation is needed,
+// only the store counter before the block's flag is raised.  Flags hold
+// epochs that grow over all launches of a propagator.
+//
+// Every wait is bounded (kGridWait): a block that gives up leaves, the others
+// follow, and the host, which keeps psi until the launch is known to be
+// complete, runs the steps again order by order.
+#include "qdx_gridfft.hpp"
+
+namespace qdx {
+
+// bound of one wait in ticks of the 100 MHz wall clock: 2 s
+constexpr unsigned long long kGridWait = 200000000ull;
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+constexpr int kAgentScope = 16;   // sc1 of the buffer instructions' cache policy
+
+// a place past the end of every exchange buffer: the buffer instructions read 0
+// there (S N <= 2^19 values of 16 bytes; 16 times this stays below 2^31)
+constexpr int kGridNowhere = 0x7ffffff;
+
+// exchange buffer with agent-scope accesses of whole complex values
+template <class R>
+struct GridX {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ GridX(void *p, long n)
+        : r(__builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(n * (long)sizeof(cx<R>)), 0x00020000)) {}
+    __device__ __forceinline__ void st(int i, cx<R> v) const {
+        if constexpr (sizeof(R) == 8)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, i * 16, 0, kAgentScope);
+        else
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, i * 8, 0, kAgentScope);
+    }
+    __device__ __forceinline__ cx<R> ld(int i) const {
+        if constexpr (sizeof(R) == 8)
+            return __builtin_bit_cast(cx<R>, __builtin_amdgcn_raw_buffer_load_b128(r, i * 16, 0, kAgentScope));
+        else
+            return __builtin_bit_cast(cx<R>, __builtin_amdgcn_raw_buffer_load_b64(r, i * 8, 0, kAgentScope));
+    }
+};
+
+// this thread's stores have reached the coherence point
+__device__ __forceinline__ void grid_drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Flags and partial sums are kept in kGridCopies copies: a block writes all of
+// them in one store instruction and reads only the copy of its group (b mod
+// 8, the blocks of one XCD).  One copy polled by every wave of 256 blocks took
+// 4 us to pass a barrier, 1.1 us with 32 blocks.
+constexpr int kGridCopies = 8;
+constexpr int kGridCopyBytes = kGridBlocks * 4 + 4 * kGridBlocks * 8 + 256;   // flags, four slots of partial sums
+static_assert(kGridCopies * kGridCopyBytes <= (int)kGridSyncBytes, "sync area");
+__device__ __forceinline__ unsigned *grid_flags(char *sync, int copy) {
+    return reinterpret_cast<unsigned *>(sync + copy * kGridCopyBytes);
+}
+__device__ __forceinline__ double *grid_slot(char *sync, int copy, int slot) {
+    return reinterpret_cast<double *>(sync + copy * kGridCopyBytes + kGridBlocks * 4) + slot * kGridBlocks;
+}
+
+// by wave 0: this block's flag
+__device__ __forceinline__ void grid_signal(char *sync, unsigned epoch) {
+    if (threadIdx.x < kGridCopies)
+        __hip_atomic_store(grid_flags(sync, threadIdx.x) + blockIdx.x, epoch, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+// by wave 0: this block's partial sum, also where the host looks for it
+__device__ __forceinline__ void grid_put(char *sync, int slot, double v, double *partials) {
+    if (threadIdx.x < kGridCopies)
+        __hip_atomic_store(grid_slot(sync, threadIdx.x, slot) + blockIdx.x, v, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    else if (threadIdx.x == kGridCopies)
+        partials[slot * kMaxPartials + blockIdx.x] = v;
+}
+
+// by wave 0: waits until the first n blocks' flags have reached epoch; false
+// after kGridWait.  n <= kGridBlocks.
+__device__ __forceinline__ bool grid_wait(char *sync, int n, unsigned epoch) {
+    const unsigned *flags = grid_flags(sync, blockIdx.x % kGridCopies);
+    const int lane = threadIdx.x & 63;
+    unsigned long long t0 = 0;
+    for (bool first = true;; first = false) {
+        unsigned f[kGridBlocks / 64];
+#pragma unroll
+        for (int i = 0; i < kGridBlocks / 64; ++i)
+            f[i] = lane + 64 * i < n
+                       ? __hip_atomic_load(flags + lane + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                       : epoch;
+        bool good = true;
+#pragma unroll
+        for (int i = 0; i < kGridBlocks / 64; ++i) good = good && (int)(f[i] - epoch) >= 0;
+        if (__all(good)) break;
+        if (first) t0 = wall_clock64();
+        else if (wall_clock64() - t0 > kGridWait) return false;
+    }
+    asm volatile("" ::: "memory");   // loads of the exchanged data stay behind
+    return true;
+}
+
+// by wave 0: sum of the first n blocks' partials, the same in every block; lane 0
+__device__ __forceinline__ double grid_sum(char *sync, int slot, int n) {
+    const double *p = grid_slot(sync, blockIdx.x % kGridCopies, slot);
+    const int lane = threadIdx.x & 63;
+    double a[kGridBlocks / 64], t = 0;
+#pragma unroll
+    for (int i = 0; i < kGridBlocks / 64; ++i)
+        a[i] = lane + 64 * i < n ? __hip_atomic_load(p + lane + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                 : 0.0;
+#pragma unroll
+    for (int i = 0; i < kGridBlocks / 64; ++i) t += a[i];
+    return dpp_wave_sum(t);
+}
+
+// A block's rows and columns: what each of its threads owns of them, where
+// that sits in the exchange buffers, and the filters' tables in LDS.
+template <class R, int S>
+struct GridBlock {
+    int b, N0, N1, n, nrb, ncb;
+    bool row, col;          // this block owns rows / columns
+    int rst, cst;           // state of this thread's row / column
+    int gi0;                // grid point of the row's first element (the others m0 apart)
+    int rA[8], rB[8], cA[8], cB[8];   // places of the row's and the column's elements in A and B
+    GridAxis<R> ax[2];
+    const double *f[2];     // the factor tables, per state
+    __device__ GridBlock(const GridRun &a, const GridShape &g, const LinePlan &p0, const LinePlan &p1, cx<R> *smem) {
+        b = blockIdx.x;
+        N0 = p0.L;
+        N1 = p1.L;
+        n = N0 * N1;
+        nrb = g.nrb;
+        ncb = g.ncb;
+        row = b < nrb;
+        col = b < ncb;
+        const int rb = g.rb, cw = g.cw, chunk = S * rb * cw, tid = threadIdx.x;
+        const int len0 = grid_line_len(g.R2[0], g.R3[0]), len1 = grid_line_len(g.R2[1], g.R3[1]);
+        const int lines = max(rb * S * len0, cw * S * len1);
+        cx<R> *tw = smem + lines;
+        for (int d = 0; d < 2; ++d) {
+            GridAxis<R> &A = ax[d];
+            A.m = (d ? N1 : N0) / 8;
+            A.R2 = g.R2[d];
+            A.R3 = g.R3[d];
+            A.RS = grid_rs(A.R3);
+            A.nl = (d ? cw : rb) * S;
+            A.lt = tid / A.nl;
+            A.a = A.lt / A.R3;
+            A.b = A.lt - A.a * A.R3;
+            A.buf = smem + (tid - A.lt * A.nl);
+            if (d == 0 || N1 != N0) {
+                grid_tables(reinterpret_cast<const cx<R> *>(d ? p1.tw : p0.tw), A.m, A.R3, tw, tw + 7 * A.m);
+                A.tw1 = tw;
+                A.tw2 = tw + 7 * A.m;
+                tw += grid_tw_len(A.m);
+            } else {
+                A.tw1 = ax[0].tw1;
+                A.tw2 = ax[0].tw2;
+            }
+        }
+        f[0] = reinterpret_cast<double *>(tw);
+        f[1] = f[0] + S * len0;
+        const int lr = tid - ax[0].lt * ax[0].nl, r = lr / S, lc = tid - ax[1].lt * ax[1].nl, c = lc / S;
+        rst = lr - r * S;
+        cst = lc - c * S;
+        ax[0].on = row && ax[0].lt < ax[0].m && b * rb + r < N1;
+        ax[1].on = col && ax[1].lt < ax[1].m && b * cw + c < N0;
+        gi0 = (b * rb + r) * N0 + ax[0].lt;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int x = ax[0].lt + q * ax[0].m, xb = x / cw, xc = x - xb * cw;
+            rA[q] = (xb * nrb + b) * chunk + (xc * rb + r) * S + rst;
+            rB[q] = (b * ncb + xb) * chunk + (r * cw + xc) * S + rst;
+            if (!ax[0].on) rB[q] = kGridNowhere;
+            const int y = ax[1].lt + q * ax[1].m, yb = y / rb, yr = y - yb * rb;
+            cA[q] = (b * nrb + yb) * chunk + (c * rb + yr) * S + cst;
+            cB[q] = (yb * ncb + b) * chunk + (yr * cw + c) * S + cst;
+        }
+    }
+    __device__ int gi(int q) const { return gi0 + q * ax[0].m; }
+    // the axis of the filter `ph` as this thread takes part in it
+    __device__ GridAxis<R> axis(int ph) const {
+        GridAxis<R> A = ax[0];
+        if (ph) A = ax[1];
+        return A;
+    }
+};
+
+// per-state observables of the state before a step (Reporter.cpp:101-137) as
+// per-block partial sums, and its norm for the break test (slot 2)
+template <class R, int S>
+__device__ __forceinline__ void grid_observe(const GridRun &a, const GridBlock<R, S> &B, int step,
+                                             const cx<double> (&ps)[8], double (*red)[3 * S], double *partials) {
+    const int tid = threadIdx.x, wave = tid >> 6, nw = (blockDim.x + 63) >> 6;
+    double o[3] = {0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        o[0] += ps[q].r * ps[q].r + ps[q].i * ps[q].i;
+        if (a.psi0 && B.ax[0].on) {
+            const cx<double> z = reinterpret_cast<const cx<double> *>(a.psi0)[(long)B.rst * B.n + B.gi(q)];
+            o[1] += ps[q].r * z.r + ps[q].i * z.i;
+            o[2] += ps[q].r * z.i - ps[q].i * z.r;
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double v = dpp_wave_sum(s == B.rst ? o[c] : 0.0);
+            if ((tid & 63) == 0) red[wave][3 * s + c] = v;
+        }
+    lds_barrier();
+    if (!B.row) return;
+    if (tid < 3 * S) {
+        double v = 0;
+        for (int w = 0; w < nw; ++w) v += red[w][tid];
+        a.obsp[((long)step * 3 * S + tid) * B.nrb + B.b] = v;
+    }
+    if (wave == 0 && partials) {
+        double v = 0;
+        for (int s = 0; s < S; ++s)
+            for (int w = 0; w < nw; ++w) v += red[w][3 * s];
+        grid_put(a.sync, 2, v, partials);
+    }
+}
+
+// Chebyshev steps of a 2D grid (OCheby::real_time_step, and with IMAG
+// imag_time_step, OCheby.cpp:92-297): the operands, break tests and orders of
+// the per-order kernels.  partials: slots of the per-order kernels, one value
+// per row block.  NIP: negative imaginary potential (one state).
+template <class R, int S, bool IMAG, bool NIP, bool PRIMES>
+__global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamDev<R> h, LinePlan p0, LinePlan p1,
+                                                    const double *__restrict__ coef, int order, double offset,
+                                                    double offset_i, double inv_scaling, double prec,
+                                                    const cx<double> *__restrict__ psi, ChebyCtl *ctl,
+                                                    double *__restrict__ partials) {
+    extern __shared__ __align__(16) char smem_raw[];
+    __shared__ double red[4][3 * S], bc;
+    __shared__ int bad;
+    __shared__ const R *Wp[S][S], *Mp[S][S];   // (scalar registers are short in the order loop)
+    const int tid = threadIdx.x, wave = tid >> 6, nw = (blockDim.x + 63) >> 6;
+    const GridBlock<R, S> B(a, g, p0, p1, reinterpret_cast<cx<R> *>(smem_raw));
+    const int st = B.rst;
+    const bool on = B.ax[0].on;
+    if (tid == 0) {
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+#pragma unroll
+            for (int j = 0; j < S; ++j) {
+                Wp[i][j] = h.W[i][j];
+                Mp[i][j] = h.mu[i][j];
+            }
+    }
+    const double uni = st ? h.unity[S - 1] : h.unity[0];
+    for (int s = 0; s < S; ++s) {
+        const int len0 = grid_line_len(g.R2[0], g.R3[0]), len1 = grid_line_len(g.R2[1], g.R3[1]);
+        grid_factors(h.tk[s][0], h.inv_nd[0], g.R2[0], g.R3[0], const_cast<double *>(B.f[0]) + s * len0);
+        grid_factors(h.tk[s][1], h.inv_nd[1], g.R2[1], g.R3[1], const_cast<double *>(B.f[1]) + s * len1);
+    }
+    if (tid == 0) bad = 0;
+    const long nx = (long)S * g.nrb * g.rb * g.ncb * g.cw;
+    const GridX<R> XA(a.A, nx), XB(a.B, nx);
+    cx<double> ps[8];
+    double wi[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        ps[q] = on ? psi[(long)st * B.n + B.gi(q)] : mk<double>(0, 0);
+        if (NIP) wi[q] = on ? (offset_i + (h.Wi[0] ? (double)h.Wi[0][B.gi(q)] : 0.0)) * inv_scaling : 0.0;
+    }
+    constexpr int NS = IMAG ? 3 : 2;
+    auto slot = [](int k) { return k % NS == 2 ? 3 : k % NS; };
+    unsigned epoch = a.epoch;
+    double norm0 = 0, acc = 0, last_acc = 0;
+    int last = 1;
+    bool broke = false;
+    __syncthreads();
+    for (int step = 0; step < a.nsteps; ++step) {
+        double wv[S][8];
+#pragma unroll
+        for (int j = 0; j < S; ++j) {
+            const double E = a.fields ? a.fields[((long)step * S + st) * S + j] : a.field0[st * S + j];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                double w = j == st ? uni : 0.0;
+                if (on && Wp[st][j]) w += (double)Wp[st][j][B.gi(q)];
+                if (on && Mp[st][j]) w += E * (double)Mp[st][j][B.gi(q)];
+                wv[j][q] = w;
+            }
+        }
+        cx<R> pm1[8], pm2[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            pm1[q] = from_d<R>(ps[q]);
+            pm2[q] = mk<R>(0, 0);
+        }
+        grid_observe<R, S>(a, B, step, ps, red, partials);
+        last = 1;
+        broke = false;
+        acc = last_acc = 0;
+        for (int k = 1; k < order; ++k) {
+            const cx<double> ck = mk<double>(coef[2 * k], coef[2 * k + 1]);
+            cx<R> x[8], v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                x[q] = pm1[q];
+                if (on) XA.st(B.rA[q], pm1[q]);
+            }
+            ++epoch;
+#pragma unroll 1
+            for (int ph = 0; ph < 2; ++ph) {
+                if (ph ? B.col : B.row) {
+                    // the block's flag goes up inside the row filter, once its stores have landed
+                    grid_filter<PRIMES>(x, B.axis(ph), ph ? B.f[1] + B.cst * grid_line_len(g.R2[1], g.R3[1])
+                                                  : B.f[0] + st * grid_line_len(g.R2[0], g.R3[0]),
+                                [&] { if (ph == 0) grid_drain(); },
+                                [&] { if (ph == 0 && wave == 0) grid_signal(a.sync, epoch); });
+                } else {
+                    lds_barrier();   // publishes bc
+                }
+                if (ph) break;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[q] = x[q];
+                if (wave == 0 && !grid_wait(a.sync, B.nrb, epoch) && tid == 0) bad = 1;
+                lds_barrier();
+                if (bad) break;
+                if (B.ax[1].on) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) x[q] = XA.ld(B.cA[q]);
+                }
+                // sum |psi|^2 of the step start or of order k - 1
+                if (wave == 0 && (k == 1 || (k >= 3 && prec > 0))) {
+                    const double s = grid_sum(a.sync, k == 1 ? 2 : slot(k - 1), B.nrb);
+                    if (tid == 0) bc = s;
+                }
+            }
+            if (bad) {
+                if (tid == 0) *a.status = 1;
+                return;
+            }
+            if (k == 1) norm0 = bc;
+            if (k >= 3 && prec > 0) {
+                // break test of order k - 1 (OCheby.cpp:179-182, 283-285)
+                last_acc = acc;
+                acc = bc;
+                if (IMAG ? (k >= 4 && fabs(acc - last_acc) / last_acc < prec) : fabs(norm0 - acc) / norm0 < prec) {
+                    broke = true;
+                    break;
+                }
+            }
+            last = k;
+            if (B.ax[1].on) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) XB.st(B.cB[q], x[q]);
+            }
+            grid_drain();
+            lds_barrier();
+            ++epoch;
+            if (wave == 0) {
+                if (B.col) grid_signal(a.sync, epoch);
+                if (B.row && !grid_wait(a.sync, B.ncb, epoch) && tid == 0) bad = 1;
+            }
+            lds_barrier();
+            if (bad) {
+                if (tid == 0) *a.status = 1;
+                return;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) x[q] = XB.ld(B.rB[q]);   // 0 for threads without a row
+            const double two = k == 1 ? 1.0 : 2.0;   // phi_1 = (H - offset) phi_0 / R * (-i); pm2 = 0 there
+            double sum = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                cx<double> hp = to_d(v[q]) + to_d(x[q]);
+                const cx<double> p = to_d(pm1[q]);
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    // the other state's value sits one lane away
+                    cx<double> pj = p;
+                    if constexpr (S == 2) {
+                        const cx<R> o = mk<R>(dpp<kXor1>(pm1[q].r), dpp<kXor1>(pm1[q].i));
+                        if (j != st) pj = to_d(o);
+                    }
+                    hp.r += wv[j][q] * pj.r;
+                    hp.i += wv[j][q] * pj.i;
+                }
+                cx<double> bb = mk<double>((hp.r - offset * p.r) * inv_scaling, (hp.i - offset * p.i) * inv_scaling);
+                if (NIP) {
+                    bb.r += wi[q] * p.i;
+                    bb.i -= wi[q] * p.r;
+                }
+                const cx<double> mm = to_d(pm2[q]);
+                cx<double> pk;
+                if (IMAG) pk = mk<double>(-two * bb.r - mm.r, -two * bb.i - mm.i);
+                else pk = mk<double>(two * bb.i + mm.r, -two * bb.r + mm.i);
+                if (k == 1) ps[q] = cmul(mk<double>(coef[0], coef[1]), ps[q]);
+                ps[q] = ps[q] + cmul(ck, pk);
+                sum += ps[q].r * ps[q].r + ps[q].i * ps[q].i;
+                pm2[q] = pm1[q];
+                pm1[q] = from_d<R>(pk);
+            }
+            if (k >= 2 && (prec > 0 || k == order - 1)) {
+                const double s = dpp_wave_sum(sum);
+                if ((tid & 63) == 0) red[wave][0] = s;
+                lds_barrier();
+                if (B.row && wave == 0) {
+                    double t = 0;
+                    for (int w = 0; w < nw; ++w) t += red[w][0];
+                    grid_put(a.sync, slot(k), t, partials);
+                }
+            }
+        }
+        if (B.b == 0 && tid == 0 && a.orders) a.orders[step] = last;
+        lds_barrier();   // the next step's first writes to red follow the last reads
+    }
+    if (B.b == 0 && tid == 0) {
+        ctl->norm0 = norm0;
+        ctl->done = broke;
+        ctl->accnorm = acc;
+        ctl->last_order = last;
+    }
+    if (on) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) reinterpret_cast<cx<double> *>(a.out)[(long)st * B.n + B.gi(q)] = ps[q];
+    }
+}
+
+// After a run: psi from its staging copy and the observables of each step
+// (blocks past ncopy, one per step: 4 S doubles as qdx_prop_run lays them
+// out); nothing when the run gave up.  report: host-visible status.
+__global__ void __launch_bounds__(256) k_grid_finish(GridRun a, int S, long n, int nrb, int ncopy,
+                                                     cx<double> *__restrict__ psi, double *__restrict__ obs,
+                                                     volatile int *report) {
+    const int status = *a.status;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *report = status;
+    if (status) return;
+    if ((int)blockIdx.x < ncopy) {
+        const cx<double> *out = reinterpret_cast<const cx<double> *>(a.out);
+        for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < S * n; i += (long)ncopy * 256) psi[i] = out[i];
+        return;
+    }
+    const int step = blockIdx.x - ncopy, wave = threadIdx.x >> 6;
+    for (int o = wave; o < 3 * S; o += 4) {
+        const double *p = a.obsp + ((long)step * 3 * S + o) * nrb;
+        double t = 0;
+        for (int i = threadIdx.x & 63; i < nrb; i += 64) t += p[i];
+        t = wave_sum(t);
+        if ((threadIdx.x & 63) == 0) {
+            const int s = o / 3, c = o - 3 * s;
+            double *d = obs + (long)step * 4 * S;
+            if (c == 0) {
+                d[2 * s] = t;
+                d[2 * s + 1] = 0;
+            } else {
+                d[2 * S + 2 * s + c - 1] = t;
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+
+// Points of a block's lines, at least: one wave of 8 each.  A short line is a
+// latency chain, so it goes to as many CUs as there are lines (an order of
+// 64 x 64 points takes 9.4 us with 512 points per block, 10.1 with 1024, 11.8
+// with 2048; 256 x 256 12.0, 12.5, 14.6; 240 x 176 16.5, 17.2, 18.7).
+constexpr int kGridFill = 512;
+
+static size_t grid_lds_bytes(const GridShape &g, int N0, int N1, int S, size_t elem) {
+    const size_t l0 = grid_line_len(g.R2[0], g.R3[0]), l1 = grid_line_len(g.R2[1], g.R3[1]);
+    const size_t tw = grid_tw_len(N0 / 8) + (N1 == N0 ? 0 : grid_tw_len(N1 / 8));
+    return (std::max(g.rb * S * l0, g.cw * S * l1) + tw) * elem + S * (l0 + l1) * sizeof(double);
+}
+
+// m = R2 R3 for a line of 8 m points: the stages' radices (see grid_filter),
+// the pair with the fewest multiply-adds per point and passes; false when
+// there is none
+static bool grid_radices(int m, int &R2, int &R3) {
+    auto dft = [](int r) {   // operations of a butterfly, about
+        if (r == 1) return 0.0;
+        double c = 0;
+        int n = r;
+        for (int p : {2, 3, 5, 7, 11, 13, 17, 19, 23, 29, 31})
+            while (n % p == 0) {
+                n /= p;
+                c += p == 2 ? 2.0 : p == 3 ? 4.0 : p - 1.0;
+            }
+        return n > 1 ? -1.0 : c * r;
+    };
+    double best = 0;
+    R2 = 0;
+    for (int r3 = 1; r3 <= 16; ++r3) {
+        if (m % r3) continue;
+        const int r2 = m / r3;
+        const bool prime = r2 == 17 || r2 == 19 || r2 == 23 || r2 == 29 || r2 == 31;
+        if (r2 > 16 && !prime) continue;
+        // butterflies of one thread times their cost (twiddles: 4 operations),
+        // LDS accesses included
+        auto stage = [&](int r) { return ((8 + r - 1) / r) * (dft(r) + 12.0 * r + 40.0); };
+        const double c = (r2 > 1 ? stage(r2) + 60.0 : 0.0) + stage(r3);
+        if (!R2 || c < best) {
+            best = c;
+            R2 = r2;
+            R3 = r3;
+        }
+    }
+    return R2 > 0;
+}
+
+bool grid_shape(int N0, int N1, int S, int cus, GridShape &g) {
+    if (S < 1 || S > 2 || N0 % 8 || N1 % 8 || N0 < 8 || N1 < 8) return false;
+    if (!grid_radices(N0 / 8, g.R2[0], g.R3[0]) || !grid_radices(N1 / 8, g.R2[1], g.R3[1])) return false;
+    for (int d = 0; d < 2; ++d)
+        for (int r : {g.R2[d], g.R3[d]}) g.primes = g.primes || r == 11 || r == 13 || r > 16;
+    const int most = std::min(cus, kGridBlocks);
+    // lines per block: at most 256 threads at 8 points each and no more
+    // blocks than CUs; the fewest lines with kGridFill points
+    auto pick = [&](int lines, int L) {
+        int best = 0;
+        for (int r = 1; r <= lines && r * S * L <= 2048; ++r) {
+            if ((lines + r - 1) / r > most) continue;
+            best = r;
+            if (r * S * L >= kGridFill) break;
+        }
+        return best;
+    };
+    g.rb = pick(N1, N0);
+    g.cw = pick(N0, N1);
+    if (!g.rb || !g.cw) return false;
+    g.nrb = (N1 + g.rb - 1) / g.rb;
+    g.ncb = (N0 + g.cw - 1) / g.cw;
+    g.blocks = std::max(g.nrb, g.ncb);
+    g.threads = std::max(64, round64(std::max(g.rb * S * (N0 / 8), g.cw * S * (N1 / 8))));
+    // the 160 KiB of a CU (the tables of two long lines may not fit)
+    return grid_lds_bytes(g, N0, N1, S, 16) <= kLdsBytes - 1024;
+}
+
+size_t grid_exchange_len(const GridShape &g, int S) { return (size_t)S * g.nrb * g.rb * g.ncb * g.cw; }
+
+// false: the device does not hold all blocks at once
+template <class K, class... Args>
+static bool coop_launch(K kernel, int blocks, int threads, size_t lds, hipStream_t s, Args... args) {
+    set_lds(kernel, lds);
+    void *argv[] = {(void *)&args...};
+    const LaunchTiming t = g_launch_timing;
+    if (t.start) QDX_HIP(hipEventRecord(t.start, s));
+    const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kernel), dim3(blocks),
+                                                    dim3(threads), argv, (unsigned)lds, s);
+    if (e == hipErrorCooperativeLaunchTooLarge) {
+        (void)hipGetLastError();
+        g_launch_timing = LaunchTiming();
+        return false;
+    }
+    QDX_HIP(e);
+    if (t.start) {
+        QDX_HIP(hipEventRecord(t.stop, s));
+        g_launch_timing = LaunchTiming();
+    }
+    return true;
+}
+
+template <class R>
+bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
+                       const LinePlan &p0, const LinePlan &p1, const double *coef, int order, double offset,
+                       double offset_i, double inv_scaling, double prec, bool imag, const double *psi, ChebyCtl *ctl,
+                       double *partials) {
+    const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, sizeof(cx<R>));
+    auto cp = reinterpret_cast<const cx<double> *>(psi);
+    const bool nip = offset_i != 0 || h.Wi[0] != nullptr;
+    bool ran = false;
+#define QDX_GRID(S_, IMAG_, NIP_)                     \
+    do {                                              \
+        if (g.primes) QDX_GRIDP(S_, IMAG_, NIP_, true); \
+        else QDX_GRIDP(S_, IMAG_, NIP_, false);       \
+    } while (0)
+#define QDX_GRIDP(S_, IMAG_, NIP_, PR_)                                                                      \
+    ran = coop_launch(k_cheby_grid<R, S_, IMAG_, NIP_, PR_>, g.blocks, g.threads, lds, s, a, g, h, p0, p1, coef, order, offset, \
+                nip ? offset_i : 0.0, inv_scaling, prec, cp, ctl, partials)
+    if (nip) {
+        if (S != 1 || imag) throw std::runtime_error("negative imaginary potential: one state, real time only");
+        QDX_GRID(1, false, true);
+    } else if (imag) {
+        if constexpr (std::is_same<R, double>::value) {
+            if (S == 1) QDX_GRID(1, true, false);
+            else QDX_GRID(2, true, false);
+        } else {
+            throw std::runtime_error("imaginary time: FP64 only");
+        }
+    } else if (S == 1) {
+        QDX_GRID(1, false, false);
+    } else {
+        QDX_GRID(2, false, false);
+    }
+#undef QDX_GRID
+#undef QDX_GRIDP
+    return ran;
+}
+template bool launch_cheby_grid(hipStream_t, int, const HamDev<double> &, const GridShape &, const GridRun &,
+                                const LinePlan &, const LinePlan &, const double *, int, double, double, double, double,
+                                bool, const double *, ChebyCtl *, double *);
+template bool launch_cheby_grid(hipStream_t, int, const HamDev<float> &, const GridShape &, const GridRun &,
+                                const LinePlan &, const LinePlan &, const double *, int, double, double, double, double,
+                                bool, const double *, ChebyCtl *, double *);
+
+void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
+                        int *report) {
+    const int ncopy = (int)std::min<long>(1024, (S * n + 255) / 256);
+    QDX_LAUNCH(k_grid_finish, dim3(ncopy + (obs ? a.nsteps : 0)), dim3(256), 0, s, a, S, n, g.nrb, ncopy,
+               reinterpret_cast<cx<double> *>(psi), obs, report);
+    QDX_HIP(hipGetLastError());
+}
+
+}  // namespace qdx

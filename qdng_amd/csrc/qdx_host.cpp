@@ -457,6 +457,43 @@ struct StreamKeep {
     }
 };
 
+// The field values of steps first .. first + n - 1 of a run by one launch: nf
+// per step, in `field0` for a single step, else on the device (*fields).
+// Returns the steps that have them; fewer than n when the clock leaves the
+// field, and `late` then raises the error of the step after the last valid
+// one.  most: the longest launch of the run.
+long run_fields(qdx_prop *p, qdx_ham *fop, int nf, long first, long n, long most, double *field0,
+                const double **fields, std::function<void()> &late, StreamKeep &keep) {
+    std::vector<double> f;
+    HamDev<double> h;
+    const int S = p->S;
+    for (long k = 0; k < n; ++k) {
+        try {
+            fop->set_fields(h, first + k);
+        } catch (const QdxError &e) {
+            if (k == 0) throw;
+            const QdxError err = e;
+            late = [err] { throw err; };
+            n = k;
+            break;
+        }
+        for (int c = 0; c < nf; ++c) f.push_back(h.Edip[nf > 1 ? c / S : 0][nf > 1 ? c % S : 0]);
+    }
+    if (n == 1) {
+        std::copy(f.begin(), f.end(), field0);
+        return n;
+    }
+    if (p->dfields.bytes < f.size() * sizeof(double)) {
+        HIPCHK(hipStreamSynchronize(p->ctx->stream));
+        p->dfields.alloc((size_t)most * nf * sizeof(double));
+    }
+    keep.v.push_back(std::move(f));
+    HIPCHK(hipMemcpyAsync(p->dfields.p, keep.v.back().data(), keep.v.back().size() * sizeof(double),
+                          hipMemcpyHostToDevice, p->ctx->stream));
+    *fields = p->dfields.as<double>();
+    return n;
+}
+
 // Steps first .. first + nsteps - 1 of a propagation that keeps to dense
 // lines.  obs (nullable): observables before each step, 4 S doubles per step;
 // orders (nullable): H applications per step (device arrays).  The host
@@ -496,35 +533,8 @@ void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *
         a.psi0 = psi0;
         a.obs = obs ? obs + (size_t)i * 4 * S : nullptr;
         a.orders = orders ? orders + i : nullptr;
-        std::function<void()> late;   // raises the error of the step after the last valid one
-        if (fop) {
-            std::vector<double> f;
-            HamDev<double> h;
-            for (long k = 0; k < n; ++k) {
-                try {
-                    fop->set_fields(h, first + i + k);
-                } catch (const QdxError &e) {
-                    if (k == 0) throw;
-                    const QdxError err = e;
-                    late = [err] { throw err; };
-                    n = k;
-                    break;
-                }
-                for (int c = 0; c < nf; ++c) f.push_back(h.Edip[cheby ? c / S : 0][cheby ? c % S : 0]);
-            }
-            if (n == 1) {
-                std::copy(f.begin(), f.end(), a.field0);
-            } else {
-                if (p->dfields.bytes < f.size() * sizeof(double)) {
-                    HIPCHK(hipStreamSynchronize(ctx->stream));
-                    p->dfields.alloc((size_t)std::min(most, nsteps) * nf * sizeof(double));
-                }
-                keep.v.push_back(std::move(f));
-                HIPCHK(hipMemcpyAsync(p->dfields.p, keep.v.back().data(), keep.v.back().size() * sizeof(double),
-                                      hipMemcpyHostToDevice, ctx->stream));
-                a.fields = p->dfields.as<double>();
-            }
-        }
+        std::function<void()> late;
+        if (fop) n = run_fields(p, fop, nf, first + i, n, std::min(most, nsteps), a.field0, &a.fields, late, keep);
         a.nsteps = (int)n;
         if (cheby) {
             KTimer t(ctx, QDX_K_CHEBY_ROW);
@@ -541,6 +551,83 @@ void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *
         if (late) late();
         i += n;
     }
+}
+
+// --- 2D grids in registers: whole runs in one launch (qdx_grid.hip) ----------
+
+// qdx_ctx_set_line_points 4 or 8 asks for the per-order kernels
+bool grid_on(const qdx_prop *p) { return p->grid2d && p->ctx->line_ppt == 0; }
+
+// Chebyshev steps first .. first + nsteps - 1 by the persistent kernel, as
+// dense_run; returns the steps done.  Fewer than nsteps when a launch gave up
+// waiting for its blocks (psi is then the state after the steps done): the
+// caller goes on order by order.
+template <class R>
+long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
+              StreamKeep &keep) {
+    qdx_ctx *ctx = p->ctx;
+    const int S = p->S;
+    const bool fp32 = std::is_same<R, float>::value;
+    const LinePlan p0 = ctx->plan_ppt(p->grid.N[0], fp32, 4), p1 = ctx->plan_ppt(p->grid.N[1], fp32, 4);
+    const HamDev<R> *h;
+    if constexpr (std::is_same<R, float>::value) h = &p->ham->dev.h32;
+    else h = &p->ham->dev.h64;
+    qdx_ham *fop = p->ham->time_dependent() ? p->ham : nullptr;
+    // a launch runs at most 2048 orders: tens of milliseconds
+    const long most = std::max(1L, 2048L / std::max(p->k_launch, 1));
+    for (long i = 0; i < nsteps;) {
+        long n = std::min(most, nsteps - i);
+        GridRun a;
+        std::function<void()> late;
+        if (fop) n = run_fields(p, fop, S * S, first + i, n, std::min(most, nsteps), a.field0, &a.fields, late, keep);
+        a.nsteps = (int)n;
+        if (p->gepoch > (1u << 30)) {
+            HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, ctx->stream));
+            p->gepoch = 0;
+        }
+        a.epoch = p->gepoch;
+        p->gepoch += 2u * (unsigned)(p->k_launch * n);
+        a.sync = p->gflags.as<char>();
+        a.status = reinterpret_cast<int *>(a.sync + kGridSyncBytes);
+        a.A = p->phiA.p;
+        a.B = p->phiB.p;
+        a.out = p->X.as<double>();
+        const size_t obytes = (size_t)n * 3 * S * p->gs.nrb * sizeof(double);
+        if (p->gobs.bytes < obytes) p->gobs.alloc(obytes);   // no launch is in flight here
+        a.obsp = p->gobs.as<double>();
+        a.psi0 = psi0;
+        a.orders = orders ? orders + i : nullptr;
+        bool ran;
+        {
+            KTimer t(ctx, QDX_K_CHEBY_ROW);
+            ran = launch_cheby_grid<R>(ctx->stream, S, *h, p->gs, a, p0, p1, p->coefd.as<double>(), p->k_launch,
+                                       p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec, p->imag,
+                                       psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
+        }
+        if (!ran) {
+            p->grid2d = false;
+            return i;
+        }
+        launch_grid_finish(ctx->stream, S, psi->n(), p->gs, a, psi->ptr(), obs ? obs + (size_t)i * 4 * S : nullptr,
+                           p->greport);
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+        if (*p->greport) {
+            HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, ctx->stream));
+            p->gepoch = 0;
+            p->grid2d = false;
+            return i;
+        }
+        p->last_nb = p->gs.nrb;
+        p->nb_init = p->gs.nrb;
+        if (late) late();
+        i += n;
+    }
+    return nsteps;
+}
+long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
+              StreamKeep &keep) {
+    return p->precision == QDX_FP32_BULK ? grid_run<float>(p, psi, first, nsteps, psi0, obs, orders, keep)
+                                         : grid_run<double>(p, psi, first, nsteps, psi0, obs, orders, keep);
 }
 
 // |norm0 - accnorm| / norm0 of the last executed order of the last step
@@ -606,6 +693,10 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step) {
         StreamKeep keep{p->ctx->stream, {}};   // one step copies no fields
         dense_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep);
         return;
+    }
+    if (grid_on(p)) {
+        StreamKeep keep{p->ctx->stream, {}};
+        if (grid_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep) == 1) return;
     }
     if (p->kind == qdx_prop::CHEBY) {
         // QDX_COMPACT: FP64 arithmetic (compact terms when p->cmp)
@@ -1215,10 +1306,22 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
         if (precision == QDX_FP32_BULK) h->ensure32();
         // element bytes of the term buffers (compact: 8 hi + 2 lo)
         const size_t es = p->cmp ? 10 : precision == QDX_FP32_BULK ? 2 * sizeof(float) : 2 * sizeof(double);
-        const size_t nbytes = (size_t)p->S * p->grid.size() * es;
+        // 2D grids that fit the chip's registers: X holds complex128 there,
+        // compact terms are exchanged as complex128
+        int cus = 0, coop = 0;
+        HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->ctx->device));
+        HIPCHK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, p->ctx->device));
+        p->grid2d = coop && p->grid.nd == 2 && grid_shape(p->grid.N[0], p->grid.N[1], p->S, cus, p->gs);
+        const size_t nval = (size_t)p->S * p->grid.size();
+        const size_t nbytes = p->grid2d ? std::max(nval, grid_exchange_len(p->gs, p->S)) * (p->cmp ? 16 : es) : nval * es;
         p->phiA.alloc(nbytes);
         p->phiB.alloc(nbytes);
-        if (p->grid.nd > 1) p->X.alloc(nbytes);
+        if (p->grid.nd > 1) p->X.alloc(p->grid2d ? nval * 16 : nbytes);
+        if (p->grid2d) {
+            p->gflags.alloc(kGridSyncBytes + sizeof(int));
+            HIPCHK(hipMemset(p->gflags.p, 0, p->gflags.bytes));
+            HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&p->greport), sizeof(int), hipHostMallocDefault));
+        }
         p->ctl.alloc(sizeof(ChebyCtl));
         HIPCHK(hipMemset(p->ctl.p, 0, sizeof(ChebyCtl)));
         p->partials.alloc(4 * kMaxPartials * sizeof(double));
@@ -1240,7 +1343,7 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
             p->dtab.alloc(t.size() * sizeof(double));
             HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         }
-        if (p->line_step || p->dense) {
+        if (p->line_step || p->dense || p->grid2d) {
             // the same products as the per-order scalars of cheby_step
             const std::complex<double> ph =
                 imag ? std::complex<double>(std::exp(-dt * p->cp.offset), 0.0)
@@ -1466,12 +1569,19 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
                 gspo_run_fused<double>(p, ps, p0, first_step, nsteps, want ? obs : nullptr, per_step);
             }
         }
-        const bool dense = dense_on(p) && !p->backward;
+        // (an autocorrelation with the propagated function itself follows it
+        // step by step)
+        const bool whole = !p->backward && !(autocorr && psi0->ptr() == psi->ptr());
+        const bool dense = dense_on(p) && whole;
         StreamKeep keep{s, {}};
         if (dense)
             dense_run(p, psi, first_step, nsteps, autocorr ? psi0->ptr() : nullptr, norm2 || autocorr ? obs : nullptr,
                       p->kind == qdx_prop::CHEBY ? orders : nullptr, keep);
-        for (int64_t i = 0; i < (fused || dense ? 0 : nsteps); ++i) {
+        int64_t done = fused || dense ? nsteps : 0;
+        if (grid_on(p) && whole)
+            done = grid_run(p, psi, first_step, nsteps, autocorr ? psi0->ptr() : nullptr,
+                            norm2 || autocorr ? obs : nullptr, orders, keep);
+        for (int64_t i = done; i < nsteps; ++i) {
             double *o = obs + i * per_step;
             if (norm2) {
                 if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi32.as<float>(), n, S, part, o);

@@ -969,6 +969,13 @@ struct qdx_prop {
     // tables (GSPO: real part, then imaginary part)
     bool dense = false;
     DevBuf dtab, dfields;
+    // 2D grids that fit the chip's registers (Chebyshev): whole runs in one
+    // launch (qdx_grid.hip); gepoch: the flags' values so far
+    bool grid2d = false;
+    GridShape gs;
+    DevBuf gflags, gobs;
+    unsigned gepoch = 0;
+    int *greport = nullptr;   // host memory: status of the last launch
     int last_nb = 0, nb_init = 0;   // partial counts of the last Chebyshev step
     // SIL (Lanczos vectors and a buffer as device wave functions; `imag`
     // above selects imaginary time)
@@ -990,5 +997,7 @@ struct qdx_prop {
     DevBuf psi32, psi0_32;
     DevBuf obs;   // device observables of qdx_prop_run
 
-    virtual ~qdx_prop() = default;
+    virtual ~qdx_prop() {
+        if (greport) (void)hipHostFree(greport);
+    }
 };

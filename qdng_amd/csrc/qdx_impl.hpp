@@ -194,6 +194,29 @@ struct DenseRun {
     int *orders = nullptr;            // H applications per step
 };
 
+// A run of steps on a 2D grid by the persistent kernels (qdx_grid.hip): block
+// shape (rows and columns per block) and the arguments of one launch
+constexpr int kGridBlocks = 256;
+constexpr size_t kGridSyncBytes = 8 * (kGridBlocks * 4 + 4 * kGridBlocks * 8 + 256);
+struct GridShape {
+    int rb = 0, cw = 0, nrb = 0, ncb = 0, blocks = 0, threads = 0;
+    int R2[2] = {}, R3[2] = {};   // radices of the line filters (qdx_gridfft.hpp)
+    bool primes = false;          // primes above 7 among them
+};
+struct GridRun {
+    int nsteps = 0;
+    unsigned epoch = 0;               // flags reach at most epoch + 2 orders nsteps
+    char *sync = nullptr;             // flags and partial sums (kGridSyncBytes)
+    int *status = nullptr;            // set by a run that gave up waiting
+    void *A = nullptr, *B = nullptr;  // exchange buffers (grid_exchange_len values of the kernel precision)
+    double *out = nullptr;            // the final psi (complex128)
+    double *obsp = nullptr;           // per step, state and observable (3) one partial sum per row block
+    const double *fields = nullptr;   // as DenseRun
+    double field0[kMaxStates * kMaxStates] = {};
+    const double *psi0 = nullptr;
+    int *orders = nullptr;
+};
+
 // Events attached to the dispatch packet of the next kernel launch (set by the
 // host's profiling timer, consumed and cleared by that launch).
 struct LaunchTiming {
@@ -284,6 +307,21 @@ void launch_dense_cheby(hipStream_t s, int S, const HamDev<double> &h, const Den
 void launch_dense_gspo(hipStream_t s, int S, const XGroupDev<double> &pre, const XGroupDev<double> &post,
                        const DenseRun &a, const double *tabr, const double *tabi, bool mu, bool coupled,
                        double *psi);
+
+// Whole runs of a 2D grid in one cooperative launch (qdx_grid.hip).
+// grid_shape: false when the grid does not fit a device of `cus` CUs.
+// launch_cheby_grid: false when the device does not hold all blocks at once.
+// launch_grid_finish: psi, the observables (nullable) and the status of the
+// run after launch_cheby_grid.
+bool grid_shape(int N0, int N1, int S, int cus, GridShape &g);
+size_t grid_exchange_len(const GridShape &g, int S);
+template <class R>
+bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
+                       const LinePlan &p0, const LinePlan &p1, const double *coef, int order, double offset,
+                       double offset_i, double inv_scaling, double prec, bool imag, const double *psi, ChebyCtl *ctl,
+                       double *partials);
+void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
+                        int *report);
 
 // precision-independent helpers
 void launch_convert_c128_to_c64(hipStream_t s, const double *src, float *dst, long n);

@@ -1,0 +1,143 @@
+"""2D grids whose runs stay in registers (qdx_grid.hip) against the per-order
+kernels, which qdx_ctx_set_line_points(8) selects: the smallest lines, unequal
+sides (more row blocks than column blocks and the reverse), several lines per
+block, sides with odd prime factors, the largest grid of the rule and the
+first beyond it; both kinds of time, fields, the negative imaginary potential,
+runs and single steps.  Both evaluate the same series in FP64: an H
+application differs by a few 1e-16 of the kinetic range, a series of order k
+by about k times that, so 1e-11 bounds a few steps of at most a few hundred
+orders; the series lengths are equal.  In FP32 both round each term to 2^-24
+and carry that through the same recurrence: 1e-5 over these short series."""
+import numpy as np
+import pytest
+
+import cases
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm(np.asarray(a) - np.asarray(b)) / np.linalg.norm(b)
+
+
+def box(N0, N1, S, laser=False, nip=False, coupled=True, nt=12):
+    p = cases.Problem([N0, N1], [-6.0, -5.0], [6.0, 5.0], nstates=S)
+    x, y = p.axes()
+    one = np.ones(np.broadcast_shapes(x.shape, y.shape))
+    for s in range(S):
+        p.kinetic(s, [1500.0 + 300 * s, 2500.0 - 200 * s])
+        p.potential(s, s, np.minimum(0.03 * (1 + 0.3 * s) * ((x - 0.2 * s) ** 2 + y ** 2) + 0.01 * s, 1.0))
+    if S > 1 and coupled:
+        p.potential(0, 1, 0.02 * np.exp(-x ** 2 - (y - 0.3) ** 2))
+    if laser:
+        p.dipole(1 if S > 1 else 0, 0, one * x * np.exp(-x ** 2 / 8), 0.01 * np.cos(0.3 * np.arange(nt)))
+    if nip:
+        p.gobbler(0, 0, rp={0: 4.0}, order=5, gain=0.02, nip=True)
+    g = np.exp(-(x - 0.4) ** 2 - (y + 0.2) ** 2 + 0.8j * x - 0.3j * y)
+    p.psi0 = cases.normalized(p, np.stack([(1 - 0.2j * s) * g for s in range(S)]))
+    return p
+
+
+def both(make, steps, run):
+    import qdng_amd as Q
+    out = []
+    for points in (0, 8):
+        c = Q.Context(0)
+        try:
+            c.set_line_points(points)
+            p, U = make(c)
+            w, w0 = p.gpu_wf(c), p.gpu_wf(c)
+            if run:
+                n2, ac, nh, _ = U.run(w, 1, steps, w0)
+            else:
+                st = [U.apply(w, 1 + i) for i in range(steps)]
+                n2, ac, nh = [s.norm2 for s in st], [w.overlap(w0)], [s.n_hpsi for s in st]
+            out.append((w.download(), np.array(n2), np.array(ac), list(nh)))
+            del U, w, w0
+        finally:
+            c.close()
+    return out
+
+
+def check(pair, tol=1e-11):
+    (a, na, aa, ha), (b, nb, ab, hb) = pair
+    assert ha == hb
+    assert rel(a, b) < tol
+    assert np.max(np.abs(na - nb) / nb) < tol and np.max(np.abs(aa - ab)) < tol * max(1.0, np.max(np.abs(ab)))
+
+
+SHAPES = [(8, 8, 1), (8, 16, 2), (24, 8, 1), (40, 56, 2), (104, 88, 1), (16, 768, 1), (768, 16, 2), (64, 64, 1),
+          (240, 176, 1), (232, 248, 2), (256, 256, 1), (128, 384, 2), (768, 512, 1), (512, 512, 2), (768, 768, 2)]
+
+
+@pytest.mark.parametrize("N0,N1,S", SHAPES)
+@pytest.mark.parametrize("laser", [False, True])
+def test_cheby(N0, N1, S, laser):
+    import qdng_amd as Q
+    print("[gpu case] grid cheby", N0, N1, S, laser, flush=True)
+
+    def make(c):
+        p = box(N0, N1, S, laser)
+        return p, Q.Cheby(p.gpu_ham(c), 2.0, prec=1e-12)
+    check(both(make, 4, True))
+    check(both(make, 2, False))
+
+
+@pytest.mark.parametrize("precision,tol", [("fp32", 1e-5), ("compact", 5e-8)])
+@pytest.mark.parametrize("N0,N1,S", [(8, 16, 1), (240, 176, 1), (512, 512, 2)])
+def test_reduced(N0, N1, S, precision, tol):
+    import qdng_amd as Q
+    print("[gpu case] grid", precision, N0, N1, S, flush=True)
+
+    def make(c):
+        p = box(N0, N1, S, S == 1)
+        return p, Q.Cheby(p.gpu_ham(c), 2.0, prec=1e-10, precision=precision)
+    check(both(make, 4, True), tol)
+
+
+@pytest.mark.parametrize("N0,N1,S", [(16, 8, 1), (104, 88, 2), (256, 256, 1)])
+def test_imaginary_time(N0, N1, S):
+    import qdng_amd as Q
+    print("[gpu case] grid imaginary", N0, N1, S, flush=True)
+
+    def make(c):
+        p = box(N0, N1, S)
+        H = p.gpu_ham(c)
+        lo, hi = H.bounds()
+        return p, Q.Cheby(H, 3.0 / (hi - lo), prec=1e-10, imag=True)
+    # the series cancels down to exp(-R dt) = e^-3 of its terms
+    check(both(make, 3, False))
+
+
+@pytest.mark.parametrize("N0,N1", [(40, 24), (256, 128)])
+def test_nip_backward_fixed_series(N0, N1):
+    import qdng_amd as Q
+    print("[gpu case] grid nip / backward / prec 0", N0, N1, flush=True)
+
+    def nip(c):
+        p = box(N0, N1, 1, nip=True)
+        return p, Q.Cheby(p.gpu_ham(c), 2.0)
+    check(both(nip, 3, True))
+
+    def back(c):
+        p = box(N0, N1, 1, laser=True)
+        U = Q.Cheby(p.gpu_ham(c), 2.0, prec=0.0)
+        U.backward()
+        return p, U
+    check(both(back, 3, True))
+
+
+def test_long_run_and_own_autocorrelation(ctx):
+    """More orders than one launch takes; a psi0 that is psi itself follows
+    the propagation."""
+    import qdng_amd as Q
+    p = box(32, 24, 1, laser=True, nt=300)
+    U = Q.Cheby(p.gpu_ham(ctx), 2.0, prec=1e-12)
+    w, ref, w0 = p.gpu_wf(ctx), p.gpu_wf(ctx), p.gpu_wf(ctx)
+    n2, ac, nh, _ = U.run(w, 0, 250, w0)
+    for i in range(250):
+        U.apply(ref, i)
+    assert np.array_equal(w.download(), ref.download())
+    assert len(nh) == 250 and min(nh) > 3
+    n2, ac, _, _ = U.run(w, 0, 3, w)
+    assert np.allclose(ac, n2, rtol=1e-12)
