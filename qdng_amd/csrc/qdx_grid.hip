@@ -30,6 +30,7 @@
 // follow, and the host, which keeps psi until the launch is known to be
 // complete, runs the steps again order by order.
 #include "qdx_gridfft.hpp"
+#include "qdx_xsplit.hpp"
 
 namespace qdx {
 
@@ -141,11 +142,12 @@ struct GridBlock {
     int b, N0, N1, n, nrb, ncb;
     bool row, col;          // this block owns rows / columns
     int rst, cst;           // state of this thread's row / column
-    int gi0;                // grid point of the row's first element (the others m0 apart)
+    int gi0, gi1;           // grid points of the row's and the column's first element (the others m0 and m1 N0 apart)
     int rA[8], rB[8], cA[8], cB[8];   // places of the row's and the column's elements in A and B
     GridAxis<R> ax[2];
     const double *f[2];     // the factor tables, per state
-    __device__ GridBlock(const GridRun &a, const GridShape &g, const LinePlan &p0, const LinePlan &p1, cx<R> *smem) {
+    // need: the axes whose filters run (bits 0 and 1)
+    __device__ GridBlock(const GridShape &g, const LinePlan &p0, const LinePlan &p1, cx<R> *smem, int need = 3) {
         b = blockIdx.x;
         N0 = p0.L;
         N1 = p1.L;
@@ -155,6 +157,8 @@ struct GridBlock {
         row = b < nrb;
         col = b < ncb;
         const int rb = g.rb, cw = g.cw, chunk = S * rb * cw, tid = threadIdx.x;
+        // neighbouring columns share cache lines: keep them on one XCD
+        const int cb = col ? xcd_remap(b, ncb) : b;
         const int len0 = grid_line_len(g.R2[0], g.R3[0]), len1 = grid_line_len(g.R2[1], g.R3[1]);
         const int lines = max(rb * S * len0, cw * S * len1);
         cx<R> *tw = smem + lines;
@@ -170,7 +174,8 @@ struct GridBlock {
             A.b = A.lt - A.a * A.R3;
             A.buf = smem + (tid - A.lt * A.nl);
             if (d == 0 || N1 != N0) {
-                grid_tables(reinterpret_cast<const cx<R> *>(d ? p1.tw : p0.tw), A.m, A.R3, tw, tw + 7 * A.m);
+                if (N1 == N0 || (need >> d) & 1)
+                    grid_tables(reinterpret_cast<const cx<R> *>(d ? p1.tw : p0.tw), A.m, A.R3, tw, tw + 7 * A.m);
                 A.tw1 = tw;
                 A.tw2 = tw + 7 * A.m;
                 tw += grid_tw_len(A.m);
@@ -185,8 +190,9 @@ struct GridBlock {
         rst = lr - r * S;
         cst = lc - c * S;
         ax[0].on = row && ax[0].lt < ax[0].m && b * rb + r < N1;
-        ax[1].on = col && ax[1].lt < ax[1].m && b * cw + c < N0;
+        ax[1].on = col && ax[1].lt < ax[1].m && cb * cw + c < N0;
         gi0 = (b * rb + r) * N0 + ax[0].lt;
+        gi1 = ax[1].lt * N0 + cb * cw + c;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const int x = ax[0].lt + q * ax[0].m, xb = x / cw, xc = x - xb * cw;
@@ -194,8 +200,8 @@ struct GridBlock {
             rB[q] = (b * ncb + xb) * chunk + (r * cw + xc) * S + rst;
             if (!ax[0].on) rB[q] = kGridNowhere;
             const int y = ax[1].lt + q * ax[1].m, yb = y / rb, yr = y - yb * rb;
-            cA[q] = (b * nrb + yb) * chunk + (c * rb + yr) * S + cst;
-            cB[q] = (yb * ncb + b) * chunk + (yr * cw + c) * S + cst;
+            cA[q] = !ax[1].on ? kGridNowhere : (cb * nrb + yb) * chunk + (c * rb + yr) * S + cst;
+            cB[q] = (yb * ncb + cb) * chunk + (yr * cw + c) * S + cst;
         }
     }
     __device__ int gi(int q) const { return gi0 + q * ax[0].m; }
@@ -207,37 +213,27 @@ struct GridBlock {
     }
 };
 
-// per-state observables of the state before a step (Reporter.cpp:101-137) as
-// per-block partial sums, and its norm for the break test (slot 2)
-template <class R, int S>
-__device__ __forceinline__ void grid_observe(const GridRun &a, const GridBlock<R, S> &B, int step,
-                                             const cx<double> (&ps)[8], double (*red)[3 * S], double *partials) {
+// Per-state observables of the state before a step (Reporter.cpp:101-137), o:
+// this thread's share of sum |psi|^2 and sum conj(psi) psi0, as one partial sum
+// per block; put_norm: the block's norm also goes to the break test (slot 2).
+template <int S>
+__device__ __forceinline__ void grid_observe(const GridRun &a, int step, int st, const double (&o)[3],
+                                             double (*red)[3 * S], bool put_norm, double *partials) {
     const int tid = threadIdx.x, wave = tid >> 6, nw = (blockDim.x + 63) >> 6;
-    double o[3] = {0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        o[0] += ps[q].r * ps[q].r + ps[q].i * ps[q].i;
-        if (a.psi0 && B.ax[0].on) {
-            const cx<double> z = reinterpret_cast<const cx<double> *>(a.psi0)[(long)B.rst * B.n + B.gi(q)];
-            o[1] += ps[q].r * z.r + ps[q].i * z.i;
-            o[2] += ps[q].r * z.i - ps[q].i * z.r;
-        }
-    }
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            const double v = dpp_wave_sum(s == B.rst ? o[c] : 0.0);
+            const double v = dpp_wave_sum(s == st ? o[c] : 0.0);
             if ((tid & 63) == 0) red[wave][3 * s + c] = v;
         }
     lds_barrier();
-    if (!B.row) return;
     if (tid < 3 * S) {
         double v = 0;
         for (int w = 0; w < nw; ++w) v += red[w][tid];
-        a.obsp[((long)step * 3 * S + tid) * B.nrb + B.b] = v;
+        a.obsp[((long)step * 3 * S + tid) * gridDim.x + blockIdx.x] = v;
     }
-    if (wave == 0 && partials) {
+    if (wave == 0 && put_norm) {
         double v = 0;
         for (int s = 0; s < S; ++s)
             for (int w = 0; w < nw; ++w) v += red[w][3 * s];
@@ -260,7 +256,7 @@ __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamD
     __shared__ int bad;
     __shared__ const R *Wp[S][S], *Mp[S][S];   // (scalar registers are short in the order loop)
     const int tid = threadIdx.x, wave = tid >> 6, nw = (blockDim.x + 63) >> 6;
-    const GridBlock<R, S> B(a, g, p0, p1, reinterpret_cast<cx<R> *>(smem_raw));
+    const GridBlock<R, S> B(g, p0, p1, reinterpret_cast<cx<R> *>(smem_raw));
     const int st = B.rst;
     const bool on = B.ax[0].on;
     if (tid == 0) {
@@ -314,7 +310,17 @@ __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamD
             pm1[q] = from_d<R>(ps[q]);
             pm2[q] = mk<R>(0, 0);
         }
-        grid_observe<R, S>(a, B, step, ps, red, partials);
+        double o[3] = {0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            o[0] += ps[q].r * ps[q].r + ps[q].i * ps[q].i;
+            if (a.psi0 && on) {
+                const cx<double> z = reinterpret_cast<const cx<double> *>(a.psi0)[(long)st * B.n + B.gi(q)];
+                o[1] += ps[q].r * z.r + ps[q].i * z.i;
+                o[2] += ps[q].r * z.i - ps[q].i * z.r;
+            }
+        }
+        grid_observe<S>(a, step, st, o, red, B.row, partials);
         last = 1;
         broke = false;
         acc = last_acc = 0;
@@ -344,10 +350,8 @@ __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamD
                 if (wave == 0 && !grid_wait(a.sync, B.nrb, epoch) && tid == 0) bad = 1;
                 lds_barrier();
                 if (bad) break;
-                if (B.ax[1].on) {
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) x[q] = XA.ld(B.cA[q]);
-                }
+                for (int q = 0; q < 8; ++q) x[q] = XA.ld(B.cA[q]);   // 0 for threads without a column
                 // sum |psi|^2 of the step start or of order k - 1
                 if (wave == 0 && (k == 1 || (k >= 3 && prec > 0))) {
                     const double s = grid_sum(a.sync, k == 1 ? 2 : slot(k - 1), B.nrb);
@@ -445,10 +449,217 @@ __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamD
     }
 }
 
+// Split-operator steps exp(-i tau/2 W) exp(-i tau T) exp(-i tau/2 W) of a 2D
+// grid (OGSPO.cpp:114-139), W the product of the x-space operators: a phase per
+// point, whose field part (MU, one state) is formed per step, or (CPL) one 2 x 2
+// unitary of two coupled states.  exp(-i tau T) is a filter along each
+// dimension, in either order: steps that begin in the row layout filter along
+// dimension 0, hand the lines over and end in the column layout, where the
+// next step begins (its number's parity says where: single steps give the bits
+// of a run).  One exchange per step; the x-space tables and psi0 sit in
+// registers in both layouts.  Waiting for one launch costs more than a single
+// step, which is two ordinary launches of the same kernel instead (a.part 1:
+// up to the exchange, 2: the rest, psi in place).  Per step on 512 x 512 points, two coupled states,
+// observables included: 41 -> 16.2 us against the column and the row pass.
+template <class R, int S, bool MU, bool CPL, bool PRIMES>
+__global__ void __launch_bounds__(256) k_gspo_grid(GridRun a, GridShape g, XGroupDev<R> pre, LinePlan p0, LinePlan p1,
+                                                   const double *__restrict__ ek, double inv0, double inv1,
+                                                   const cx<double> *__restrict__ psi) {
+    static_assert(!MU || S == 1, "field operators act on one state");
+    static_assert(!CPL || S == 2, "two coupled states");
+    extern __shared__ __align__(16) char smem_raw[];
+    __shared__ double red[4][3 * S];
+    __shared__ int bad;
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const bool begin = a.first & 1;                    // the layout of psi before the first step
+    const bool later = begin != (a.part == 2);         // ... and of the part's filter
+    const int need = a.part ? 1 << later : 3;
+    const GridBlock<R, S> B(g, p0, p1, reinterpret_cast<cx<R> *>(smem_raw), need);
+    // factors exp(-i tau T_d(k)) / N_d; ek: per state the tables of both
+    // dimensions, (re, im)
+    cx<double> *fac = reinterpret_cast<cx<double> *>(const_cast<double *>(B.f[0]));
+    const int len0 = grid_line_len(g.R2[0], g.R3[0]), len1 = grid_line_len(g.R2[1], g.R3[1]);
+    for (int s = 0; s < S; ++s) {
+        const cx<double> *e = reinterpret_cast<const cx<double> *>(ek) + (long)s * (B.N0 + B.N1);
+        if (need & 1) grid_factors(e, inv0, g.R2[0], g.R3[0], fac + s * len0);
+        if (need & 2) grid_factors(e + B.N0, inv1, g.R2[1], g.R3[1], fac + S * len0 + s * len1);
+    }
+    const cx<double> *f0 = fac + B.rst * len0, *f1 = fac + S * len0 + B.cst * len1;
+    if (tid == 0) bad = 0;
+    const long nx = (long)S * g.nrb * g.rb * g.ncb * g.cw;
+    const GridX<R> XA(a.A, nx), XB(a.B, nx);
+    const bool on0 = B.ax[0].on, on1 = B.ax[1].on;
+    const int st0 = B.rst, st1 = B.cst;
+    // this thread's points in both layouts: the x-space group (own state and,
+    // coupled, the other one; of a field operator mu tau) and psi0
+    struct Layout {
+        cx<double> u[8], w[CPL ? 8 : 1], z[8];
+        double mu[MU ? 8 : 1];
+    } L0, L1;
+    // the usual group, one operator with a table, is read in one go (point by
+    // point the eight reads wait for each other)
+    const bool table = !MU && pre.n == 1 && pre.op[0].U;
+    auto load = [&](Layout &L, bool on, int st, auto gi) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            L.u[q] = mk<double>(1, 0);
+            L.z[q] = mk<double>(0, 0);
+            if constexpr (CPL) L.w[q] = mk<double>(0, 0);
+            if constexpr (MU) L.mu[q] = 0;
+        }
+        if (!on) return;
+        if (a.psi0) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) L.z[q] = reinterpret_cast<const cx<double> *>(a.psi0)[(long)st * B.n + gi(q)];
+        }
+        if (table) {
+            const cx<double> *U = reinterpret_cast<const cx<double> *>(pre.op[0].U);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                L.u[q] = U[(long)(CPL ? 2 * st : st) * B.n + gi(q)];
+                if constexpr (CPL) L.w[q] = U[B.n + gi(q)];
+            }
+            return;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const long i = gi(q);
+            if constexpr (CPL) {
+                cx<double> v[2] = {mk<double>(st == 0, 0), mk<double>(st == 1, 0)};
+                xgroup_point<R, 2>(pre, i, v);   // a symmetric matrix
+                L.u[q] = st ? v[1] : v[0];
+                L.w[q] = st ? v[0] : v[1];
+            } else {
+                cx<double> v[S];
+#pragma unroll
+                for (int s = 0; s < S; ++s) v[s] = mk<double>(1, 0);
+                for (int o = 0; o < pre.n; ++o) {
+                    XSplitDev<R> op = pre.op[o];
+                    if constexpr (MU) {
+                        if (op.mu[0][0]) {
+                            L.mu[q] = op.tau * (double)op.mu[0][0][i];
+                            op.mu[0][0] = nullptr;   // the field part is formed per step
+                            if (!op.V[0][0]) continue;
+                        }
+                    }
+                    xsplit_point<R, S>(op, i, v);
+                }
+                L.u[q] = S == 2 && st ? v[S - 1] : v[0];
+            }
+        }
+    };
+    const int gr = B.gi0, gc = B.gi1, m0 = B.ax[0].m, sc = B.ax[1].m * B.N0;
+    if (need & 1) load(L0, on0, st0, [&](int q) { return (long)(gr + q * m0); });
+    if (need & 2) load(L1, on1, st1, [&](int q) { return (long)gc + (long)q * sc; });
+    // the x-space group on x
+    auto apply = [&](const Layout &L, cx<R>(&x)[8], double E) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            cx<double> u = L.u[q];
+            if constexpr (MU) {
+                double sn, cs;
+                sincos(-L.mu[q] * E, &sn, &cs);
+                u = cmul(u, mk<double>(cs, sn));
+            }
+            cx<double> y = cmul(u, to_d(x[q]));
+            if constexpr (CPL) y = y + cmul(L.w[q], to_d(mk<R>(dpp<kXor1>(x[q].r), dpp<kXor1>(x[q].i))));
+            x[q] = from_d<R>(y);
+        }
+    };
+    auto observe = [&](const Layout &L, const cx<R>(&x)[8], double(&o)[3]) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const cx<double> p = to_d(x[q]);
+            o[0] += p.r * p.r + p.i * p.i;
+            o[1] += p.r * L.z[q].r + p.i * L.z[q].i;
+            o[2] += p.r * L.z[q].i - p.i * L.z[q].r;
+        }
+    };
+    cx<R> x[8];
+    bool cols = later;   // the layout of x
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        x[q] = mk<R>(0, 0);
+        if (a.part == 2) {
+            x[q] = cols ? XA.ld(B.cA[q]) : XB.ld(B.rB[q]);
+        } else if (cols) {
+            if (on1) x[q] = from_d<R>(psi[(long)st1 * B.n + gc + (long)q * sc]);
+        } else if (on0) {
+            x[q] = from_d<R>(psi[(long)st0 * B.n + gr + q * m0]);
+        }
+    }
+    unsigned epoch = a.epoch;
+    __syncthreads();
+    // two half steps per step, each with one filter
+#pragma unroll 1
+    for (int half = a.part == 2; half < 2 * a.nsteps; ++half) {
+        const int step = half >> 1;
+        const bool second = half & 1;
+        const double E = MU ? (a.fields ? a.fields[step] : a.field0[0]) : 0.0;
+        if (!second) {
+            if (a.observe) {
+                double o[3] = {0, 0, 0};
+                if (cols) observe(L1, x, o);
+                else observe(L0, x, o);
+                grid_observe<S>(a, step, cols ? st1 : st0, o, red, false, nullptr);
+            }
+            if (cols) apply(L1, x, E);
+            else apply(L0, x, E);
+        }
+        if (cols ? B.col : B.row)
+            grid_filter<PRIMES>(x, B.axis(cols), cols ? f1 : f0, [] {}, [] {});
+        if (second) {
+            if (cols) apply(L1, x, E);
+            else apply(L0, x, E);
+            continue;
+        }
+        // hand over to the other layout
+        if (cols) {
+            if (on1) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) XB.st(B.cB[q], x[q]);
+            }
+        } else if (on0) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) XA.st(B.rA[q], x[q]);
+        }
+        if (a.part == 1) return;
+        grid_drain();
+        lds_barrier();
+        ++epoch;
+        if (wave == 0) {
+            if (cols ? B.col : B.row) grid_signal(a.sync, epoch);
+            if ((cols ? B.row : B.col) && !grid_wait(a.sync, cols ? B.ncb : B.nrb, epoch) && tid == 0) bad = 1;
+        }
+        lds_barrier();
+        if (bad) {
+            if (tid == 0) *a.status = 1;
+            return;
+        }
+        if (cols) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) x[q] = XB.ld(B.rB[q]);   // 0 for threads without a row
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) x[q] = XA.ld(B.cA[q]);
+        }
+        cols = !cols;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        cx<double> *out = reinterpret_cast<cx<double> *>(a.out);
+        if (cols) {
+            if (on1) out[(long)st1 * B.n + gc + (long)q * sc] = to_d(x[q]);
+        } else if (on0) {
+            out[(long)st0 * B.n + gr + q * m0] = to_d(x[q]);
+        }
+    }
+}
+
 // After a run: psi from its staging copy and the observables of each step
 // (blocks past ncopy, one per step: 4 S doubles as qdx_prop_run lays them
 // out); nothing when the run gave up.  report: host-visible status.
-__global__ void __launch_bounds__(256) k_grid_finish(GridRun a, int S, long n, int nrb, int ncopy,
+__global__ void __launch_bounds__(256) k_grid_finish(GridRun a, int S, long n, int nb, int ncopy,
                                                      cx<double> *__restrict__ psi, double *__restrict__ obs,
                                                      volatile int *report) {
     const int status = *a.status;
@@ -461,9 +672,9 @@ __global__ void __launch_bounds__(256) k_grid_finish(GridRun a, int S, long n, i
     }
     const int step = blockIdx.x - ncopy, wave = threadIdx.x >> 6;
     for (int o = wave; o < 3 * S; o += 4) {
-        const double *p = a.obsp + ((long)step * 3 * S + o) * nrb;
+        const double *p = a.obsp + ((long)step * 3 * S + o) * nb;
         double t = 0;
-        for (int i = threadIdx.x & 63; i < nrb; i += 64) t += p[i];
+        for (int i = threadIdx.x & 63; i < nb; i += 64) t += p[i];
         t = wave_sum(t);
         if ((threadIdx.x & 63) == 0) {
             const int s = o / 3, c = o - 3 * s;
@@ -487,10 +698,11 @@ __global__ void __launch_bounds__(256) k_grid_finish(GridRun a, int S, long n, i
 // with 2048; 256 x 256 12.0, 12.5, 14.6; 240 x 176 16.5, 17.2, 18.7).
 constexpr int kGridFill = 512;
 
-static size_t grid_lds_bytes(const GridShape &g, int N0, int N1, int S, size_t elem) {
+// factor: bytes of a filter's factor (8 real, 16 complex)
+static size_t grid_lds_bytes(const GridShape &g, int N0, int N1, int S, size_t elem, size_t factor) {
     const size_t l0 = grid_line_len(g.R2[0], g.R3[0]), l1 = grid_line_len(g.R2[1], g.R3[1]);
     const size_t tw = grid_tw_len(N0 / 8) + (N1 == N0 ? 0 : grid_tw_len(N1 / 8));
-    return (std::max(g.rb * S * l0, g.cw * S * l1) + tw) * elem + S * (l0 + l1) * sizeof(double);
+    return (std::max(g.rb * S * l0, g.cw * S * l1) + tw) * elem + S * (l0 + l1) * factor;
 }
 
 // m = R2 R3 for a line of 8 m points: the stages' radices (see grid_filter),
@@ -528,7 +740,7 @@ static bool grid_radices(int m, int &R2, int &R3) {
     return R2 > 0;
 }
 
-bool grid_shape(int N0, int N1, int S, int cus, GridShape &g) {
+bool grid_shape(int N0, int N1, int S, int cus, bool gspo, GridShape &g) {
     if (S < 1 || S > 2 || N0 % 8 || N1 % 8 || N0 < 8 || N1 < 8) return false;
     if (!grid_radices(N0 / 8, g.R2[0], g.R3[0]) || !grid_radices(N1 / 8, g.R2[1], g.R3[1])) return false;
     for (int d = 0; d < 2; ++d)
@@ -553,7 +765,7 @@ bool grid_shape(int N0, int N1, int S, int cus, GridShape &g) {
     g.blocks = std::max(g.nrb, g.ncb);
     g.threads = std::max(64, round64(std::max(g.rb * S * (N0 / 8), g.cw * S * (N1 / 8))));
     // the 160 KiB of a CU (the tables of two long lines may not fit)
-    return grid_lds_bytes(g, N0, N1, S, 16) <= kLdsBytes - 1024;
+    return grid_lds_bytes(g, N0, N1, S, 16, gspo ? 16 : 8) <= kLdsBytes - 1024;
 }
 
 size_t grid_exchange_len(const GridShape &g, int S) { return (size_t)S * g.nrb * g.rb * g.ncb * g.cw; }
@@ -585,7 +797,7 @@ bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape
                        const LinePlan &p0, const LinePlan &p1, const double *coef, int order, double offset,
                        double offset_i, double inv_scaling, double prec, bool imag, const double *psi, ChebyCtl *ctl,
                        double *partials) {
-    const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, sizeof(cx<R>));
+    const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, sizeof(cx<R>), sizeof(double));
     auto cp = reinterpret_cast<const cx<double> *>(psi);
     const bool nip = offset_i != 0 || h.Wi[0] != nullptr;
     bool ran = false;
@@ -623,10 +835,46 @@ template bool launch_cheby_grid(hipStream_t, int, const HamDev<float> &, const G
                                 const LinePlan &, const LinePlan &, const double *, int, double, double, double, double,
                                 bool, const double *, ChebyCtl *, double *);
 
+template <class R>
+bool launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
+                      bool coupled, const LinePlan &p0, const LinePlan &p1, const double *ek, double inv0, double inv1,
+                      const double *psi) {
+    const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, sizeof(cx<R>), 16);
+    auto cp = reinterpret_cast<const cx<double> *>(psi);
+    bool ran = true;
+    // the parts of a single step wait for nothing
+    auto launch = [&](auto kernel) {
+        if (!a.part) {
+            ran = coop_launch(kernel, g.blocks, g.threads, lds, s, a, g, pre, p0, p1, ek, inv0, inv1, cp);
+            return;
+        }
+        set_lds(kernel, lds);
+        QDX_LAUNCH(kernel, dim3(g.blocks), dim3(g.threads), lds, s, a, g, pre, p0, p1, ek, inv0, inv1, cp);
+        QDX_HIP(hipGetLastError());
+    };
+#define QDX_GRID(S_, MU_, CPL_)                                                                                  \
+    do {                                                                                                         \
+        if (g.primes) launch(k_gspo_grid<R, S_, MU_, CPL_, true>);                                               \
+        else launch(k_gspo_grid<R, S_, MU_, CPL_, false>);                                                       \
+    } while (0)
+    if (mu) QDX_GRID(1, true, false);
+    else if (coupled) QDX_GRID(2, false, true);
+    else if (S == 1) QDX_GRID(1, false, false);
+    else QDX_GRID(2, false, false);
+#undef QDX_GRID
+    return ran;
+}
+template bool launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<double> &, bool,
+                               bool, const LinePlan &, const LinePlan &, const double *, double, double,
+                               const double *);
+template bool launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<float> &, bool,
+                               bool, const LinePlan &, const LinePlan &, const double *, double, double,
+                               const double *);
+
 void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
                         int *report) {
     const int ncopy = (int)std::min<long>(1024, (S * n + 255) / 256);
-    QDX_LAUNCH(k_grid_finish, dim3(ncopy + (obs ? a.nsteps : 0)), dim3(256), 0, s, a, S, n, g.nrb, ncopy,
+    QDX_LAUNCH(k_grid_finish, dim3(ncopy + (obs ? a.nsteps : 0)), dim3(256), 0, s, a, S, n, g.blocks, ncopy,
                reinterpret_cast<cx<double> *>(psi), obs, report);
     QDX_HIP(hipGetLastError());
 }

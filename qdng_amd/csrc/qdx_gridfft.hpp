@@ -304,11 +304,14 @@ __device__ __forceinline__ void grid_tables(const cx<R> *tab, int m, int R3, cx<
     for (int i = threadIdx.x; i < m; i += blockDim.x) tw2[i] = tab[(8 * (i / R3) * (i % R3)) % N];
 }
 // factors f[k] (already scaled by g) at the places of k, by the whole block
-__device__ __forceinline__ void grid_factors(const double *f, double g, int R2, int R3, double *dst) {
+__device__ __forceinline__ double scaled_factor(double f, double g) { return f * g; }
+__device__ __forceinline__ cx<double> scaled_factor(cx<double> f, double g) { return mk<double>(f.r * g, f.i * g); }
+template <class F>
+__device__ __forceinline__ void grid_factors(const F *f, double g, int R2, int R3, F *dst) {
     const int RS = grid_rs(R3), m = R2 * R3;
     for (int i = threadIdx.x; i < 8 * m; i += blockDim.x) {
         const int k1 = i / m, a = (i % m) / R3, b = i % R3;
-        dst[(k1 * R2 + a) * RS + b] = f ? f[k1 + 8 * (a + R2 * b)] * g : 0.0;
+        dst[(k1 * R2 + a) * RS + b] = f ? scaled_factor(f[k1 + 8 * (a + R2 * b)], g) : F{};
     }
 }
 

@@ -558,65 +558,121 @@ void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *
 // qdx_ctx_set_line_points 4 or 8 asks for the per-order kernels
 bool grid_on(const qdx_prop *p) { return p->grid2d && p->ctx->line_ppt == 0; }
 
-// Chebyshev steps first .. first + nsteps - 1 by the persistent kernel, as
-// dense_run; returns the steps done.  Fewer than nsteps when a launch gave up
-// waiting for its blocks (psi is then the state after the steps done): the
-// caller goes on order by order.
+// what a launch of n steps of the persistent kernels needs; signals: the flags'
+// values it uses at most
+GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const double *psi0, int *orders) {
+    GridRun a;
+    a.nsteps = (int)n;
+    a.first = (int)(first & 1);
+    if (p->gepoch > (1u << 30)) {
+        HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, p->ctx->stream));
+        p->gepoch = 0;
+    }
+    a.epoch = p->gepoch;
+    p->gepoch += signals;
+    a.sync = p->gflags.as<char>();
+    a.status = reinterpret_cast<int *>(a.sync + kGridSyncBytes);
+    a.A = p->phiA.p;
+    a.B = p->phiB.p;
+    a.out = p->X.as<double>();
+    const size_t obytes = (size_t)n * 3 * p->S * p->gs.blocks * sizeof(double);
+    if (p->gobs.bytes < obytes) p->gobs.alloc(obytes);   // no launch is in flight here
+    a.obsp = p->gobs.as<double>();
+    a.psi0 = psi0;
+    a.orders = orders;
+    return a;
+}
+
+// After a launch (ran: it was made): psi and the observables; false, and the
+// propagator keeps to the per-order kernels from then on, when the launch was
+// not made or gave up waiting for its blocks (psi is unchanged then).
+bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, bool ran, double *obs) {
+    hipStream_t s = p->ctx->stream;
+    if (ran) {
+        launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->greport);
+        HIPCHK(hipStreamSynchronize(s));
+        if (!*p->greport) return true;
+        HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, s));
+        p->gepoch = 0;
+    }
+    p->grid2d = false;
+    return false;
+}
+
+// Steps first .. first + nsteps - 1 by the persistent kernels, as dense_run;
+// returns the steps done, fewer than nsteps when a launch failed (grid_end):
+// the caller goes on with the per-order kernels.  split: a single step by
+// ordinary launches where there are such (split operator).
 template <class R>
 long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
-              StreamKeep &keep) {
+              StreamKeep &keep, bool split) {
     qdx_ctx *ctx = p->ctx;
     const int S = p->S;
-    const bool fp32 = std::is_same<R, float>::value;
+    const bool fp32 = std::is_same<R, float>::value, cheby = p->kind == qdx_prop::CHEBY;
     const LinePlan p0 = ctx->plan_ppt(p->grid.N[0], fp32, 4), p1 = ctx->plan_ppt(p->grid.N[1], fp32, 4);
-    const HamDev<R> *h;
-    if constexpr (std::is_same<R, float>::value) h = &p->ham->dev.h32;
-    else h = &p->ham->dev.h64;
-    qdx_ham *fop = p->ham->time_dependent() ? p->ham : nullptr;
-    // a launch runs at most 2048 orders: tens of milliseconds
-    const long most = std::max(1L, 2048L / std::max(p->k_launch, 1));
+    auto dev = [](qdx_ham *o) -> const HamDev<R> & {
+        if constexpr (std::is_same<R, float>::value) return o->dev.h32;
+        else return o->dev.h64;
+    };
+    qdx_ham *fop = nullptr;   // the operator whose field changes with the clock
+    if (cheby) {
+        if (p->ham->time_dependent()) fop = p->ham;
+    } else {
+        for (qdx_ham *o : p->ops)
+            if (o->time_dependent()) fop = o;
+    }
+    // split operators: those ahead of the kinetic one (p->ops[0]); the ones
+    // behind it are the same in reverse order, and they commute (grid2d)
+    XGroupDev<R> pre;
+    bool coupled = false;
+    const double *ek = nullptr;
+    if (!cheby) {
+        pre.n = 0;
+        for (size_t i = p->ops.size() - 1; i > 0; --i) pre.op[pre.n++] = xsplit<R>(p, p->ops[i], p->dt * 0.5, first);
+        for (int i = 0; i < pre.n; ++i) coupled = coupled || pre.op[i].coupled;
+        ek = kinetic_exp_table(p, p->ops[0], p->dt);
+    }
+    // a launch runs at most 2048 orders or split-operator steps: tens of
+    // milliseconds
+    const long most = cheby ? std::max(1L, 2048L / std::max(p->k_launch, 1)) : 2048L;
     for (long i = 0; i < nsteps;) {
         long n = std::min(most, nsteps - i);
-        GridRun a;
+        const double *fields = nullptr;
+        double field0[kMaxStates * kMaxStates] = {};
         std::function<void()> late;
-        if (fop) n = run_fields(p, fop, S * S, first + i, n, std::min(most, nsteps), a.field0, &a.fields, late, keep);
-        a.nsteps = (int)n;
-        if (p->gepoch > (1u << 30)) {
-            HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, ctx->stream));
-            p->gepoch = 0;
+        if (fop)
+            n = run_fields(p, fop, cheby ? S * S : 1, first + i, n, std::min(most, nsteps), field0, &fields, late, keep);
+        if (!cheby && split) {
+            // a single step in two launches, psi in place
+            GridRun a = grid_args(p, first, 1, 0, nullptr, nullptr);
+            std::copy(field0, field0 + kMaxStates * kMaxStates, a.field0);
+            a.out = psi->ptr();
+            const HamDev<R> &h = dev(p->ops[0]);
+            for (a.part = 1; a.part <= 2; ++a.part) {
+                KTimer t(ctx, QDX_K_GSPO_ROW);
+                launch_gspo_grid<R>(ctx->stream, S, p->gs, a, pre, fop != nullptr, coupled, p0, p1, ek, h.inv_nd[0],
+                                    h.inv_nd[1], psi->ptr());
+            }
+            return 1;
         }
-        a.epoch = p->gepoch;
-        p->gepoch += 2u * (unsigned)(p->k_launch * n);
-        a.sync = p->gflags.as<char>();
-        a.status = reinterpret_cast<int *>(a.sync + kGridSyncBytes);
-        a.A = p->phiA.p;
-        a.B = p->phiB.p;
-        a.out = p->X.as<double>();
-        const size_t obytes = (size_t)n * 3 * S * p->gs.nrb * sizeof(double);
-        if (p->gobs.bytes < obytes) p->gobs.alloc(obytes);   // no launch is in flight here
-        a.obsp = p->gobs.as<double>();
-        a.psi0 = psi0;
-        a.orders = orders ? orders + i : nullptr;
+        GridRun a = grid_args(p, first + i, n, (unsigned)(cheby ? 2 * p->k_launch * n : n), psi0,
+                              orders ? orders + i : nullptr);
+        a.fields = fields;
+        std::copy(field0, field0 + kMaxStates * kMaxStates, a.field0);
+        a.observe = obs != nullptr;
         bool ran;
-        {
+        if (cheby) {
             KTimer t(ctx, QDX_K_CHEBY_ROW);
-            ran = launch_cheby_grid<R>(ctx->stream, S, *h, p->gs, a, p0, p1, p->coefd.as<double>(), p->k_launch,
-                                       p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec, p->imag,
-                                       psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
+            ran = launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), p->gs, a, p0, p1, p->coefd.as<double>(),
+                                       p->k_launch, p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec,
+                                       p->imag, psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
+        } else {
+            KTimer t(ctx, QDX_K_GSPO_ROW);
+            const HamDev<R> &h = dev(p->ops[0]);
+            ran = launch_gspo_grid<R>(ctx->stream, S, p->gs, a, pre, fop != nullptr, coupled, p0, p1, ek, h.inv_nd[0],
+                                      h.inv_nd[1], psi->ptr());
         }
-        if (!ran) {
-            p->grid2d = false;
-            return i;
-        }
-        launch_grid_finish(ctx->stream, S, psi->n(), p->gs, a, psi->ptr(), obs ? obs + (size_t)i * 4 * S : nullptr,
-                           p->greport);
-        HIPCHK(hipStreamSynchronize(ctx->stream));
-        if (*p->greport) {
-            HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, ctx->stream));
-            p->gepoch = 0;
-            p->grid2d = false;
-            return i;
-        }
+        if (!grid_end(p, psi, a, ran, obs ? obs + (size_t)i * 4 * S : nullptr)) return i;
         p->last_nb = p->gs.nrb;
         p->nb_init = p->gs.nrb;
         if (late) late();
@@ -625,9 +681,31 @@ long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *p
     return nsteps;
 }
 long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
-              StreamKeep &keep) {
-    return p->precision == QDX_FP32_BULK ? grid_run<float>(p, psi, first, nsteps, psi0, obs, orders, keep)
-                                         : grid_run<double>(p, psi, first, nsteps, psi0, obs, orders, keep);
+              StreamKeep &keep, bool split = false) {
+    return p->precision == QDX_FP32_BULK ? grid_run<float>(p, psi, first, nsteps, psi0, obs, orders, keep, split)
+                                         : grid_run<double>(p, psi, first, nsteps, psi0, obs, orders, keep, split);
+}
+
+// The exchange buffers, flags and staging of the persistent kernels (p->gs is
+// set); es: bytes of an exchanged value.
+void grid_buffers(qdx_prop *p, size_t es) {
+    const size_t nval = (size_t)p->S * p->grid.size(), nx = std::max(nval, grid_exchange_len(p->gs, p->S));
+    p->phiA.alloc(nx * es);
+    p->phiB.alloc(nx * es);
+    p->X.alloc(nval * 16);
+    p->gflags.alloc(kGridSyncBytes + sizeof(int));
+    HIPCHK(hipMemset(p->gflags.p, 0, p->gflags.bytes));
+    HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&p->greport), sizeof(int), hipHostMallocDefault));
+}
+
+// the block shape of a 2D grid on this device; false: it takes the per-order
+// kernels
+bool grid_fits(qdx_prop *p) {
+    if (p->grid.nd != 2) return false;
+    int cus = 0, coop = 0;
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->ctx->device));
+    HIPCHK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, p->ctx->device));
+    return coop && grid_shape(p->grid.N[0], p->grid.N[1], p->S, cus, p->kind == qdx_prop::GSPO, p->gs);
 }
 
 // |norm0 - accnorm| / norm0 of the last executed order of the last step
@@ -658,29 +736,34 @@ double cheby_last_nconv(qdx_prop *p) {
 void sil_step(qdx_prop *p, qdx_wf *psi, long step);
 void arnoldi_step(qdx_prop *p, qdx_wf *psi, long step);
 
-void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step);
+void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32);
+
+// steps of a propagation that keeps to the persistent kernels.  Backward
+// split-operator steps, which run one by one, take the per-order kernels: one
+// launch that is waited for costs more than their three.
+bool grid_steps(const qdx_prop *p) { return grid_on(p) && !(p->kind == qdx_prop::GSPO && p->backward); }
 
 // FP32 split-operator propagation holds psi in FP32 between the steps (the
-// dense line kernels keep complex128)
+// dense line kernels and the persistent ones keep complex128 between launches)
 bool psi_in_fp32(const qdx_prop *p) {
-    return p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK && !dense_on(p);
+    return p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK && !dense_on(p) && !grid_steps(p);
 }
 
 // OPropagator::Backward() in real time (exponent +i dt, with the operators
 // conjugated, OPropagator.h:82-100): exp(+i H* dt) psi = conj(exp(-i H dt)
 // conj(psi)), the forward step between two conjugations (exact: conjugation
 // commutes with every rounding of the forward step)
-void prop_step(qdx_prop *p, qdx_wf *psi, long step) {
-    if (!p->backward) return prop_step_forward(p, psi, step);
-    const bool g32 = psi_in_fp32(p);
+// g32: the caller holds psi in FP32 (psi_in_fp32 when it began)
+void prop_step(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
+    if (!p->backward) return prop_step_forward(p, psi, step, g32);
     void *d = g32 ? static_cast<void *>(p->psi32.as<float>()) : static_cast<void *>(psi->ptr());
     const long n = (long)p->S * psi->n();
     launch_conj(p->ctx->stream, d, n, g32);
-    prop_step_forward(p, psi, step);
+    prop_step_forward(p, psi, step, g32);
     launch_conj(p->ctx->stream, d, n, g32);
 }
 
-void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step) {
+void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
     if (p->kind == qdx_prop::SIL) {
         sil_step(p, psi, step);
         return;
@@ -694,9 +777,9 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step) {
         dense_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep);
         return;
     }
-    if (grid_on(p)) {
+    if (grid_steps(p) && !g32) {
         StreamKeep keep{p->ctx->stream, {}};
-        if (grid_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep) == 1) return;
+        if (grid_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep, true) == 1) return;
     }
     if (p->kind == qdx_prop::CHEBY) {
         // QDX_COMPACT: FP64 arithmetic (compact terms when p->cmp)
@@ -704,8 +787,15 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step) {
         else cheby_step<double>(p, psi, step);
         // record executed order count of this step
     } else {
-        if (p->precision == QDX_FP32_BULK) gspo_step<float>(p, p->psi32.as<float>(), step);
-        else gspo_step<double>(p, psi->ptr(), step);
+        if (p->precision == QDX_FP32_BULK) {
+            // the caller holds psi in complex128 when a persistent launch failed
+            const long n = (long)p->S * psi->n();
+            if (!g32) launch_convert_c128_to_c64(p->ctx->stream, psi->ptr(), p->psi32.as<float>(), n);
+            gspo_step<float>(p, p->psi32.as<float>(), step);
+            if (!g32) launch_convert_c64_to_c128(p->ctx->stream, p->psi32.as<float>(), psi->ptr(), n);
+        } else {
+            gspo_step<double>(p, psi->ptr(), step);
+        }
     }
 }
 
@@ -1306,21 +1396,14 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
         if (precision == QDX_FP32_BULK) h->ensure32();
         // element bytes of the term buffers (compact: 8 hi + 2 lo)
         const size_t es = p->cmp ? 10 : precision == QDX_FP32_BULK ? 2 * sizeof(float) : 2 * sizeof(double);
-        // 2D grids that fit the chip's registers: X holds complex128 there,
-        // compact terms are exchanged as complex128
-        int cus = 0, coop = 0;
-        HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->ctx->device));
-        HIPCHK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, p->ctx->device));
-        p->grid2d = coop && p->grid.nd == 2 && grid_shape(p->grid.N[0], p->grid.N[1], p->S, cus, p->gs);
-        const size_t nval = (size_t)p->S * p->grid.size();
-        const size_t nbytes = p->grid2d ? std::max(nval, grid_exchange_len(p->gs, p->S)) * (p->cmp ? 16 : es) : nval * es;
-        p->phiA.alloc(nbytes);
-        p->phiB.alloc(nbytes);
-        if (p->grid.nd > 1) p->X.alloc(p->grid2d ? nval * 16 : nbytes);
+        p->grid2d = grid_fits(p.get());
         if (p->grid2d) {
-            p->gflags.alloc(kGridSyncBytes + sizeof(int));
-            HIPCHK(hipMemset(p->gflags.p, 0, p->gflags.bytes));
-            HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&p->greport), sizeof(int), hipHostMallocDefault));
+            grid_buffers(p.get(), p->cmp ? 16 : es);   // compact terms are exchanged as complex128
+        } else {
+            const size_t nbytes = (size_t)p->S * p->grid.size() * es;
+            p->phiA.alloc(nbytes);
+            p->phiB.alloc(nbytes);
+            if (p->grid.nd > 1) p->X.alloc(nbytes);
         }
         p->ctl.alloc(sizeof(ChebyCtl));
         HIPCHK(hipMemset(p->ctl.p, 0, sizeof(ChebyCtl)));
@@ -1470,6 +1553,17 @@ static void gspo_create_impl(qdx_ham *const *ops, int32_t nops, double dt, int32
             p->dtab.alloc(t.size() * sizeof(double));
             HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         }
+        // 2D grids in real time, by the same rule (several x-space operators
+        // commute when none couples two states)
+        bool coupled = false;
+        for (qdx_ham *o : p->ops)
+            for (auto &t : o->terms) coupled = coupled || t.row != t.col;
+        p->grid2d = !imag && nkin == 1 && p->ops[0]->terms[0].kind == T_KIN && nx <= (coupled ? 1 : kMaxXOps) &&
+                    nfield <= (p->S == 1 ? 1 : 0) && grid_fits(p.get());
+        if (p->grid2d) {
+            grid_buffers(p.get(), es);
+            HIPCHK(hipDeviceSynchronize());
+        }
         ctx_acquire(p->ctx);
         *out = p.release();
     }
@@ -1490,7 +1584,7 @@ int qdx_prop_apply(qdx_prop *p, qdx_wf *psi, int64_t step, qdx_step_stats *stats
         hipStream_t s = p->ctx->stream;
         const bool g32 = psi_in_fp32(p);
         if (g32) launch_convert_c128_to_c64(s, psi->ptr(), p->psi32.as<float>(), (long)p->S * psi->n());
-        prop_step(p, psi, step);
+        prop_step(p, psi, step, g32);
         if (g32)
             launch_convert_c64_to_c128(s, p->psi32.as<float>(), psi->ptr(), (long)p->S * psi->n());
         if (stats) {
@@ -1532,12 +1626,27 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
         hipStream_t s = p->ctx->stream;
         const int S = p->S;
         const long n = psi->n();
-        const bool g32 = psi_in_fp32(p);
         // device observables: per step, per state (re, im) of <psi|psi> and <psi|psi0>
         const size_t per_step = 4 * S;
         p->obs.alloc(std::max<size_t>(1, (size_t)nsteps * per_step + nsteps) * sizeof(double));
         double *obs = p->obs.as<double>();
         int *orders = reinterpret_cast<int *>(obs + nsteps * per_step);
+        // whole runs by one kernel (an autocorrelation with the propagated
+        // function itself follows it step by step)
+        const bool whole = !p->backward && !(autocorr && psi0->ptr() == psi->ptr());
+        StreamKeep keep{s, {}};
+        int64_t done = 0;
+        if (whole && (dense_on(p) || grid_steps(p))) {
+            const double *z = autocorr ? psi0->ptr() : nullptr;
+            double *o = norm2 || autocorr ? obs : nullptr;
+            int *ord = p->kind == qdx_prop::CHEBY ? orders : nullptr;
+            done = nsteps;
+            if (dense_on(p)) dense_run(p, psi, first_step, nsteps, z, o, ord, keep);
+            else done = grid_run(p, psi, first_step, nsteps, z, o, ord, keep);
+        }
+        // (split operator: the fused run, which reads that psi0 before it writes psi)
+        const bool self = !whole && !p->backward && gspo_fusable(p).ok;
+        const bool g32 = psi_in_fp32(p) || (self && p->precision == QDX_FP32_BULK);
         if (g32) {
             launch_convert_c128_to_c64(s, psi->ptr(), p->psi32.as<float>(), (long)S * n);
             if (autocorr) {
@@ -1549,7 +1658,7 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
         if (!part || p->partials.bytes < kMaxPartials * sizeof(double))
             fail(QDX_ERR_STATE, "propagator has no reduction buffer for the observables");
         std::vector<int> sil_counts;
-        const bool fused = nsteps > 0 && !p->backward && gspo_fusable(p).ok;
+        const bool fused = done == 0 && nsteps > 0 && !p->backward && (self || !grid_on(p)) && gspo_fusable(p).ok;
         if (fused) {
             // observables before step 0 here; those before the later steps
             // from the row passes between the steps (psi0: autocorrelation)
@@ -1569,18 +1678,7 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
                 gspo_run_fused<double>(p, ps, p0, first_step, nsteps, want ? obs : nullptr, per_step);
             }
         }
-        // (an autocorrelation with the propagated function itself follows it
-        // step by step)
-        const bool whole = !p->backward && !(autocorr && psi0->ptr() == psi->ptr());
-        const bool dense = dense_on(p) && whole;
-        StreamKeep keep{s, {}};
-        if (dense)
-            dense_run(p, psi, first_step, nsteps, autocorr ? psi0->ptr() : nullptr, norm2 || autocorr ? obs : nullptr,
-                      p->kind == qdx_prop::CHEBY ? orders : nullptr, keep);
-        int64_t done = fused || dense ? nsteps : 0;
-        if (grid_on(p) && whole)
-            done = grid_run(p, psi, first_step, nsteps, autocorr ? psi0->ptr() : nullptr,
-                            norm2 || autocorr ? obs : nullptr, orders, keep);
+        if (fused) done = nsteps;
         for (int64_t i = done; i < nsteps; ++i) {
             double *o = obs + i * per_step;
             if (norm2) {
@@ -1591,7 +1689,7 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
                 if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi0_32.as<float>(), n, S, part, o + 2 * S);
                 else launch_overlap(s, psi->ptr(), psi0->ptr(), n, S, part, o + 2 * S);
             }
-            prop_step(p, psi, first_step + i);
+            prop_step(p, psi, first_step + i, g32);
             if (p->kind == qdx_prop::CHEBY)
                 HIPCHK(hipMemcpyAsync(orders + i, &p->ctl.as<ChebyCtl>()->last_order, sizeof(int),
                                       hipMemcpyDeviceToDevice, s));
@@ -1984,7 +2082,7 @@ int qdx_eigen_imag(qdx_prop *U, qdx_ham *Hin, const qdx_wf *psi0, int32_t nef, i
             double dff = 1;
             while (s < max_steps && dff > conv) {
                 chk(qdx_wf_copy(psi_old, psi));
-                prop_step(U, psi, s);
+                prop_step(U, psi, s, psi_in_fp32(U));
                 if (i > 0) {   // OProjection::Apply (OProjection.cpp:133-149), psi -= P psi
                     std::vector<std::complex<double>> c(i);
                     for (int j = 0; j < i; ++j) ovl(ef[j], psi, c[j]);
@@ -2038,7 +2136,7 @@ int qdx_eigen_ac(qdx_prop *U, qdx_ham *Hin, const qdx_wf *psi0, int32_t nsteps, 
         qdx_wf *psi = tmp.make(p0);
         chk(qdx_wf_copy(psi, p0));
         for (int i = 1; i < N; ++i) {
-            prop_step(U, psi, i - 1);
+            prop_step(U, psi, i - 1, psi_in_fp32(U));
             ovl(psi, p0, ac[i]);
             if (std::isnan(ac[i].real())) fail(QDX_ERR_OVERFLOW, "Correlation is not a number");
         }
@@ -2074,7 +2172,7 @@ int qdx_eigen_ac(qdx_prop *U, qdx_ham *Hin, const qdx_wf *psi0, int32_t nsteps, 
         U->arn_order = arn_order0;
         chk(qdx_wf_copy(psi, p0));
         for (int s = 1; s < N; ++s) {
-            prop_step(U, psi, s - 1);
+            prop_step(U, psi, s - 1, psi_in_fp32(U));
             for (int k = 0; k < n_ef; ++k) {
                 const double ph = ek[k] * double(s) * dt;
                 chk(qdx_wf_axpy(ef[k], std::cos(ph), std::sin(ph), psi));

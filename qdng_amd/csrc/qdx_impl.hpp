@@ -205,12 +205,15 @@ struct GridShape {
 };
 struct GridRun {
     int nsteps = 0;
+    int first = 0;                    // parity of the first step's number
+    int part = 0;                     // GSPO: 1, 2 the parts of a single step, 0 a whole run
+    bool observe = false;             // partial sums of the observables are wanted (GSPO)
     unsigned epoch = 0;               // flags reach at most epoch + 2 orders nsteps
     char *sync = nullptr;             // flags and partial sums (kGridSyncBytes)
     int *status = nullptr;            // set by a run that gave up waiting
     void *A = nullptr, *B = nullptr;  // exchange buffers (grid_exchange_len values of the kernel precision)
     double *out = nullptr;            // the final psi (complex128)
-    double *obsp = nullptr;           // per step, state and observable (3) one partial sum per row block
+    double *obsp = nullptr;           // per step, state and observable (3) one partial sum per block
     const double *fields = nullptr;   // as DenseRun
     double field0[kMaxStates * kMaxStates] = {};
     const double *psi0 = nullptr;
@@ -313,13 +316,17 @@ void launch_dense_gspo(hipStream_t s, int S, const XGroupDev<double> &pre, const
 // launch_cheby_grid: false when the device does not hold all blocks at once.
 // launch_grid_finish: psi, the observables (nullable) and the status of the
 // run after launch_cheby_grid.
-bool grid_shape(int N0, int N1, int S, int cus, GridShape &g);
+bool grid_shape(int N0, int N1, int S, int cus, bool gspo, GridShape &g);
 size_t grid_exchange_len(const GridShape &g, int S);
 template <class R>
 bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
                        const LinePlan &p0, const LinePlan &p1, const double *coef, int order, double offset,
                        double offset_i, double inv_scaling, double prec, bool imag, const double *psi, ChebyCtl *ctl,
                        double *partials);
+template <class R>
+bool launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
+                      bool coupled, const LinePlan &p0, const LinePlan &p1, const double *ek, double inv0, double inv1,
+                      const double *psi);
 void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
                         int *report);
 

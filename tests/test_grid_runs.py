@@ -141,3 +141,45 @@ def test_long_run_and_own_autocorrelation(ctx):
     assert len(nh) == 250 and min(nh) > 3
     n2, ac, _, _ = U.run(w, 0, 3, w)
     assert np.allclose(ac, n2, rtol=1e-12)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("fp32", 1e-5)])
+@pytest.mark.parametrize("N0,N1,S,laser,coupled", [
+    (8, 8, 1, False, False), (8, 16, 2, False, True), (104, 88, 1, True, False), (40, 56, 2, False, False),
+    (16, 768, 1, True, False), (768, 16, 2, False, True), (240, 176, 1, True, False), (232, 248, 2, False, True),
+    (256, 256, 1, False, False), (768, 512, 1, True, False), (512, 512, 2, False, True), (768, 768, 2, False, True)])
+def test_gspo(N0, N1, S, laser, coupled, precision, tol):
+    """Runs of odd and even length from an odd step on, single steps, the
+    observables in both layouts."""
+    import qdng_amd as Q
+    print("[gpu case] grid gspo", N0, N1, S, laser, coupled, precision, flush=True)
+
+    def make(c):
+        p = box(N0, N1, S, laser, coupled=coupled)
+        ops = [p.gpu_split_op(c, [k]) for k in (("kin", "pot", "dip") if laser else ("kin", "pot"))]
+        return p, Q.GSPO(ops, 2.0, precision=precision)
+    check(both(make, 5, True), tol)
+    check(both(make, 8, True), tol)
+    check(both(make, 3, False), tol)
+
+
+def test_gspo_steps_and_runs_agree(ctx):
+    """Single steps give the bits of a run longer than one launch; backward
+    steps lead back; a psi0 that is psi itself stands for the initial state."""
+    import qdng_amd as Q
+    p = box(40, 24, 1, laser=True, nt=2100)
+    G = Q.GSPO([p.gpu_split_op(ctx, [k]) for k in ("kin", "pot", "dip")], 0.5)
+    w, ref, w0 = p.gpu_wf(ctx), p.gpu_wf(ctx), p.gpu_wf(ctx)
+    _, ac, _, _ = G.run(w, 0, 2060, w0)
+    for i in range(2060):
+        G.apply(ref, i)
+    assert np.array_equal(w.download(), ref.download())
+    self = p.gpu_wf(ctx)
+    _, ac_self, _, _ = G.run(self, 0, 50, self)
+    assert np.allclose(ac_self, ac[:50], rtol=1e-11)
+    G.backward()
+    G.run(w, 2059, 1)
+    G.run(w, 2058, 1)
+    G.backward(False)
+    G.run(w, 2058, 2)
+    assert rel(w.download(), ref.download()) < 1e-12
