@@ -1,5 +1,5 @@
 // gfx950 persistent kernels of 2D grids that fit the chip's registers: whole
-// Chebyshev runs in one cooperative launch.
+// Chebyshev and split-operator runs in one launch.
 //
 // A 2D grid of up to 2^19 points and states is bound by latency when every
 // order is two launches (row kernel and column pass): each of them reads its
@@ -26,16 +26,21 @@
 // only the store counter before the block's flag is raised.  Flags hold
 // epochs that grow over all launches of a propagator.
 //
-// Every wait is bounded (kGridWait): a block that gives up leaves, the others
-// follow, and the host, which keeps psi until the launch is known to be
-// complete, runs the steps again order by order.
+// All blocks have to be on the chip together: there are at most as many as
+// CUs, each fits a CU by itself, and the host lets one such launch run per
+// device and process at a time.  (Cooperative launches would say so to the
+// runtime, but they cost 20 us more, and once a process has made one its other
+// streams run slower: a batch of jobs 34 -> 45 ms.)  Other processes on the
+// GPU can still hold CUs, so every wait is bounded (kGridWait): a block that
+// gives up leaves, the others follow, and the host, which keeps psi until the
+// launch is known to be complete, runs the steps again order by order.
 #include "qdx_gridfft.hpp"
 #include "qdx_xsplit.hpp"
 
 namespace qdx {
 
-// bound of one wait in ticks of the 100 MHz wall clock: 2 s
-constexpr unsigned long long kGridWait = 200000000ull;
+// bound of one wait in ticks of the 100 MHz wall clock: 0.1 s
+constexpr unsigned long long kGridWait = 10000000ull;
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -770,45 +775,25 @@ bool grid_shape(int N0, int N1, int S, int cus, bool gspo, GridShape &g) {
 
 size_t grid_exchange_len(const GridShape &g, int S) { return (size_t)S * g.nrb * g.rb * g.ncb * g.cw; }
 
-// false: the device does not hold all blocks at once
-template <class K, class... Args>
-static bool coop_launch(K kernel, int blocks, int threads, size_t lds, hipStream_t s, Args... args) {
-    set_lds(kernel, lds);
-    void *argv[] = {(void *)&args...};
-    const LaunchTiming t = g_launch_timing;
-    if (t.start) QDX_HIP(hipEventRecord(t.start, s));
-    const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(kernel), dim3(blocks),
-                                                    dim3(threads), argv, (unsigned)lds, s);
-    if (e == hipErrorCooperativeLaunchTooLarge) {
-        (void)hipGetLastError();
-        g_launch_timing = LaunchTiming();
-        return false;
-    }
-    QDX_HIP(e);
-    if (t.start) {
-        QDX_HIP(hipEventRecord(t.stop, s));
-        g_launch_timing = LaunchTiming();
-    }
-    return true;
-}
-
 template <class R>
-bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
+void launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
                        const LinePlan &p0, const LinePlan &p1, const double *coef, int order, double offset,
                        double offset_i, double inv_scaling, double prec, bool imag, const double *psi, ChebyCtl *ctl,
                        double *partials) {
     const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, sizeof(cx<R>), sizeof(double));
     auto cp = reinterpret_cast<const cx<double> *>(psi);
     const bool nip = offset_i != 0 || h.Wi[0] != nullptr;
-    bool ran = false;
 #define QDX_GRID(S_, IMAG_, NIP_)                     \
     do {                                              \
         if (g.primes) QDX_GRIDP(S_, IMAG_, NIP_, true); \
         else QDX_GRIDP(S_, IMAG_, NIP_, false);       \
     } while (0)
-#define QDX_GRIDP(S_, IMAG_, NIP_, PR_)                                                                      \
-    ran = coop_launch(k_cheby_grid<R, S_, IMAG_, NIP_, PR_>, g.blocks, g.threads, lds, s, a, g, h, p0, p1, coef, order, offset, \
-                nip ? offset_i : 0.0, inv_scaling, prec, cp, ctl, partials)
+#define QDX_GRIDP(S_, IMAG_, NIP_, PR_)                                                                        \
+    do {                                                                                                       \
+        set_lds(k_cheby_grid<R, S_, IMAG_, NIP_, PR_>, lds);                                                   \
+        QDX_LAUNCH((k_cheby_grid<R, S_, IMAG_, NIP_, PR_>), dim3(g.blocks), dim3(g.threads), lds, s, a, g, h,  \
+                   p0, p1, coef, order, offset, nip ? offset_i : 0.0, inv_scaling, prec, cp, ctl, partials);   \
+    } while (0)
     if (nip) {
         if (S != 1 || imag) throw std::runtime_error("negative imaginary potential: one state, real time only");
         QDX_GRID(1, false, true);
@@ -826,28 +811,22 @@ bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape
     }
 #undef QDX_GRID
 #undef QDX_GRIDP
-    return ran;
+    QDX_HIP(hipGetLastError());
 }
-template bool launch_cheby_grid(hipStream_t, int, const HamDev<double> &, const GridShape &, const GridRun &,
+template void launch_cheby_grid(hipStream_t, int, const HamDev<double> &, const GridShape &, const GridRun &,
                                 const LinePlan &, const LinePlan &, const double *, int, double, double, double, double,
                                 bool, const double *, ChebyCtl *, double *);
-template bool launch_cheby_grid(hipStream_t, int, const HamDev<float> &, const GridShape &, const GridRun &,
+template void launch_cheby_grid(hipStream_t, int, const HamDev<float> &, const GridShape &, const GridRun &,
                                 const LinePlan &, const LinePlan &, const double *, int, double, double, double, double,
                                 bool, const double *, ChebyCtl *, double *);
 
 template <class R>
-bool launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
+void launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
                       bool coupled, const LinePlan &p0, const LinePlan &p1, const double *ek, double inv0, double inv1,
                       const double *psi) {
     const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, sizeof(cx<R>), 16);
     auto cp = reinterpret_cast<const cx<double> *>(psi);
-    bool ran = true;
-    // the parts of a single step wait for nothing
     auto launch = [&](auto kernel) {
-        if (!a.part) {
-            ran = coop_launch(kernel, g.blocks, g.threads, lds, s, a, g, pre, p0, p1, ek, inv0, inv1, cp);
-            return;
-        }
         set_lds(kernel, lds);
         QDX_LAUNCH(kernel, dim3(g.blocks), dim3(g.threads), lds, s, a, g, pre, p0, p1, ek, inv0, inv1, cp);
         QDX_HIP(hipGetLastError());
@@ -862,12 +841,11 @@ bool launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a
     else if (S == 1) QDX_GRID(1, false, false);
     else QDX_GRID(2, false, false);
 #undef QDX_GRID
-    return ran;
 }
-template bool launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<double> &, bool,
+template void launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<double> &, bool,
                                bool, const LinePlan &, const LinePlan &, const double *, double, double,
                                const double *);
-template bool launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<float> &, bool,
+template void launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<float> &, bool,
                                bool, const LinePlan &, const LinePlan &, const double *, double, double,
                                const double *);
 

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -583,26 +584,31 @@ GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const doubl
     return a;
 }
 
-// After a launch (ran: it was made): psi and the observables; false, and the
-// propagator keeps to the per-order kernels from then on, when the launch was
-// not made or gave up waiting for its blocks (psi is unchanged then).
-bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, bool ran, double *obs) {
+// After a launch: psi and the observables; false, and the propagator keeps to
+// the per-order kernels from then on, when it gave up waiting for its blocks
+// (psi is unchanged then).
+bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, double *obs) {
     hipStream_t s = p->ctx->stream;
-    if (ran) {
-        launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->greport);
-        HIPCHK(hipStreamSynchronize(s));
-        if (!*p->greport) return true;
-        HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, s));
-        p->gepoch = 0;
-    }
+    launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->greport);
+    HIPCHK(hipStreamSynchronize(s));
+    if (!*p->greport) return true;
+    HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, s));
+    p->gepoch = 0;
     p->grid2d = false;
     return false;
 }
 
+// Two persistent launches at once could each hold CUs that the other waits
+// for: one at a time per device (held from the launch to its end).
+std::mutex &grid_mutex(int device) {
+    static std::mutex m[64];
+    return m[device & 63];
+}
+
 // Steps first .. first + nsteps - 1 by the persistent kernels, as dense_run;
-// returns the steps done, fewer than nsteps when a launch failed (grid_end):
+// returns the steps done, fewer than nsteps when a launch gave up (grid_end):
 // the caller goes on with the per-order kernels.  split: a single step by
-// ordinary launches where there are such (split operator).
+// launches that wait for nothing, where there are such (split operator).
 template <class R>
 long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
               StreamKeep &keep, bool split) {
@@ -660,19 +666,19 @@ long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *p
         a.fields = fields;
         std::copy(field0, field0 + kMaxStates * kMaxStates, a.field0);
         a.observe = obs != nullptr;
-        bool ran;
+        std::lock_guard<std::mutex> alone(grid_mutex(ctx->device));
         if (cheby) {
             KTimer t(ctx, QDX_K_CHEBY_ROW);
-            ran = launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), p->gs, a, p0, p1, p->coefd.as<double>(),
+            launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), p->gs, a, p0, p1, p->coefd.as<double>(),
                                        p->k_launch, p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec,
                                        p->imag, psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
         } else {
             KTimer t(ctx, QDX_K_GSPO_ROW);
             const HamDev<R> &h = dev(p->ops[0]);
-            ran = launch_gspo_grid<R>(ctx->stream, S, p->gs, a, pre, fop != nullptr, coupled, p0, p1, ek, h.inv_nd[0],
+            launch_gspo_grid<R>(ctx->stream, S, p->gs, a, pre, fop != nullptr, coupled, p0, p1, ek, h.inv_nd[0],
                                       h.inv_nd[1], psi->ptr());
         }
-        if (!grid_end(p, psi, a, ran, obs ? obs + (size_t)i * 4 * S : nullptr)) return i;
+        if (!grid_end(p, psi, a, obs ? obs + (size_t)i * 4 * S : nullptr)) return i;
         p->last_nb = p->gs.nrb;
         p->nb_init = p->gs.nrb;
         if (late) late();
@@ -702,10 +708,9 @@ void grid_buffers(qdx_prop *p, size_t es) {
 // kernels
 bool grid_fits(qdx_prop *p) {
     if (p->grid.nd != 2) return false;
-    int cus = 0, coop = 0;
+    int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->ctx->device));
-    HIPCHK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, p->ctx->device));
-    return coop && grid_shape(p->grid.N[0], p->grid.N[1], p->S, cus, p->kind == qdx_prop::GSPO, p->gs);
+    return grid_shape(p->grid.N[0], p->grid.N[1], p->S, cus, p->kind == qdx_prop::GSPO, p->gs);
 }
 
 // |norm0 - accnorm| / norm0 of the last executed order of the last step
@@ -788,7 +793,7 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
         // record executed order count of this step
     } else {
         if (p->precision == QDX_FP32_BULK) {
-            // the caller holds psi in complex128 when a persistent launch failed
+            // the caller holds psi in complex128 when a persistent launch gave up
             const long n = (long)p->S * psi->n();
             if (!g32) launch_convert_c128_to_c64(p->ctx->stream, psi->ptr(), p->psi32.as<float>(), n);
             gspo_step<float>(p, p->psi32.as<float>(), step);

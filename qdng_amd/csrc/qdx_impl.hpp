@@ -311,20 +311,19 @@ void launch_dense_gspo(hipStream_t s, int S, const XGroupDev<double> &pre, const
                        const DenseRun &a, const double *tabr, const double *tabi, bool mu, bool coupled,
                        double *psi);
 
-// Whole runs of a 2D grid in one cooperative launch (qdx_grid.hip).
+// Whole runs of a 2D grid in one launch (qdx_grid.hip).
 // grid_shape: false when the grid does not fit a device of `cus` CUs.
-// launch_cheby_grid: false when the device does not hold all blocks at once.
 // launch_grid_finish: psi, the observables (nullable) and the status of the
 // run after launch_cheby_grid.
 bool grid_shape(int N0, int N1, int S, int cus, bool gspo, GridShape &g);
 size_t grid_exchange_len(const GridShape &g, int S);
 template <class R>
-bool launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
+void launch_cheby_grid(hipStream_t s, int S, const HamDev<R> &h, const GridShape &g, const GridRun &a,
                        const LinePlan &p0, const LinePlan &p1, const double *coef, int order, double offset,
                        double offset_i, double inv_scaling, double prec, bool imag, const double *psi, ChebyCtl *ctl,
                        double *partials);
 template <class R>
-bool launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
+void launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
                       bool coupled, const LinePlan &p0, const LinePlan &p1, const double *ek, double inv0, double inv1,
                       const double *psi);
 void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
