@@ -661,6 +661,203 @@ __global__ void __launch_bounds__(256) k_gspo_grid(GridRun a, GridShape g, XGrou
     }
 }
 
+// The Lanczos vectors and the tridiagonal matrix of one short iterative Lanczos
+// step on a 2D grid (OSIL::BuildLZB, OSIL.cpp:79-190; real or imaginary time):
+// q_0 = psi, q_{k+1} = (H - alpha_k) q_k - beta_{k-1} q_{k-1}, normalised, until
+// the error estimate ends it.  H q as in k_cheby_grid; the two sums of an
+// iteration go round over the blocks' partial sums.  res: psinorm^2, the
+// number of iterations, alpha[order], beta[order] (norms).  Every vector is
+// stored once, for the combination that follows.  An iteration on 192 x 256
+// points took 84 us with launches and host round trips for each sum, 22 us here.
+template <int S, bool PRIMES>
+__global__ void __launch_bounds__(256) k_sil_grid(GridRun a, GridShape g, HamDev<double> h, LinePlan p0, LinePlan p1,
+                                                  SilVectors qv, int order, double dt, double err_max, double weight,
+                                                  const cx<double> *__restrict__ psi, double *__restrict__ res) {
+    extern __shared__ __align__(16) char smem_raw[];
+    __shared__ double red[4], bc;
+    __shared__ int bad;
+    using C = cx<double>;
+    const int tid = threadIdx.x, wave = tid >> 6, nw = (blockDim.x + 63) >> 6;
+    const GridBlock<double, S> B(g, p0, p1, reinterpret_cast<C *>(smem_raw));
+    const int st = B.rst;
+    const bool on = B.ax[0].on;
+    const int len0 = grid_line_len(g.R2[0], g.R3[0]), len1 = grid_line_len(g.R2[1], g.R3[1]);
+    for (int s = 0; s < S; ++s) {
+        grid_factors(h.tk[s][0], h.inv_nd[0], g.R2[0], g.R3[0], const_cast<double *>(B.f[0]) + s * len0);
+        grid_factors(h.tk[s][1], h.inv_nd[1], g.R2[1], g.R3[1], const_cast<double *>(B.f[1]) + s * len1);
+    }
+    if (tid == 0) bad = 0;
+    const long nx = (long)S * g.nrb * g.rb * g.ncb * g.cw;
+    const GridX<double> XA(a.A, nx), XB(a.B, nx);
+    const double uni = st ? h.unity[S - 1] : h.unity[0];
+    C cur[8], prev[8];
+    double wv[S][8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        cur[q] = on ? psi[(long)st * B.n + B.gi(q)] : mk<double>(0, 0);
+        prev[q] = mk<double>(0, 0);
+#pragma unroll
+        for (int j = 0; j < S; ++j) {
+            double w = j == st ? uni : 0.0;
+            if (on && h.W[st][j]) w += h.W[st][j][B.gi(q)];
+            if (on && h.mu[st][j]) w += h.Edip[st][j] * h.mu[st][j][B.gi(q)];
+            wv[j][q] = w;
+        }
+    }
+    unsigned epoch = a.epoch;
+    // sum over the grid of v, in every thread; false: gave up
+    auto total = [&](double v, int slot, double &out) {
+        const double s = dpp_wave_sum(v);
+        if ((tid & 63) == 0) red[wave] = s;
+        lds_barrier();
+        ++epoch;
+        if (wave == 0) {
+            double t = 0;
+            for (int w = 0; w < nw; ++w) t += red[w];
+            if (B.row) {
+                if (tid < kGridCopies)
+                    __hip_atomic_store(grid_slot(a.sync, tid, slot) + B.b, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                grid_drain();
+                grid_signal(a.sync, epoch);
+            }
+            if (!grid_wait(a.sync, B.nrb, epoch)) {
+                if (tid == 0) bad = 1;
+            } else {
+                const double r = grid_sum(a.sync, slot, B.nrb);
+                if (tid == 0) bc = r;
+            }
+        }
+        lds_barrier();
+        out = bc;
+        return !bad;
+    };
+    auto norm2 = [&](const C(&x)[8]) {
+        double t = 0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) t += x[q].r * x[q].r + x[q].i * x[q].i;
+        return t;
+    };
+    __syncthreads();
+    bool ok = true;
+    double psin = 0, alpha = 0, beta0 = 0, beta1 = 0, beta2 = 0, pdt = 1, prod = 1;
+    ok = total(norm2(cur), 0, psin);
+    const double psinorm = sqrt(psin * weight);
+    // iteration it: H q_{it-1}, alpha_{it-1}, q_it, beta_{it-1}; it = order: only
+    // the last diagonal element
+    int it = 1;
+    for (; ok; ++it) {
+        C x[8], v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            x[q] = cur[q];
+            if (on) XA.st(B.rA[q], cur[q]);
+        }
+        ++epoch;
+#pragma unroll 1
+        for (int ph = 0; ph < 2; ++ph) {
+            if (ph ? B.col : B.row)
+                grid_filter<PRIMES>(x, B.axis(ph), ph ? B.f[1] + B.cst * len1 : B.f[0] + st * len0,
+                                    [&] { if (ph == 0) grid_drain(); },
+                                    [&] { if (ph == 0 && wave == 0) grid_signal(a.sync, epoch); });
+            if (ph) break;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = x[q];
+            if (wave == 0 && !grid_wait(a.sync, B.nrb, epoch) && tid == 0) bad = 1;
+            lds_barrier();
+            if (bad) break;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) x[q] = XA.ld(B.cA[q]);   // 0 for threads without a column
+        }
+        if (bad) break;
+        if (B.ax[1].on) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) XB.st(B.cB[q], x[q]);
+        }
+        grid_drain();
+        lds_barrier();
+        ++epoch;
+        if (wave == 0) {
+            if (B.col) grid_signal(a.sync, epoch);
+            if (B.row && !grid_wait(a.sync, B.ncb, epoch) && tid == 0) bad = 1;
+        }
+        lds_barrier();
+        if (bad) break;
+        double dot = 0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            C hp = v[q] + XB.ld(B.rB[q]);   // 0 for threads without a row
+#pragma unroll
+            for (int j = 0; j < S; ++j) {
+                C pj = cur[q];
+                if constexpr (S == 2) {   // the other state's value sits one lane away
+                    const C o = mk<double>(dpp<kXor1>(cur[q].r), dpp<kXor1>(cur[q].i));
+                    if (j != st) pj = o;
+                }
+                hp.r += wv[j][q] * pj.r;
+                hp.i += wv[j][q] * pj.i;
+            }
+            v[q] = hp;
+            dot += cur[q].r * hp.r + cur[q].i * hp.i;
+        }
+        if (!total(dot, 1, alpha)) break;
+        alpha *= weight;
+        if (B.b == 0 && tid == 0) res[2 + it - 1] = alpha;
+        if (it == order) break;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            C w = mk<double>(v[q].r - alpha * cur[q].r, v[q].i - alpha * cur[q].i);
+            w.r -= beta1 * prev[q].r;
+            w.i -= beta1 * prev[q].i;
+            v[q] = w;
+        }
+        // error estimate dt^(it-2) beta_0 prod beta_i / i over 1 <= i <= it - 3,
+        // before this iteration's norm is known (OSIL.cpp:128-135)
+        double err = 0;
+        if (it >= 2) {
+            if (it > 2) pdt *= dt;
+            if (it > 3) prod *= beta2 / (it - 3);
+            err = fabs(pdt * beta0 * prod);
+        }
+        beta2 = beta1;
+        double b2;
+        if (!total(norm2(v), 0, b2)) break;
+        beta1 = sqrt(b2 * weight);
+        if (it == 1) beta0 = beta1;
+        if (B.b == 0 && tid == 0) res[2 + order + it - 1] = beta1;
+        const double f = 1 / beta1;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            prev[q] = cur[q];
+            cur[q] = mk<double>(v[q].r * f, v[q].i * f);
+            if (on) reinterpret_cast<C *>(qv.q[it])[(long)st * B.n + B.gi(q)] = cur[q];
+        }
+        if (it >= 2 && err < err_max * psinorm) break;
+    }
+    if (bad) {
+        if (tid == 0) *a.status = 1;
+        return;
+    }
+    if (B.b == 0 && tid == 0) {
+        res[0] = psin;
+        res[1] = it;
+    }
+}
+
+// psi <- c_0 psi + sum over 0 < i < n of c_i q_i
+__global__ void __launch_bounds__(256) k_sil_combine(SilVectors qv, SilCoeffs c, int n, long len,
+                                                     cx<double> *__restrict__ psi) {
+    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < len; e += (long)gridDim.x * 256) {
+        cx<double> y = cmul(mk<double>(c.c[0], c.c[1]), psi[e]);
+#pragma unroll 4
+        for (int i = 1; i < n; ++i)
+            y = y + cmul(mk<double>(c.c[2 * i], c.c[2 * i + 1]), reinterpret_cast<const cx<double> *>(qv.q[i])[e]);
+        psi[e] = y;
+    }
+}
+
+// the status of a launch of k_sil_grid to the host
+__global__ void k_grid_report(GridRun a, volatile int *report) { *report = *a.status; }
+
 // After a run: psi from its staging copy and the observables of each step
 // (blocks past ncopy, one per step: 4 S doubles as qdx_prop_run lays them
 // out); nothing when the run gave up.  report: host-visible status.
@@ -848,6 +1045,30 @@ template void launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRu
 template void launch_gspo_grid(hipStream_t, int, const GridShape &, const GridRun &, const XGroupDev<float> &, bool,
                                bool, const LinePlan &, const LinePlan &, const double *, double, double,
                                const double *);
+
+void launch_sil_grid(hipStream_t s, int S, const HamDev<double> &h, const GridShape &g, const GridRun &a,
+                     const LinePlan &p0, const LinePlan &p1, const SilVectors &q, int order, double dt, double err,
+                     double weight, const double *psi, double *res, int *report) {
+    const size_t lds = grid_lds_bytes(g, p0.L, p1.L, S, 16, sizeof(double));
+    auto cp = reinterpret_cast<const cx<double> *>(psi);
+    auto launch = [&](auto kernel) {
+        set_lds(kernel, lds);
+        QDX_LAUNCH(kernel, dim3(g.blocks), dim3(g.threads), lds, s, a, g, h, p0, p1, q, order, dt, err, weight, cp, res);
+        QDX_HIP(hipGetLastError());
+    };
+    if (S == 1 && g.primes) launch(k_sil_grid<1, true>);
+    else if (S == 1) launch(k_sil_grid<1, false>);
+    else if (g.primes) launch(k_sil_grid<2, true>);
+    else launch(k_sil_grid<2, false>);
+    QDX_LAUNCH(k_grid_report, dim3(1), dim3(1), 0, s, a, report);
+    QDX_HIP(hipGetLastError());
+}
+
+void launch_sil_combine(hipStream_t s, const SilVectors &q, const SilCoeffs &c, int n, long len, double *psi) {
+    const int nb = (int)std::min<long>(2048, (len + 255) / 256);
+    QDX_LAUNCH(k_sil_combine, dim3(nb), dim3(256), 0, s, q, c, n, len, reinterpret_cast<cx<double> *>(psi));
+    QDX_HIP(hipGetLastError());
+}
 
 void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
                         int *report) {

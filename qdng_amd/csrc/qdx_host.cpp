@@ -2250,6 +2250,11 @@ static void krylov_create(qdx_ham *h, double dt, int32_t order, double err, int3
         }
         // reduction partials of qdx_prop_run's observables
         p->partials.alloc(kMaxPartials * sizeof(double));
+        p->sil_grid = !arnoldi && order <= kSilMost && grid_fits(p.get());
+        if (p->sil_grid) {
+            grid_buffers(p.get(), 16);
+            HIPCHK(hipDeviceSynchronize());
+        }
         ctx_acquire(p->ctx);
         *out = p.release();
     }
@@ -2303,6 +2308,52 @@ int qdx_prop_destroy(qdx_prop *p) {
 
 namespace {
 
+// The Lanczos basis of a step by the persistent kernel (2D grids): fills the
+// matrix elements, the vectors 1 .. convorder - 1, the number of vectors and
+// of H applications.  False: not available, or the launch gave up (nothing
+// has changed).
+bool sil_grid_basis(qdx_prop *p, qdx_wf *psi, long step, std::vector<double> &alpha, std::vector<double> &beta,
+                    int &convorder, int &napply) {
+    qdx_ctx *ctx = p->ctx;
+    if (!p->sil_grid || ctx->line_ppt != 0) return false;
+    const int order = p->sil_order;
+    hipStream_t s = ctx->stream;
+    p->ham->finalize();
+    HamDev<double> h = p->ham->dev.h64;
+    p->ham->set_fields(h, step);
+    SilVectors qv;
+    for (int i = 0; i < order; ++i) qv.q[i] = p->lzb[i]->ptr();
+    GridRun a = grid_args(p, step, 1, 4u * (unsigned)order + 8, nullptr, nullptr);
+    const size_t nres = 2 + 2 * (size_t)order;
+    std::vector<double> res(nres);
+    {
+        std::lock_guard<std::mutex> alone(grid_mutex(ctx->device));
+        launch_sil_grid(s, p->S, h, p->gs, a, ctx->plan_ppt(p->grid.N[0], false, 4),
+                        ctx->plan_ppt(p->grid.N[1], false, 4), qv, order, p->dt, p->sil_err, psi->grid.weight(),
+                        psi->ptr(), p->partials.as<double>(), p->greport);
+        HIPCHK(hipMemcpyAsync(res.data(), p->partials.p, nres * sizeof(double), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+    }
+    if (*p->greport) {
+        HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, s));
+        p->gepoch = 0;
+        p->sil_grid = false;
+        return false;
+    }
+    const int it = (int)res[1];
+    if (!std::isfinite(res[0])) fail(QDX_ERR_OVERFLOW, "Norm is not a number");
+    for (int i = 0; i < order; ++i) {
+        // (the series ends at iteration it: alpha_0 .. alpha_{it-1}, and
+        // beta_{it-1} when the error estimate ended it)
+        if (i < it) alpha[i] = res[2 + i];
+        if (i < std::min(it, order - 1)) beta[i] = res[2 + order + i];
+        if (!std::isfinite(beta[i])) fail(QDX_ERR_OVERFLOW, "Norm is not a number");
+    }
+    convorder = std::min(it + 1, order);
+    napply = std::min(it + 1, order);
+    return true;
+}
+
 // OSIL::BuildLZB + DiagLZB (OSIL.cpp:79-190) over device operations: the
 // Lanczos vectors live on the device, the tridiagonal matrix is diagonalised
 // on the host.  QDng's own details are kept: q_0 is psi unnormalised, the
@@ -2325,34 +2376,38 @@ void sil_step(qdx_prop *p, qdx_wf *psi, long step) {
     };
     auto scale = [&](qdx_wf *w, double f) { launch_scale_axpy(s, w->ptr(), nullptr, n, f, 0.0, 0.0); };
     std::complex<double> z;
-    const double psinorm = norm_of(psi);
-    chk(qdx_wf_copy(q[0], psi));
-    chk(qdx_ham_apply(H, buf, q[0], step));
-    ++napply;
-    ovl(q[0], buf, z);
-    alpha[0] = z.real();
-    chk(qdx_wf_copy(q[1], buf));
-    chk(qdx_wf_axpy(q[1], -alpha[0], 0.0, q[0]));
-    beta[0] = norm_of(q[1]);
-    scale(q[1], 1 / beta[0]);
-    int convorder = 2, it;
-    for (it = 2; it < order; it++) {
-        double err = std::pow(p->dt, it - 2) * beta[0];
-        for (int i = 1; i < it - 2; i++) err *= beta[i] / double(i);
-        err = std::fabs(err);
-        convorder++;
-        chk(qdx_ham_apply(H, q[it], q[it - 1], step));
+    int convorder = 2;
+    const bool grid = sil_grid_basis(p, psi, step, alpha, beta, convorder, napply);
+    if (!grid) {
+        const double psinorm = norm_of(psi);
+        chk(qdx_wf_copy(q[0], psi));
+        chk(qdx_ham_apply(H, buf, q[0], step));
         ++napply;
-        ovl(q[it - 1], q[it], z);
-        alpha[it - 1] = z.real();
-        chk(qdx_wf_axpy(q[it], -alpha[it - 1], 0.0, q[it - 1]));
-        chk(qdx_wf_axpy(q[it], -beta[it - 2], 0.0, q[it - 2]));
-        beta[it - 1] = norm_of(q[it]);
-        scale(q[it], 1 / beta[it - 1]);
-        if (err < p->sil_err * psinorm) break;
+        ovl(q[0], buf, z);
+        alpha[0] = z.real();
+        chk(qdx_wf_copy(q[1], buf));
+        chk(qdx_wf_axpy(q[1], -alpha[0], 0.0, q[0]));
+        beta[0] = norm_of(q[1]);
+        scale(q[1], 1 / beta[0]);
+        int it;
+        for (it = 2; it < order; it++) {
+            double err = std::pow(p->dt, it - 2) * beta[0];
+            for (int i = 1; i < it - 2; i++) err *= beta[i] / double(i);
+            err = std::fabs(err);
+            convorder++;
+            chk(qdx_ham_apply(H, q[it], q[it - 1], step));
+            ++napply;
+            ovl(q[it - 1], q[it], z);
+            alpha[it - 1] = z.real();
+            chk(qdx_wf_axpy(q[it], -alpha[it - 1], 0.0, q[it - 1]));
+            chk(qdx_wf_axpy(q[it], -beta[it - 2], 0.0, q[it - 2]));
+            beta[it - 1] = norm_of(q[it]);
+            scale(q[it], 1 / beta[it - 1]);
+            if (err < p->sil_err * psinorm) break;
+        }
+        chk(qdx_ham_expec(H, q[it - 1], step, &alpha[it - 1]));
+        ++napply;
     }
-    chk(qdx_ham_expec(H, q[it - 1], step, &alpha[it - 1]));
-    ++napply;
     // Z e^{c Lambda} Z^T e_0, c = -i dt (real time) or -dt (imaginary)
     std::vector<double> T((size_t)order * order, 0.0), ev, Z;
     for (int i = 0; i < order; ++i) {
@@ -2367,6 +2422,18 @@ void sil_step(qdx_prop *p, qdx_wf *psi, long step) {
         for (int i = 0; i < order; ++i) vect[i] += Z[(size_t)i * order + k] * w;
     }
     // psi = vect_0 psi + sum_{i < convorder} vect_i q_i (q_0 holds psi)
+    if (grid) {
+        SilVectors qv;
+        SilCoeffs c;
+        for (int i = 0; i < convorder; ++i) {
+            qv.q[i] = q[i]->ptr();
+            c.c[2 * i] = vect[i].real();
+            c.c[2 * i + 1] = vect[i].imag();
+        }
+        launch_sil_combine(s, qv, c, convorder, n, psi->ptr());
+        p->sil_napply = napply;
+        return;
+    }
     launch_scale_axpy(s, psi->ptr(), q[0]->ptr(), n, 0.0, vect[0].real(), vect[0].imag());
     for (int i = 1; i < convorder; ++i) chk(qdx_wf_axpy(psi, vect[i].real(), vect[i].imag(), q[i]));
     p->sil_napply = napply;

@@ -975,6 +975,7 @@ struct qdx_prop {
     GridShape gs;
     DevBuf gflags, gobs;
     unsigned gepoch = 0;
+    bool sil_grid = false;    // the Lanczos basis by the persistent kernel
     int *greport = nullptr;   // host memory: status of the last launch
     int last_nb = 0, nb_init = 0;   // partial counts of the last Chebyshev step
     // SIL (Lanczos vectors and a buffer as device wave functions; `imag`

@@ -220,6 +220,15 @@ struct GridRun {
     int *orders = nullptr;
 };
 
+// Lanczos vectors and their coefficients as kernel arguments
+constexpr int kSilMost = 32;
+struct SilVectors {
+    double *q[kSilMost] = {};
+};
+struct SilCoeffs {
+    double c[2 * kSilMost] = {};   // (re, im)
+};
+
 // Events attached to the dispatch packet of the next kernel launch (set by the
 // host's profiling timer, consumed and cleared by that launch).
 struct LaunchTiming {
@@ -326,6 +335,10 @@ template <class R>
 void launch_gspo_grid(hipStream_t s, int S, const GridShape &g, const GridRun &a, const XGroupDev<R> &pre, bool mu,
                       bool coupled, const LinePlan &p0, const LinePlan &p1, const double *ek, double inv0, double inv1,
                       const double *psi);
+void launch_sil_grid(hipStream_t s, int S, const HamDev<double> &h, const GridShape &g, const GridRun &a,
+                     const LinePlan &p0, const LinePlan &p1, const SilVectors &q, int order, double dt, double err,
+                     double weight, const double *psi, double *res, int *report);
+void launch_sil_combine(hipStream_t s, const SilVectors &q, const SilCoeffs &c, int n, long len, double *psi);
 void launch_grid_finish(hipStream_t s, int S, long n, const GridShape &g, const GridRun &a, double *psi, double *obs,
                         int *report);
 

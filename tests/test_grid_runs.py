@@ -183,3 +183,22 @@ def test_gspo_steps_and_runs_agree(ctx):
     G.backward(False)
     G.run(w, 2058, 2)
     assert rel(w.download(), ref.download()) < 1e-12
+
+
+@pytest.mark.parametrize("imag", [False, True])
+@pytest.mark.parametrize("N0,N1,S,order", [(8, 8, 1, 20), (40, 24, 2, 20), (16, 768, 1, 5), (192, 256, 1, 20),
+                                           (232, 88, 2, 32), (104, 88, 1, 3), (64, 64, 1, 33)])
+def test_lanczos(N0, N1, S, order, imag):
+    """Converged and truncated series, one more vector than the kernel takes.
+    The Lanczos vectors lose their orthogonality at rounding level over the
+    order, by far less than 1e-10 of the state."""
+    import qdng_amd as Q
+    print("[gpu case] grid lanczos", N0, N1, S, order, imag, flush=True)
+
+    def make(c):
+        p = box(N0, N1, S, laser=not imag)
+        H = p.gpu_ham(c)
+        lo, hi = H.bounds()
+        return p, Q.SIL(H, 2.0 / (hi - lo), order=order, imag=imag)
+    check(both(make, 3, True), 1e-10)
+    check(both(make, 2, False), 1e-10)
