@@ -910,7 +910,7 @@ static size_t grid_lds_bytes(const GridShape &g, int N0, int N1, int S, size_t e
 // m = R2 R3 for a line of 8 m points: the stages' radices (see grid_filter),
 // the pair with the fewest multiply-adds per point and passes; false when
 // there is none
-static bool grid_radices(int m, int &R2, int &R3) {
+bool grid_radices(int m, int &R2, int &R3) {
     auto dft = [](int r) {   // operations of a butterfly, about
         if (r == 1) return 0.0;
         double c = 0;

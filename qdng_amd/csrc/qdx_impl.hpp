@@ -324,6 +324,7 @@ void launch_dense_gspo(hipStream_t s, int S, const XGroupDev<double> &pre, const
 // grid_shape: false when the grid does not fit a device of `cus` CUs.
 // launch_grid_finish: psi, the observables (nullable) and the status of the
 // run after launch_cheby_grid.
+bool grid_radices(int m, int &R2, int &R3);
 bool grid_shape(int N0, int N1, int S, int cus, bool gspo, GridShape &g);
 size_t grid_exchange_len(const GridShape &g, int S);
 template <class R>

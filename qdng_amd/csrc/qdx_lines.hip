@@ -1,6 +1,7 @@
 // gfx950 strided line passes (kinetic parts along dimensions >= 1, GSPO
 // kinetic split operator, forward/inverse transforms) and H applied to a
 // complex128 vector (Operator::Apply).
+#include "qdx_gridfft.hpp"
 #include "qdx_kernels_common.hpp"
 
 namespace qdx {
@@ -319,6 +320,98 @@ void Launch<R>::col_pass(hipStream_t s, const GridDev &g, int S, int dim, int mo
     QDX_HIP(hipGetLastError());
 }
 
+// Mode 4 of k_col by the in-place line filter (qdx_gridfft.hpp): half the LDS
+// and half the exchanges of the two Stockham transforms, so that more blocks
+// share a CU.  128^3 points: FP64 (67 MB) 32.7 -> 24.0 us, compact terms (42
+// MB) 20.5 -> 17.6.  Mode 5 stays with k_col: its larger stride and third
+// stream bound it elsewhere (36.5 against 37.6 us here, compact 24.6 against
+// 28.6).
+template <class R, bool CMP>
+__global__ void __launch_bounds__(256, 3) k_kin_filter(GridDev g, int S, int dim, int W, LinePlan p, int R2, int R3,
+                                                       HamDev<R> h, cx<R> *__restrict__ Y,
+                                                       const cx<R> *__restrict__ src, ChebyCtl *ctl, ConvCheck cc) {
+    if (ctl && ctl->done) return;
+    extern __shared__ __align__(16) char smem_raw[];
+    __shared__ double bc;
+    const int N0 = g.N[0], L = g.N[dim], len = grid_line_len(R2, R3);
+    const long estride = dim_stride(g, dim);
+    const int nother = col_nother(g, dim), tiles0 = (N0 + W - 1) / W;
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int rest = b / tiles0, oth = rest % nother, st = rest / nother;
+    GridAxis<R> A;
+    A.m = L / 8;
+    A.R2 = R2;
+    A.R3 = R3;
+    A.RS = grid_rs(R3);
+    A.nl = W;
+    A.lt = threadIdx.x / W;
+    A.a = A.lt / R3;
+    A.b = A.lt - A.a * R3;
+    const int c = threadIdx.x - A.lt * W, c0 = (b % tiles0) * W + c;
+    A.on = A.lt < A.m && c0 < N0;
+    int kk[kMaxDims] = {0, 0, 0, 0};
+    const long boff = (long)st * g.size + col_other(g, dim, oth, kk) + c0;   // element of this thread's column
+    const long nT = (long)S * g.size;
+    cx<R> *smem = reinterpret_cast<cx<R> *>(smem_raw), *tw = smem + W * len;
+    double *f = reinterpret_cast<double *>(tw + grid_tw_len(A.m));
+    A.buf = smem + c;
+    A.tw1 = tw;
+    A.tw2 = tw + 7 * A.m;
+    cx<R> v[8];
+    if (A.on) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = tld<CMP>(src, boff + (long)(A.lt + q * A.m) * estride, nT);
+    }
+    grid_tables(reinterpret_cast<const cx<R> *>(p.tw), A.m, R3, tw, tw + 7 * A.m);
+    grid_factors(h.tk[st][0] ? h.tk[st][dim] : nullptr, h.inv_nd[dim], R2, R3, f);
+    {
+        double a;
+        if (prev_converged(cc, &bc, &a)) {   // as k_col
+            if (ctl && b == 0 && threadIdx.x == 0) {
+                ctl->done = 1;
+                ctl->accnorm = a;
+            }
+            return;
+        }
+    }
+    __syncthreads();
+    grid_filter<false>(v, A, f, [] {}, [] {});
+    if (!A.on) return;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) tst<CMP>(Y, boff + (long)(A.lt + q * A.m) * estride, nT, v[q]);
+}
+
+// false: the line or the grid does not suit k_kin_filter (lines of 8 m points
+// with small prime factors; at least four adjacent columns per block)
+template <class R>
+static bool kin_filter(hipStream_t s, const GridDev &g, int S, int dim, const LinePlan &p,
+                       const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp) {
+    const int L = g.N[dim], m = L / 8;
+    int R2, R3;
+    if (L % 8 || !grid_radices(m, R2, R3) || R2 == 11 || R2 == 13 || R2 > 16 || R3 == 11 || R3 == 13) return false;
+    int W = 256 / m;
+    if (W > 16) W = 16;
+    if (W > g.N[0]) W = g.N[0];
+    if (W < 4) return false;
+    const int nb = ((g.N[0] + W - 1) / W) * col_nother(g, dim) * S;
+    const int threads = std::max(64, round64(W * m));
+    const size_t lds = ((size_t)W * grid_line_len(R2, R3) + grid_tw_len(m)) * sizeof(cx<R>) +
+                       grid_line_len(R2, R3) * sizeof(double);
+    auto launch = [&](auto kernel) {
+        set_lds(kernel, lds);
+        QDX_LAUNCH(kernel, dim3(nb), dim3(threads), lds, s, g, S, dim, W, p, R2, R3, h, reinterpret_cast<cx<R> *>(Y),
+                   reinterpret_cast<const cx<R> *>(src), ctl, cc);
+        QDX_HIP(hipGetLastError());
+    };
+    if (cmp) {
+        if constexpr (std::is_same<R, double>::value) launch(k_kin_filter<R, true>);
+        else throw std::runtime_error("compact terms: FP64 only");
+    } else {
+        launch(k_kin_filter<R, false>);
+    }
+    return true;
+}
+
 template <class R, int P>
 static void kin_pass_P(hipStream_t s, const GridDev &g, int S, int dim, bool accumulate, const LinePlan &plan,
                        const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp) {
@@ -359,6 +452,7 @@ static void kin_pass_P(hipStream_t s, const GridDev &g, int S, int dim, bool acc
 template <class R>
 void Launch<R>::kin_pass(hipStream_t s, const GridDev &g, int S, int dim, bool accumulate, const LinePlan &plan,
                          const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp) {
+    if (!accumulate && kin_filter<R>(s, g, S, dim, plan, h, src, Y, ctl, cc, cmp)) return;
     if (plan.ppt == 4) kin_pass_P<R, 4>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
     else kin_pass_P<R, 8>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
 }
