@@ -52,21 +52,6 @@ B_GSPO = {"fp64": 32 + 8, "fp32": 16 + 4}
 PRECISIONS = ("fp64", "compact", "fp32")
 
 
-TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "cheby_row_2d_512x512_2state_fp64_hbm_traffic.md")
-
-
-def measured_traffic():
-    """HBM bytes per row-kernel launch from the committed FETCH_SIZE /
-    WRITE_SIZE profile of this workload (None if it is absent)."""
-    try:
-        for line in open(TRAFFIC_PROFILE):
-            if line.startswith("traffic_bytes_per_launch:"):
-                return float(line.split(":")[1])
-    except OSError:
-        pass
-    return None
-
-
 def log(msg):
     print("[bench] " + msg, file=sys.stderr, flush=True)
 
@@ -517,7 +502,7 @@ def precision_3d(ctx, steps=5):
             ach = rb / (msrow * 1e-3) / 1e9 if msrow > 0 else 0.0
             rec[prec] = {"value": npts * hpsi / t, "unit": UNIT, "ms_per_step": t * 1e3 / steps,
                          "hpsi_per_step": [int(nh.min()), int(nh.max())], "order": U.order,
-                         "roofline": {"bound": "hbm", "kernel": "k_cheby_row", "achieved": ach,
+                         "roofline": {"bound": "hbm", "kernel": "k_cheby_grid", "achieved": ach,
                                       "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                                       "avg_launch_us": msrow / max(nrow, 1) * 1e3}}
             if prec == "fp64":
@@ -679,26 +664,21 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
-            "traffic": measured_traffic(),
-            "traffic_source": "profiles/cheby_row_2d_512x512_2state_fp64_hbm_traffic.md (rocprofv3 FETCH_SIZE x 2.000 "
-                              "+ WRITE_SIZE x 1.000, calibrated on a 256 MiB device copy)",
-            "kernel": "qdx::k_cheby_row<double, 2, false, false, 256, 4, false, false>",
-            "points_per_thread": 4,
+            "traffic": None,
+            "traffic_note": "the kernel keeps psi, the terms and the surfaces in registers: what it moves is the "
+                            "exchange of phi and of the filtered lines, 64 B per point and state and order",
+            "kernel": "qdx::k_cheby_grid<double, 2, false, false, false>",
+            "points_per_thread": 8,
             "launches": launches,
             "avg_launch_us": row_ms / launches * 1e3,
             "algorithmic_bytes_per_launch": row_bytes / launches,
-            "bytes_model": "96 B per grid point and state per executed order (80 B for order 1); "
-                           "early-exit launches after the break count 0 B",
-            "measured": "HIP events attached to every launch (hipExtLaunchKernelGGL) over a second "
-                        "timed pass of the same steps",
+            "bytes_model": "96 B per grid point and state per executed order (80 B for order 1), the operands of "
+                           "an order that is a kernel of its own",
+            "measured": "HIP events attached to every launch (hipExtLaunchKernelGGL; one launch runs many steps) "
+                        "over a second timed pass of the same steps",
             "ms_per_step_profiled_pass": rp["seconds"] * 1e3 / args.steps,
             "step_frac": B_ROW["fp64"] * value / 1e9 / HBM_PEAK_GBS,
-            "step_frac_note": "the whole step (row kernel, column pass, launch gaps) at the same 96 B per grid "
-                              "point and state per executed order",
-            "column_pass": {"kernel": "qdx::k_col<double, 4, 4, false>", "launches": rp["line"][0],
-                            "avg_launch_us": rp["line"][1] / max(rp["line"][0], 1) * 1e3,
-                            "algorithmic_bytes_per_launch": 32.0 * p.size * p.S,
-                            "note": "phi_{k-1} read + Y written, 16 B each per point and state"},
+            "step_frac_note": "the whole step at the same 96 B per grid point and state per executed order",
         },
     }
 
@@ -753,11 +733,10 @@ def main():
                 "value": v, "unit": UNIT, "ms_per_step": rr["seconds"] * 1e3 / args.steps,
                 "hpsi_per_step": [int(rr["n_hpsi"].min()), int(rr["n_hpsi"].max())], "vs_fp64": v / value,
                 "l2_vs_oracle": ex.get("parity", {}).get(prec, {}).get("l2_vs_oracle"),
-                "roofline": {"bound": "hbm", "kernel": "k_cheby_row", "achieved": bb / (lms * 1e-3) / 1e9,
+                "roofline": {"bound": "hbm", "kernel": "k_cheby_grid", "achieved": bb / (lms * 1e-3) / 1e9,
                              "peak": HBM_PEAK_GBS, "unit": "GB/s",
                              "frac": bb / (lms * 1e-3) / 1e9 / HBM_PEAK_GBS, "avg_launch_us": lms / ln * 1e3,
-                             "bytes_model": f"{B_ROW[prec]} B per grid point and state per executed order"},
-                "col_kernel_avg_launch_us": rq["line"][1] / max(rq["line"][0], 1) * 1e3}
+                             "bytes_model": f"{B_ROW[prec]} B per grid point and state per executed order"}}
             log(f"{prec}: {v:.4g} grid-pt*Hpsi/s")
         configs["cheby_2d_512x512_2state"] = rec2d
         # GSPO on the same workload: at least 100 timed steps
@@ -770,11 +749,10 @@ def main():
             eff = B_GSPO[prec] * v / 1e9
             gs["precisions"][prec] = {
                 "value": v, "unit": "grid-pt*step/s", "ms_per_step": t * 1e3 / gsteps, "steps": gsteps,
-                "roofline": {"bound": "hbm", "kernel": "whole step (row pass + column pass)", "achieved": eff,
+                "roofline": {"bound": "hbm", "kernel": "k_gspo_grid (whole runs)", "achieved": eff,
                              "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": eff / HBM_PEAK_GBS,
                              "bytes_model": f"{B_GSPO[prec]} B per grid point and state per step"},
-                "row_kernel_avg_launch_us": rowk[1] / max(rowk[0], 1) * 1e3, "row_launches": rowk[0],
-                "col_kernel_avg_launch_us": colk[1] / max(colk[0], 1) * 1e3, "col_launches": colk[0]}
+                "kernel_us_per_step": (rowk[1] + colk[1]) / gsteps * 1e3, "launches": rowk[0] + colk[0]}
             log(f"gspo {prec}: {v:.4g} grid-pt*step/s, {t * 1e3 / gsteps:.4f} ms/step")
         gs["value"] = gs["precisions"]["fp64"]["value"]
         gs["roofline"] = gs["precisions"]["fp64"]["roofline"]

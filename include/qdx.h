@@ -475,7 +475,11 @@ int qdx_ctx_get_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, int32_t *
  * radix are 4 or 2, else first and last radix 4.  Both give the same
  * transform up to rounding.  Single-state 1D lines run a whole step in one
  * block, with 4 points per thread up to 1024 points and 8 above, unless 8
- * is set.  No
+ * is set.  With 0, short 1D lines (Chebyshev up to 512 points, 256 for two
+ * states; split operator up to 384) and 2D grids of up to 2^19 points and
+ * states (Chebyshev, split operator, short iterative Lanczos; one or two
+ * states) run whole propagations in one kernel instead; 4 or 8 selects the
+ * kernels above for them too.  No
  * QDng counterpart: FFTW lays out its own threads (src/fft/fft.cpp:95-110). */
 int qdx_ctx_set_line_points(qdx_ctx *ctx, int32_t points);
 int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points);
