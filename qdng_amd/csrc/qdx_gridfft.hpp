@@ -1,5 +1,6 @@
-// Line filters of the persistent grid kernels (included by qdx_grid.hip):
-// IFFT . diag(f) . FFT of lines of N = 8 m points, 8 points per thread.
+// Line filters of the persistent grid kernels and of the kinetic pass of larger
+// grids: IFFT . diag(f) . FFT of lines of N = 8 m points, 8 points per thread.
+// Also the DPP and barrier helpers that the dense 1D kernels share.
 //
 // With n = n1 m + n2 and k = k1 + 8 k2 the transform is a radix-8 stage over
 // n1 on registers (thread lt owns the points lt + q m), a twiddle, and for
