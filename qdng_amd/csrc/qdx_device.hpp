@@ -355,7 +355,11 @@ __host__ __device__ constexpr int tw_lds_len(int L) { return L + (L >> 3); }
 // tw: the table exp(-2 pi i q / L), q in [0, L): the padded LDS copy made by
 // stage_twiddles (tsh = kTwLds; the barrier at the start of fft_line
 // publishes it) or the table in memory (tsh = kTwMem).
-template <class R, int P, bool IP = false>
+// GEN: the plan may hold odd primes above 3.  The batched kernels take lengths
+// 2^a 3^b only and leave that stage out: its code alone slows the others (a
+// mixed batch of 64 FP32 jobs, 40 ticks: 24.4 ms on the device with it, 24.2
+// without).
+template <class R, int P, bool IP = false, bool GEN = true>
 __device__ __forceinline__ void fft_line(cx<R> (&v)[P], const LdsLine<R> &ln, const LinePlan &p, const cx<R> *tw,
                                          int sign, int lt, bool active, int tsh) {
     static_assert(P == 8 || P == 4, "8 or 4 points per thread");
@@ -427,8 +431,10 @@ __device__ __forceinline__ void fft_line(cx<R> (&v)[P], const LdsLine<R> &ln, co
             case 8: mid_stage<8, R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh); break;
             case 4: mid_stage<4, R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh); break;
             case 2: mid_stage<2, R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh); break;
-            case 3: mid_stage<3, R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh); break;
-            default: mid_stage_gen<R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh, r); break;
+            default:
+                if (!GEN || r == 3) mid_stage<3, R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh);
+                else if constexpr (GEN) mid_stage_gen<R, P>(in, out, ln, L, Ns, TL, lv, sign, tw, tsh, r);
+                break;
             }
         }
         __syncthreads();
@@ -483,11 +489,12 @@ __device__ __forceinline__ void fft_line(cx<R> (&v)[P], const LdsLine<R> &ln, co
     }
 }
 
-// the 8-points-per-thread transform of the batched kernels
+// the 8-points-per-thread transform of the batched kernels (lengths 2^a 3^b
+// only: the batch refuses other jobs)
 template <class R, bool IP = false>
 __device__ __forceinline__ void fft8(cx<R> (&v)[8], const LdsLine<R> &ln, const LinePlan &p, const cx<R> *tw,
                                      int sign, int lt, bool active, int tsh) {
-    fft_line<R, 8, IP>(v, ln, p, tw, sign, lt, active, tsh);
+    fft_line<R, 8, IP, false>(v, ln, p, tw, sign, lt, active, tsh);
 }
 
 // ---------------------------------------------------------------------------
