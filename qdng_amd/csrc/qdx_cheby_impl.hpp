@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(512) k_cheby_init(GridDev g, LinePlan p0, int 
 // -i Wi(x) and the offset its imaginary part (b = (H - offset) phi / R with
 // complex offset, OCheby.cpp:104-105, 168).
 template <class R, int S, bool ONE_D, bool PRO, int NT, int P = 8, bool IMAG = false, bool CMP = false,
-          bool NIP = false>
+          bool NIP = false, bool GEN = true>
 __global__ void __launch_bounds__(NT) k_cheby_row(GridDev g, HamDev<R> h, LinePlan p0, ChebyOrder ord,
                                                     ConvCheck cc, int rb, const cx<R> *__restrict__ phim1,
                                                     cx<R> *__restrict__ phim2, cx<R> *__restrict__ X,
@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(NT) k_cheby_row(GridDev g, HamDev<R> h, LinePl
     if (ctl->done) return;
     extern __shared__ __align__(16) char smem_raw[];
     __shared__ double red[16];
-    RowBlock<R, P> B(g, rb, S, reinterpret_cast<cx<R> *>(smem_raw), p0);
+    RowBlock<R, P, GEN> B(g, rb, S, reinterpret_cast<cx<R> *>(smem_raw), p0);
     const int st = B.st;
     const long base = (long)st * g.size;
     const long nT = (long)S * g.size;   // elements of each term buffer
@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(NT) k_cheby_row(GridDev g, HamDev<R> h, LinePl
 // multi-kernel layout) and the break are recorded after the loop; the step
 // start's sum goes to slot 2 * kMaxPartials.  A block of one wave reduces
 // with shuffles alone.
-template <class R, int NT, bool NIP = false, int P = 8>
+template <class R, int NT, bool NIP = false, int P = 8, bool GEN = true>
 __global__ void __launch_bounds__(NT) k_cheby_line(GridDev g, HamDev<R> h, LinePlan p0, const double *coef,
                                                    int order, double offset, double offset_i, double inv_scaling,
                                                    double prec, cx<double> *__restrict__ psi, ChebyCtl *ctl,
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(NT) k_cheby_line(GridDev g, HamDev<R> h, LineP
     extern __shared__ __align__(16) char smem_raw[];
     __shared__ double red[16];
     __shared__ double bc;
-    RowBlock<R, P> B(g, 1, 1, reinterpret_cast<cx<R> *>(smem_raw), p0);
+    RowBlock<R, P, GEN> B(g, 1, 1, reinterpret_cast<cx<R> *>(smem_raw), p0);
     double *cs = reinterpret_cast<double *>(B.after);   // 2 * order coefficients
     const bool one_wave = blockDim.x <= 64;
     const double *tk0 = h.tk[0][0];
@@ -420,7 +420,9 @@ int Launch<R>::cheby_init(hipStream_t s, const GridDev &g, int S, const LinePlan
     return nb;
 }
 
-template <class R, int S, bool ONE_D, bool PRO, int P>
+// GEN: as fft_line; the first order, imaginary time and the negative imaginary
+// potential have those instances only
+template <class R, int S, bool ONE_D, bool PRO, int P, bool GEN>
 static int cheby_row_SKP(hipStream_t st, const GridDev &g, const HamDev<R> &h, const LinePlan &plan,
                          const ChebyOrder &ord, const ConvCheck &cc, bool imag, const R *phim1, R *phim2, R *X, double *psi,
                          ChebyCtl *ctl, double *partials, const double *init_part, int nb_init, bool cmp) {
@@ -458,12 +460,12 @@ static int cheby_row_SKP(hipStream_t st, const GridDev &g, const HamDev<R> &h, c
         if constexpr (std::is_same<R, double>::value && !ONE_D && S <= 2) {
             if (imag) throw std::runtime_error("compact terms: real time only");
             if (r.threads <= 256) {
-                set_lds(k_cheby_row<R, S, ONE_D, PRO, 256, P, false, true>, r.lds);
-                QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 256, P, false, true>), dim3(r.nb), dim3(r.threads), r.lds,
+                set_lds(k_cheby_row<R, S, ONE_D, PRO, 256, P, false, true, false, GEN>, r.lds);
+                QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 256, P, false, true, false, GEN>), dim3(r.nb), dim3(r.threads), r.lds,
                            st, g, h, p0, ord, cc, r.rb, cphim1, cphim2, cX, cpsi, ctl, partials, init_part, nb_init);
             } else {
-                set_lds(k_cheby_row<R, S, ONE_D, PRO, 512, P, false, true>, r.lds);
-                QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 512, P, false, true>), dim3(r.nb), dim3(r.threads), r.lds,
+                set_lds(k_cheby_row<R, S, ONE_D, PRO, 512, P, false, true, false, GEN>, r.lds);
+                QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 512, P, false, true, false, GEN>), dim3(r.nb), dim3(r.threads), r.lds,
                            st, g, h, p0, ord, cc, r.rb, cphim1, cphim2, cX, cpsi, ctl, partials, init_part, nb_init);
             }
         } else {
@@ -478,12 +480,12 @@ static int cheby_row_SKP(hipStream_t st, const GridDev &g, const HamDev<R> &h, c
             throw std::runtime_error("imaginary time: FP64 only");
         }
     } else if (r.threads <= 256) {
-        set_lds(k_cheby_row<R, S, ONE_D, PRO, 256, P>, r.lds);
-        QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 256, P>), dim3(r.nb), dim3(r.threads), r.lds, st, g, h, p0, ord,
+        set_lds(k_cheby_row<R, S, ONE_D, PRO, 256, P, false, false, false, GEN>, r.lds);
+        QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 256, P, false, false, false, GEN>), dim3(r.nb), dim3(r.threads), r.lds, st, g, h, p0, ord,
                    cc, r.rb, cphim1, cphim2, cX, cpsi, ctl, partials, init_part, nb_init);
     } else {
-        set_lds(k_cheby_row<R, S, ONE_D, PRO, 512, P>, r.lds);
-        QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 512, P>), dim3(r.nb), dim3(r.threads), r.lds, st, g, h, p0, ord,
+        set_lds(k_cheby_row<R, S, ONE_D, PRO, 512, P, false, false, false, GEN>, r.lds);
+        QDX_LAUNCH((k_cheby_row<R, S, ONE_D, PRO, 512, P, false, false, false, GEN>), dim3(r.nb), dim3(r.threads), r.lds, st, g, h, p0, ord,
                    cc, r.rb, cphim1, cphim2, cX, cpsi, ctl, partials, init_part, nb_init);
     }
     QDX_HIP(hipGetLastError());
@@ -496,14 +498,16 @@ template <class R, int S, bool ONE_D, bool PRO>
 static int cheby_row_SK(hipStream_t st, const GridDev &g, const HamDev<R> &h, const LinePlan &plan,
                         const ChebyOrder &ord, const ConvCheck &cc, bool imag, const R *phim1, R *phim2, R *X, double *psi,
                         ChebyCtl *ctl, double *partials, const double *init_part, int nb_init, bool cmp) {
+    const bool gen = PRO || plan.odd_prime();
+    auto run = [&](auto launch) {
+        return launch(st, g, h, plan, ord, cc, imag, phim1, phim2, X, psi, ctl, partials, init_part, nb_init, cmp);
+    };
     if (plan.ppt == 4) {
         if constexpr (!ONE_D)
-            return cheby_row_SKP<R, S, ONE_D, PRO, 4>(st, g, h, plan, ord, cc, imag, phim1, phim2, X, psi, ctl, partials,
-                                                      init_part, nb_init, cmp);
+            return gen ? run(cheby_row_SKP<R, S, ONE_D, PRO, 4, true>) : run(cheby_row_SKP<R, S, ONE_D, PRO, 4, PRO>);
         throw std::runtime_error("4 points per thread: grids with nd >= 2 only");
     }
-    return cheby_row_SKP<R, S, ONE_D, PRO, 8>(st, g, h, plan, ord, cc, imag, phim1, phim2, X, psi, ctl, partials, init_part,
-                                              nb_init, cmp);
+    return gen ? run(cheby_row_SKP<R, S, ONE_D, PRO, 8, true>) : run(cheby_row_SKP<R, S, ONE_D, PRO, 8, PRO>);
 }
 
 template <class R, int S>
@@ -550,11 +554,16 @@ void Launch<R>::cheby_line(hipStream_t s, const GridDev &g, const HamDev<R> &h, 
     auto cpsi = reinterpret_cast<cx<double> *>(psi);
     const bool nip = offset_i != 0 || h.Wi[0] != nullptr;   // negative imaginary potential
     const double oi = nip ? offset_i : 0.0;
-#define QDX_LINE(NT_, NIP_, P_)                                                                              \
-    do {                                                                                                     \
-        set_lds(k_cheby_line<R, NT_, NIP_, P_>, lds);                                                        \
-        QDX_LAUNCH((k_cheby_line<R, NT_, NIP_, P_>), dim3(1), dim3(threads), lds, s, g, h, p, coef, order,   \
-                   offset, oi, inv_scaling, prec, cpsi, ctl, partials);                                      \
+    auto launch = [&](auto kernel) {
+        set_lds(kernel, lds);
+        QDX_LAUNCH(kernel, dim3(1), dim3(threads), lds, s, g, h, p, coef, order, offset, oi, inv_scaling, prec, cpsi,
+                   ctl, partials);
+    };
+    const bool gen = p.odd_prime();
+#define QDX_LINE(NT_, NIP_, P_)                                       \
+    do {                                                              \
+        if (NIP_ || gen) launch(k_cheby_line<R, NT_, NIP_, P_>);      \
+        else launch(k_cheby_line<R, NT_, NIP_, P_, NIP_>);            \
     } while (0)
     if (P == 4) {   // short lines: 4 points per thread, at most one 256-thread block
         if (threads > 256) throw std::runtime_error("whole-step line kernel: 4 points per thread up to 1024 points");

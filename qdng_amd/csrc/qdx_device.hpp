@@ -355,10 +355,13 @@ __host__ __device__ constexpr int tw_lds_len(int L) { return L + (L >> 3); }
 // tw: the table exp(-2 pi i q / L), q in [0, L): the padded LDS copy made by
 // stage_twiddles (tsh = kTwLds; the barrier at the start of fft_line
 // publishes it) or the table in memory (tsh = kTwMem).
-// GEN: the plan may hold odd primes above 3.  The batched kernels take lengths
-// 2^a 3^b only and leave that stage out: its code alone slows the others (a
-// mixed batch of 64 FP32 jobs, 40 ticks: 24.4 ms on the device with it, 24.2
-// without).
+// GEN: the plan may hold odd primes above 3.  The code of that stage alone slows
+// the other lengths, so the kernels of the main path have instances without it
+// (LinePlan::odd_prime chooses) and the batched kernels, which take lengths 2^a
+// 3^b only, leave it out.  With it and without: a mixed batch of 64 FP32 jobs, 40
+// ticks, 24.4 and 24.2 ms on the device; a Chebyshev step of 768 x 768 points and
+// two states 4.09 and 3.96 ms; split-operator steps on 128^3 points 133 and 129
+// us, on 1024 x 1024 points 81 and 77 us.
 template <class R, int P, bool IP = false, bool GEN = true>
 __device__ __forceinline__ void fft_line(cx<R> (&v)[P], const LdsLine<R> &ln, const LinePlan &p, const cx<R> *tw,
                                          int sign, int lt, bool active, int tsh) {

@@ -17,15 +17,15 @@ namespace qdx {
 // opart[2 (s nb + b)] = sum |psi|^2 and, after 2 S nb entries, the
 // (re, im) of sum conj(psi) psi0 (Reporter observables, Reporter.cpp:101-137).
 // The x-space operators act on all states of a point at once, so the S lines
-// of a row are exchanged through LDS around them.
-template <class R, int S, bool ONE_D, int PHASE, bool IMAG = false, int P = 8>
+// of a row are exchanged through LDS around them.  GEN: as fft_line.
+template <class R, int S, bool ONE_D, int PHASE, bool IMAG = false, int P = 8, bool GEN = true>
 __global__ void __launch_bounds__(512) k_gspo_row(GridDev g, HamDev<R> kin, double tau, LinePlan p0, int rb,
                                                    XGroupDev<R> pre, XGroupDev<R> post, cx<R> *__restrict__ psi,
                                                    cx<R> *__restrict__ X, const cx<R> *__restrict__ psi0,
                                                    double *__restrict__ opart) {
     extern __shared__ __align__(16) char smem_raw[];
     cx<R> *smem = reinterpret_cast<cx<R> *>(smem_raw);
-    RowBlock<R, P> B(g, rb, S, smem, p0);
+    RowBlock<R, P, GEN> B(g, rb, S, smem, p0);
     const int st = B.st;
     const long base = (long)st * g.size;
     cx<R> v[P];
@@ -261,7 +261,7 @@ void Launch<R>::gspo_unitary(hipStream_t s, const GridDev &g, int S, const XSpli
 }
 
 // returns the number of row blocks launched
-template <class R, bool ONE_D, int PHASE, bool IMAG, int P>
+template <class R, bool ONE_D, int PHASE, bool IMAG, int P, bool GEN>
 static int gspo_row_launch_IP(hipStream_t s, const GridDev &g, int S, const HamDev<R> &kin, double tau,
                               const LinePlan &plan, const XGroupDev<R> &pre, const XGroupDev<R> &post, R *psi,
                               R *X, const R *psi0, double *opart) {
@@ -271,8 +271,8 @@ static int gspo_row_launch_IP(hipStream_t s, const GridDev &g, int S, const HamD
         RowLaunch r = row_launch<R>(g, SS, p0, SS > 1);
         if (opart && (long)4 * SS * r.nb > kMaxPartials)
             throw std::runtime_error("grid too large for the observables' partial sums");
-        set_lds(k_gspo_row<R, SS, ONE_D, PHASE, IMAG, P>, r.lds);
-        QDX_LAUNCH((k_gspo_row<R, SS, ONE_D, PHASE, IMAG, P>), dim3(r.nb), dim3(r.threads), r.lds, s, g, kin, tau,
+        set_lds(k_gspo_row<R, SS, ONE_D, PHASE, IMAG, P, GEN>, r.lds);
+        QDX_LAUNCH((k_gspo_row<R, SS, ONE_D, PHASE, IMAG, P, GEN>), dim3(r.nb), dim3(r.threads), r.lds, s, g, kin, tau,
                    p0, r.rb, pre, post, reinterpret_cast<cx<R> *>(psi), reinterpret_cast<cx<R> *>(X),
                    reinterpret_cast<const cx<R> *>(psi0), opart);
         nb = r.nb;
@@ -281,18 +281,22 @@ static int gspo_row_launch_IP(hipStream_t s, const GridDev &g, int S, const HamD
     return nb;
 }
 
-// 4 points per thread on grids with nd >= 2 when the plan asks for it
+// 4 points per thread on grids with nd >= 2 when the plan asks for it;
+// imaginary time has the GEN instances only
 template <class R, bool ONE_D, int PHASE, bool IMAG>
 static int gspo_row_launch_I(hipStream_t s, const GridDev &g, int S, const HamDev<R> &kin, double tau,
                              const LinePlan &plan, const XGroupDev<R> &pre, const XGroupDev<R> &post, R *psi,
                              R *X, const R *psi0, double *opart) {
+    const bool gen = IMAG || plan.odd_prime();
+    auto run = [&](auto launch) { return launch(s, g, S, kin, tau, plan, pre, post, psi, X, psi0, opart); };
     if constexpr (!ONE_D) {
         if (plan.ppt == 4)
-            return gspo_row_launch_IP<R, ONE_D, PHASE, IMAG, 4>(s, g, S, kin, tau, plan, pre, post, psi, X, psi0,
-                                                                 opart);
+            return gen ? run(gspo_row_launch_IP<R, ONE_D, PHASE, IMAG, 4, true>)
+                       : run(gspo_row_launch_IP<R, ONE_D, PHASE, IMAG, 4, IMAG>);
     }
     if (plan.ppt != 8) throw std::runtime_error("GSPO rows: 8 or 4 points per thread (4 for nd >= 2)");
-    return gspo_row_launch_IP<R, ONE_D, PHASE, IMAG, 8>(s, g, S, kin, tau, plan, pre, post, psi, X, psi0, opart);
+    return gen ? run(gspo_row_launch_IP<R, ONE_D, PHASE, IMAG, 8, true>)
+               : run(gspo_row_launch_IP<R, ONE_D, PHASE, IMAG, 8, IMAG>);
 }
 
 // imag: imaginary time (FP64 only)

@@ -27,6 +27,12 @@ struct LinePlan {
     int tw_lds = 1;    // kernels stage the table in LDS (set by the launcher)
     int ppt = 8;       // points per thread of the line kernels (8, or 4: first
                        // and last radix 4 or 2)
+    // a stage of an odd prime above 3 (the kernels' GEN instances)
+    bool odd_prime() const {
+        for (int i = 0; i < nst; ++i)
+            if (rad[i] > 3 && rad[i] % 2) return true;
+        return false;
+    }
 };
 
 // Grid as the kernels see it: N[d] points in dimension d, dimension 0

@@ -35,7 +35,8 @@ __device__ __forceinline__ double kin_sum(const HamDev<R> &h, int st, const Grid
 
 // Row-block geometry: rb rows of dimension 0 for each of S states; line
 // l = st * rb + rr; P points per thread.  Two padded LDS buffers per line.
-template <class R, int P = 8>
+// GEN: as fft_line.
+template <class R, int P = 8, bool GEN = true>
 struct RowBlock {
     int L, TL, rb, nl, line, lt, st, rr;
     long nrows, row;
@@ -76,8 +77,8 @@ struct RowBlock {
     }
     // transform with the LDS or the global twiddle table; both calls inline
     __device__ void fft(cx<R> (&v)[P], const LinePlan &p, int sign) {
-        if (twl) fft_line<R, P>(v, ln, p, tw, sign, lt, active, kTwLds);
-        else fft_line<R, P>(v, ln, p, reinterpret_cast<const cx<R> *>(p.tw), sign, lt, active, kTwMem);
+        if (twl) fft_line<R, P, false, GEN>(v, ln, p, tw, sign, lt, active, kTwLds);
+        else fft_line<R, P, false, GEN>(v, ln, p, reinterpret_cast<const cx<R> *>(p.tw), sign, lt, active, kTwMem);
     }
     __device__ long gidx(int q) const { return row * L + lt + q * TL; }
 };

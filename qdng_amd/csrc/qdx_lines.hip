@@ -16,7 +16,8 @@ namespace qdx {
 //      4: X = IFFT(T_dim/N_dim FFT(src)), the dimension's part of the
 //         separable kinetic operator, 5: X += the same.
 // CMP (modes 4 and 5): src and X in the compact 40-bit term storage.
-template <class R, int MODE, int P = 8, bool IMAG = false, bool CMP = false>
+// GEN: as fft_line.
+template <class R, int MODE, int P = 8, bool IMAG = false, bool CMP = false, bool GEN = true>
 __global__ void __launch_bounds__(512) k_col(GridDev g, int S, int dim, int W, LinePlan p, HamDev<R> h, double tau,
                                               cx<R> *__restrict__ X, const cx<R> *__restrict__ src,
                                               ChebyCtl *ctl, ConvCheck cc, const double *__restrict__ ek) {
@@ -50,8 +51,8 @@ __global__ void __launch_bounds__(512) k_col(GridDev g, int S, int dim, int W, L
     cx<R> v[P], yv[P];
     const bool tw_in_lds = p.tw_lds;
     auto FFT = [&](int sign) {
-        if (tw_in_lds) fft_line<R, P>(v, ln, p, twl, sign, lt, active, kTwLds);
-        else fft_line<R, P>(v, ln, p, reinterpret_cast<const cx<R> *>(p.tw), sign, lt, active, kTwMem);
+        if (tw_in_lds) fft_line<R, P, false, GEN>(v, ln, p, twl, sign, lt, active, kTwLds);
+        else fft_line<R, P, false, GEN>(v, ln, p, reinterpret_cast<const cx<R> *>(p.tw), sign, lt, active, kTwMem);
     };
 
     if (active) {
@@ -231,10 +232,10 @@ __global__ void __launch_bounds__(512) k_apply_row(GridDev g, HamDev<R> h, LineP
     }
 }
 
-template <class R, int P>
-static void col_pass_P4(hipStream_t s, const GridDev &g, int S, int dim, int mode, const LinePlan &plan,
-                        const HamDev<R> &h, double tau, R *X, ChebyCtl *ctl, const ConvCheck &cc, int imag,
-                        const double *ek) {
+template <class R, int P, bool GEN>
+static void col_pass_P(hipStream_t s, const GridDev &g, int S, int dim, int mode, const LinePlan &plan,
+                       const HamDev<R> &h, double tau, R *X, ChebyCtl *ctl, const ConvCheck &cc, int imag,
+                       const double *ek) {
     const int L = g.N[dim];
     const int W = col_tile(g, S, dim, L, sizeof(cx<R>), P);
     const int nb = (g.N[0] / W) * col_nother(g, dim) * S;
@@ -245,79 +246,38 @@ static void col_pass_P4(hipStream_t s, const GridDev &g, int S, int dim, int mod
     pl.tw_lds = 1;
     const cx<R> *none = nullptr;
     const double *ekp = mode == 3 && !imag ? ek : nullptr;
+    auto launch = [&](auto kernel) {
+        set_lds(kernel, lds);
+        QDX_LAUNCH(kernel, dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
+        QDX_HIP(hipGetLastError());
+    };
     switch (mode) {
-    case 0:
-        set_lds(k_col<R, 0, P>, lds);
-        QDX_LAUNCH((k_col<R, 0, P>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
-        break;
-    case 1:
-        set_lds(k_col<R, 1, P>, lds);
-        QDX_LAUNCH((k_col<R, 1, P>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
-        break;
-    case 3:
-        if (imag) {
-            if constexpr (std::is_same<R, double>::value) {
-                set_lds(k_col<R, 3, P, true>, lds);
-                QDX_LAUNCH((k_col<R, 3, P, true>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x,
-                           none, ctl, cc, ekp);
-            } else {
-                throw std::runtime_error("imaginary time: FP64 only");
-            }
-            break;
-        }
-        set_lds(k_col<R, 3, P>, lds);
-        QDX_LAUNCH((k_col<R, 3, P>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
+    case 0: launch(k_col<R, 0, P, false, false, GEN>); break;
+    case 1: launch(k_col<R, 1, P, false, false, GEN>); break;
+    case 2:   // H psi
+        if constexpr (P == 8) launch(k_col<R, 2>);
+        else throw std::runtime_error("line pass: mode 0, 1 or 3 at 4 points per thread");
         break;
     default:
-        throw std::runtime_error("line pass: mode 0, 1 or 3 at 4 points per thread");
+        if (!imag) {
+            launch(k_col<R, 3, P, false, false, GEN>);
+        } else {
+            if constexpr (std::is_same<R, double>::value) launch(k_col<R, 3, P, true>);
+            else throw std::runtime_error("imaginary time: FP64 only");
+        }
+        break;
     }
-    QDX_HIP(hipGetLastError());
 }
 
 template <class R>
 void Launch<R>::col_pass(hipStream_t s, const GridDev &g, int S, int dim, int mode, const LinePlan &plan,
                          const HamDev<R> &h, double tau, R *X, ChebyCtl *ctl, const ConvCheck &cc, int imag,
                          const double *ek) {
-    if (plan.ppt == 4) return col_pass_P4<R, 4>(s, g, S, dim, mode, plan, h, tau, X, ctl, cc, imag, ek);
-    const int L = g.N[dim];
-    const int W = col_tile(g, S, dim, L, sizeof(cx<R>));
-    const int nb = (g.N[0] / W) * col_nother(g, dim) * S;
-    const int threads = std::max(64, round64(W * (L / 8)));
-    const size_t lds = col_lds_bytes(W, L, sizeof(cx<R>));
-    cx<R> *x = reinterpret_cast<cx<R> *>(X);
-    LinePlan pl = plan;
-    pl.tw_lds = 1;
-    const cx<R> *none = nullptr;
-    const double *ekp = mode == 3 && !imag ? ek : nullptr;
-    switch (mode) {
-    case 0:
-        set_lds(k_col<R, 0>, lds);
-        QDX_LAUNCH((k_col<R, 0>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
-        break;
-    case 1:
-        set_lds(k_col<R, 1>, lds);
-        QDX_LAUNCH((k_col<R, 1>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
-        break;
-    case 2:
-        set_lds(k_col<R, 2>, lds);
-        QDX_LAUNCH((k_col<R, 2>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
-        break;
-    default:
-        if (imag) {   // imaginary time: FP64 only
-            if constexpr (std::is_same<R, double>::value) {
-                set_lds(k_col<R, 3, 8, true>, lds);
-                QDX_LAUNCH((k_col<R, 3, 8, true>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none,
-                           ctl, cc, ekp);
-            } else {
-                throw std::runtime_error("imaginary time: FP64 only");
-            }
-            break;
-        }
-        set_lds(k_col<R, 3>, lds);
-        QDX_LAUNCH((k_col<R, 3>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, tau, x, none, ctl, cc, ekp);
-        break;
-    }
-    QDX_HIP(hipGetLastError());
+    const bool gen = plan.odd_prime();
+    if (plan.ppt == 4 && gen) col_pass_P<R, 4, true>(s, g, S, dim, mode, plan, h, tau, X, ctl, cc, imag, ek);
+    else if (plan.ppt == 4) col_pass_P<R, 4, false>(s, g, S, dim, mode, plan, h, tau, X, ctl, cc, imag, ek);
+    else if (gen) col_pass_P<R, 8, true>(s, g, S, dim, mode, plan, h, tau, X, ctl, cc, imag, ek);
+    else col_pass_P<R, 8, false>(s, g, S, dim, mode, plan, h, tau, X, ctl, cc, imag, ek);
 }
 
 // Mode 4 of k_col by the in-place line filter (qdx_gridfft.hpp): half the LDS
@@ -412,7 +372,7 @@ static bool kin_filter(hipStream_t s, const GridDev &g, int S, int dim, const Li
     return true;
 }
 
-template <class R, int P>
+template <class R, int P, bool GEN>
 static void kin_pass_P(hipStream_t s, const GridDev &g, int S, int dim, bool accumulate, const LinePlan &plan,
                        const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp) {
     const int L = g.N[dim];
@@ -425,36 +385,34 @@ static void kin_pass_P(hipStream_t s, const GridDev &g, int S, int dim, bool acc
     const double *ekp = nullptr;
     LinePlan pl = plan;
     pl.tw_lds = 1;
+    auto launch = [&](auto kernel) {
+        set_lds(kernel, lds);
+        QDX_LAUNCH(kernel, dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, 0.0, y, in, ctl, cc, ekp);
+        QDX_HIP(hipGetLastError());
+    };
     if (cmp) {
         if constexpr (std::is_same<R, double>::value) {
-            if (accumulate) {
-                set_lds(k_col<R, 5, P, false, true>, lds);
-                QDX_LAUNCH((k_col<R, 5, P, false, true>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, 0.0, y,
-                           in, ctl, cc, ekp);
-            } else {
-                set_lds(k_col<R, 4, P, false, true>, lds);
-                QDX_LAUNCH((k_col<R, 4, P, false, true>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, 0.0, y,
-                           in, ctl, cc, ekp);
-            }
+            if (accumulate) launch(k_col<R, 5, P, false, true, GEN>);
+            else launch(k_col<R, 4, P, false, true, GEN>);
         } else {
             throw std::runtime_error("compact terms: FP64 only");
         }
     } else if (accumulate) {
-        set_lds(k_col<R, 5, P>, lds);
-        QDX_LAUNCH((k_col<R, 5, P>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, 0.0, y, in, ctl, cc, ekp);
+        launch(k_col<R, 5, P, false, false, GEN>);
     } else {
-        set_lds(k_col<R, 4, P>, lds);
-        QDX_LAUNCH((k_col<R, 4, P>), dim3(nb), dim3(threads), lds, s, g, S, dim, W, pl, h, 0.0, y, in, ctl, cc, ekp);
+        launch(k_col<R, 4, P, false, false, GEN>);
     }
-    QDX_HIP(hipGetLastError());
 }
 
 template <class R>
 void Launch<R>::kin_pass(hipStream_t s, const GridDev &g, int S, int dim, bool accumulate, const LinePlan &plan,
                          const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp) {
     if (!accumulate && kin_filter<R>(s, g, S, dim, plan, h, src, Y, ctl, cc, cmp)) return;
-    if (plan.ppt == 4) kin_pass_P<R, 4>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
-    else kin_pass_P<R, 8>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
+    const bool gen = plan.odd_prime();
+    if (plan.ppt == 4 && gen) kin_pass_P<R, 4, true>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
+    else if (plan.ppt == 4) kin_pass_P<R, 4, false>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
+    else if (gen) kin_pass_P<R, 8, true>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
+    else kin_pass_P<R, 8, false>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
 }
 
 template <class R, int S>
