@@ -495,6 +495,18 @@ long run_fields(qdx_prop *p, qdx_ham *fop, int nf, long first, long n, long most
     return n;
 }
 
+// Steps of one dense launch.  It holds a CU that a persistent launch of another
+// context may need all the while, so it ends well within that one's wait
+// (kGridWait, 0.1 s): about 10 ms by the time an order or a split-operator step
+// takes (orders: 128 points 0.9 us, 512 points 3.6, 256 points and two states
+// 2.4; steps: 128 points 1.7 us, 384 points 4.0, 256 points and two coupled
+// states 6.1), a thousand times a launch's own cost.
+long dense_launch_steps(const qdx_prop *p) {
+    const double n2 = (double)p->grid.N[0] * p->grid.N[0] * p->S;
+    const double us = p->kind == qdx_prop::CHEBY ? (1.0 + 1.1e-5 * n2) * std::max(p->k_launch, 1) : 2.0 + 3.3e-5 * n2;
+    return std::max(1L, (long)(10000.0 / us));
+}
+
 // Steps first .. first + nsteps - 1 of a propagation that keeps to dense
 // lines.  obs (nullable): observables before each step, 4 S doubles per step;
 // orders (nullable): H applications per step (device arrays).  The host
@@ -524,9 +536,7 @@ void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *
         fop = p->ham;
     }
     const int nf = cheby ? S * S : 1;   // field values per step
-    // a launch runs at most 2^16 orders (2^14 split-operator steps): tens of
-    // milliseconds
-    const long most = cheby ? std::max(1L, 65536L / std::max(p->k_launch, 1)) : 16384L;
+    const long most = dense_launch_steps(p);
     for (long i = 0; i < nsteps;) {
         long n = std::min(most, nsteps - i);
         DenseRun a;

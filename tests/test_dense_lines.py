@@ -140,3 +140,32 @@ def test_clock_beyond_the_field(ctx):
         U.run(w, 0, 6)
     U.run(ref, 0, 4)
     assert np.array_equal(w.download(), ref.download())
+
+
+@pytest.mark.parametrize("N,S,kind,steps", [(512, 1, "cheby", 250), (256, 2, "cheby", 400), (128, 4, "cheby", 400),
+                                            (384, 1, "gspo", 9000), (256, 2, "gspo", 6000)])
+def test_launches_are_short(N, S, kind, steps):
+    """A long run comes in launches of about 10 ms: another context's
+    persistent launch waits 0.1 s for the CU.  Twice that covers a clock
+    that has not ramped up."""
+    import qdng_amd as Q
+    print("[gpu case] dense launch length", N, S, kind, flush=True)
+    c = Q.Context(0)
+    try:
+        p = line(N, S)
+        if kind == "cheby":
+            H = p.gpu_ham(c)
+            lo, hi = H.bounds()
+            U = Q.Cheby(H, 50.0 / (hi - lo), prec=1e-10)
+        else:
+            U = Q.GSPO([p.gpu_split_op(c, [k]) for k in ("kin", "pot")], 0.5)
+        w = p.gpu_wf(c)
+        c.profile(True)
+        U.run(w, 0, steps)
+        n, ms = c.kernel_time(Q.K_CHEBY_ROW if kind == "cheby" else Q.K_GSPO_ROW)
+        c.profile(False)
+        assert ms > 20.0, "the run is too short to need two launches"
+        assert ms / n < 20.0
+        del U, w
+    finally:
+        c.close()
