@@ -484,6 +484,20 @@ int qdx_ctx_get_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, int32_t *
 int qdx_ctx_set_line_points(qdx_ctx *ctx, int32_t points);
 int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points);
 
+/* Waits of the persistent kernels.  Whole propagations of 2D grids run in
+ * launches whose blocks wait for each other.  Where other work holds the GPU's
+ * CUs a wait can last; past its bound (0.1 s) the launch gives up without a
+ * trace in psi, its steps run by the per-order kernels and the next launch tries
+ * again, after three misses in a row only every 64 steps, then more rarely.
+ * Results are those of the per-order kernels for the steps concerned (equal
+ * up to rounding).  set_wait_limit: after `skip` further launches on this context
+ * the next `count` bound their waits by `us` microseconds instead (at most 10^6;
+ * 0: they give up at the first wait, which serves to test callers).
+ * persistent_stats: launches so far and those that gave up (either may be
+ * NULL).  No QDng counterpart (its propagators run on the host). */
+int qdx_ctx_set_wait_limit(qdx_ctx *ctx, int64_t us, int64_t skip, int64_t count);
+int qdx_ctx_persistent_stats(qdx_ctx *ctx, int64_t *launches, int64_t *given_up);
+
 /* Tile shape of the batched kernels for 2D Chebyshev jobs of one grid
  * shape.  Row tiles: row_lines lines of dimension 0 (N0/8 threads each) in a
  * block of row_threads (256 or 512) threads.  Column tiles: col_width

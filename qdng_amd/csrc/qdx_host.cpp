@@ -497,7 +497,7 @@ long run_fields(qdx_prop *p, qdx_ham *fop, int nf, long first, long n, long most
 
 // Steps of one dense launch.  It holds a CU that a persistent launch of another
 // context may need all the while, so it ends well within that one's wait
-// (kGridWait, 0.1 s): about 10 ms by the time an order or a split-operator step
+// (kGridWaitUs, 0.1 s): about 10 ms by the time an order or a split-operator step
 // takes (orders: 128 points 0.9 us, 512 points 3.6, 256 points and two states
 // 2.4; steps: 128 points 1.7 us, 384 points 4.0, 256 points and two coupled
 // states 6.1), a thousand times a launch's own cost.
@@ -568,9 +568,32 @@ void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *
 
 // qdx_ctx_set_line_points 4 or 8 asks for the per-order kernels
 bool grid_on(const qdx_prop *p) { return p->grid2d && p->ctx->line_ppt == 0; }
+// ... and so do launches that gave up again and again (grid_missed)
+bool grid_ready(const qdx_prop *p) { return grid_on(p) && p->gskip == 0; }
+
+// Usual bound of a wait: a launch whose blocks are all on the chip waits for
+// microseconds, one that shares the GPU for as long as the others' kernels run.
+constexpr int64_t kGridWaitUs = 100000;
+
+// the bound of the waits of the next persistent launch, in ticks of 10 ns
+unsigned grid_wait_ticks(qdx_ctx *c) {
+    const int64_t i = c->grid_launches++ - c->wait_first;
+    const bool set = i >= 0 && i < c->wait_count;
+    return (unsigned)(100 * (set ? c->wait_us : kGridWaitUs));
+}
+
+// A launch gave up waiting for its blocks.  Its steps go by the per-order
+// kernels; the next launch tries again, but from the third miss in a row on (each
+// costs the bound of a wait) only after 64 steps, then 128, ... 4096.
+void grid_missed(qdx_prop *p) {
+    HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, p->ctx->stream));
+    p->gepoch = 0;
+    ++p->ctx->grid_missed;
+    if (++p->gmiss >= 3) p->gskip = 64L << std::min(p->gmiss - 3, 6);
+}
 
 // what a launch of n steps of the persistent kernels needs; signals: the flags'
-// values it uses at most
+// values it uses at most (0: it waits for none)
 GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const double *psi0, int *orders) {
     GridRun a;
     a.nsteps = (int)n;
@@ -581,6 +604,7 @@ GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const doubl
     }
     a.epoch = p->gepoch;
     p->gepoch += signals;
+    if (signals) a.wait = grid_wait_ticks(p->ctx);
     a.sync = p->gflags.as<char>();
     a.status = reinterpret_cast<int *>(a.sync + kGridSyncBytes);
     a.A = p->phiA.p;
@@ -594,18 +618,24 @@ GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const doubl
     return a;
 }
 
-// After a launch: psi and the observables; false, and the propagator keeps to
-// the per-order kernels from then on, when it gave up waiting for its blocks
-// (psi is unchanged then).
+// After a launch: psi and the observables; false when it gave up waiting for its
+// blocks (psi is unchanged then).
 bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, double *obs) {
     hipStream_t s = p->ctx->stream;
     launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->greport);
     HIPCHK(hipStreamSynchronize(s));
-    if (!*p->greport) return true;
-    HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, s));
-    p->gepoch = 0;
-    p->grid2d = false;
-    return false;
+    if (*p->greport) {
+        grid_missed(p);
+        return false;
+    }
+    p->gmiss = 0;
+    return true;
+}
+
+// steps of one launch at most: 2048 orders or split-operator steps, tens of
+// milliseconds
+long grid_launch_steps(const qdx_prop *p) {
+    return p->kind == qdx_prop::CHEBY ? std::max(1L, 2048L / std::max(p->k_launch, 1)) : 2048L;
 }
 
 // Two persistent launches at once could each hold CUs that the other waits
@@ -617,7 +647,7 @@ std::mutex &grid_mutex(int device) {
 
 // Steps first .. first + nsteps - 1 by the persistent kernels, as dense_run;
 // returns the steps done, fewer than nsteps when a launch gave up (grid_end):
-// the caller goes on with the per-order kernels.  split: a single step by
+// the caller does its steps by the per-order kernels.  split: a single step by
 // launches that wait for nothing, where there are such (split operator).
 template <class R>
 long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *psi0, double *obs, int *orders,
@@ -648,9 +678,7 @@ long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *p
         for (int i = 0; i < pre.n; ++i) coupled = coupled || pre.op[i].coupled;
         ek = kinetic_exp_table(p, p->ops[0], p->dt);
     }
-    // a launch runs at most 2048 orders or split-operator steps: tens of
-    // milliseconds
-    const long most = cheby ? std::max(1L, 2048L / std::max(p->k_launch, 1)) : 2048L;
+    const long most = grid_launch_steps(p);
     for (long i = 0; i < nsteps;) {
         long n = std::min(most, nsteps - i);
         const double *fields = nullptr;
@@ -751,12 +779,12 @@ double cheby_last_nconv(qdx_prop *p) {
 void sil_step(qdx_prop *p, qdx_wf *psi, long step);
 void arnoldi_step(qdx_prop *p, qdx_wf *psi, long step);
 
-void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32);
+void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32, bool orders);
 
 // steps of a propagation that keeps to the persistent kernels.  Backward
 // split-operator steps, which run one by one, take the per-order kernels: one
 // launch that is waited for costs more than their three.
-bool grid_steps(const qdx_prop *p) { return grid_on(p) && !(p->kind == qdx_prop::GSPO && p->backward); }
+bool grid_steps(const qdx_prop *p) { return grid_ready(p) && !(p->kind == qdx_prop::GSPO && p->backward); }
 
 // FP32 split-operator propagation holds psi in FP32 between the steps (the
 // dense line kernels and the persistent ones keep complex128 between launches)
@@ -768,17 +796,18 @@ bool psi_in_fp32(const qdx_prop *p) {
 // conjugated, OPropagator.h:82-100): exp(+i H* dt) psi = conj(exp(-i H dt)
 // conj(psi)), the forward step between two conjugations (exact: conjugation
 // commutes with every rounding of the forward step)
-// g32: the caller holds psi in FP32 (psi_in_fp32 when it began)
-void prop_step(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
-    if (!p->backward) return prop_step_forward(p, psi, step, g32);
+// g32: the caller holds psi in FP32 (psi_in_fp32 when it began); orders: not by
+// the persistent kernels
+void prop_step(qdx_prop *p, qdx_wf *psi, long step, bool g32, bool orders = false) {
+    if (!p->backward) return prop_step_forward(p, psi, step, g32, orders);
     void *d = g32 ? static_cast<void *>(p->psi32.as<float>()) : static_cast<void *>(psi->ptr());
     const long n = (long)p->S * psi->n();
     launch_conj(p->ctx->stream, d, n, g32);
-    prop_step_forward(p, psi, step, g32);
+    prop_step_forward(p, psi, step, g32, orders);
     launch_conj(p->ctx->stream, d, n, g32);
 }
 
-void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
+void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32, bool orders) {
     if (p->kind == qdx_prop::SIL) {
         sil_step(p, psi, step);
         return;
@@ -792,9 +821,11 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
         dense_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep);
         return;
     }
-    if (grid_steps(p) && !g32) {
+    if (!orders && !g32 && grid_steps(p)) {
         StreamKeep keep{p->ctx->stream, {}};
         if (grid_run(p, psi, step, 1, nullptr, nullptr, nullptr, keep, true) == 1) return;
+    } else if (!orders && grid_on(p) && p->gskip > 0) {
+        --p->gskip;
     }
     if (p->kind == qdx_prop::CHEBY) {
         // QDX_COMPACT: FP64 arithmetic (compact terms when p->cmp)
@@ -803,7 +834,7 @@ void prop_step_forward(qdx_prop *p, qdx_wf *psi, long step, bool g32) {
         // record executed order count of this step
     } else {
         if (p->precision == QDX_FP32_BULK) {
-            // the caller holds psi in complex128 when a persistent launch gave up
+            // the caller may hold psi in complex128 (a persistent launch gave up)
             const long n = (long)p->S * psi->n();
             if (!g32) launch_convert_c128_to_c64(p->ctx->stream, psi->ptr(), p->psi32.as<float>(), n);
             gspo_step<float>(p, p->psi32.as<float>(), step);
@@ -907,6 +938,25 @@ int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points) {
     return guarded([&] {
         if (!ctx || !points) fail(QDX_ERR_PARAM, "NULL argument");
         *points = ctx->line_ppt;
+    });
+}
+
+int qdx_ctx_set_wait_limit(qdx_ctx *ctx, int64_t us, int64_t skip, int64_t count) {
+    return guarded([&] {
+        if (!ctx) fail(QDX_ERR_PARAM, "ctx is NULL");
+        if (us < 0 || us > 1000000) fail(QDX_ERR_PARAM, "wait limit: 0 to 1000000 us");
+        if (skip < 0 || count < 0) fail(QDX_ERR_PARAM, "negative launch count");
+        ctx->wait_us = us;
+        ctx->wait_first = ctx->grid_launches + skip;
+        ctx->wait_count = count;
+    });
+}
+
+int qdx_ctx_persistent_stats(qdx_ctx *ctx, int64_t *launches, int64_t *given_up) {
+    return guarded([&] {
+        if (!ctx) fail(QDX_ERR_PARAM, "ctx is NULL");
+        if (launches) *launches = ctx->grid_launches;
+        if (given_up) *given_up = ctx->grid_missed;
     });
 }
 
@@ -1645,72 +1695,89 @@ int qdx_prop_run(qdx_prop *p, qdx_wf *psi, int64_t first_step, int64_t nsteps, q
         const size_t per_step = 4 * S;
         p->obs.alloc(std::max<size_t>(1, (size_t)nsteps * per_step + nsteps) * sizeof(double));
         double *obs = p->obs.as<double>();
-        int *orders = reinterpret_cast<int *>(obs + nsteps * per_step);
-        // whole runs by one kernel (an autocorrelation with the propagated
-        // function itself follows it step by step)
-        const bool whole = !p->backward && !(autocorr && psi0->ptr() == psi->ptr());
-        StreamKeep keep{s, {}};
-        int64_t done = 0;
-        if (whole && (dense_on(p) || grid_steps(p))) {
-            const double *z = autocorr ? psi0->ptr() : nullptr;
-            double *o = norm2 || autocorr ? obs : nullptr;
-            int *ord = p->kind == qdx_prop::CHEBY ? orders : nullptr;
-            done = nsteps;
-            if (dense_on(p)) dense_run(p, psi, first_step, nsteps, z, o, ord, keep);
-            else done = grid_run(p, psi, first_step, nsteps, z, o, ord, keep);
-        }
-        // (split operator: the fused run, which reads that psi0 before it writes psi)
-        const bool self = !whole && !p->backward && gspo_fusable(p).ok;
-        const bool g32 = psi_in_fp32(p) || (self && p->precision == QDX_FP32_BULK);
-        if (g32) {
-            launch_convert_c128_to_c64(s, psi->ptr(), p->psi32.as<float>(), (long)S * n);
-            if (autocorr) {
-                p->psi0_32.alloc((size_t)S * n * 2 * sizeof(float));
-                launch_convert_c128_to_c64(s, psi0->ptr(), p->psi0_32.as<float>(), (long)S * n);
-            }
-        }
+        int *orders_d = reinterpret_cast<int *>(obs + nsteps * per_step);
         double *part = p->partials.as<double>();
         if (!part || p->partials.bytes < kMaxPartials * sizeof(double))
             fail(QDX_ERR_STATE, "propagator has no reduction buffer for the observables");
         std::vector<int> sil_counts;
-        const bool fused = done == 0 && nsteps > 0 && !p->backward && (self || !grid_on(p)) && gspo_fusable(p).ok;
-        if (fused) {
-            // observables before step 0 here; those before the later steps
-            // from the row passes between the steps (psi0: autocorrelation)
-            double *o = obs;
-            const bool want = norm2 || autocorr;
+        const bool want = norm2 || autocorr;
+        // whole runs by one kernel (an autocorrelation with the propagated
+        // function itself follows it step by step)
+        const bool whole = !p->backward && !(autocorr && psi0->ptr() == psi->ptr());
+        // (split operator: the fused run, which reads that psi0 before it writes psi)
+        const bool self = !whole && !p->backward && gspo_fusable(p).ok;
+        // Steps i0 .. i0 + m - 1 one by one or as a fused split-operator run;
+        // orders: by the per-order kernels, in place of the persistent ones
+        auto step_by_step = [&](int64_t i0, int64_t m, bool orders) {
+            const bool g32 = p->kind == qdx_prop::GSPO && p->precision == QDX_FP32_BULK &&
+                             (orders || self || psi_in_fp32(p));
             if (g32) {
-                float *ps = p->psi32.as<float>();
-                const float *p0 = autocorr ? p->psi0_32.as<float>() : ps;
-                if (norm2) launch_overlap_c64(s, ps, ps, n, S, part, o);
-                if (autocorr) launch_overlap_c64(s, ps, p0, n, S, part, o + 2 * S);
-                gspo_run_fused<float>(p, ps, p0, first_step, nsteps, want ? obs : nullptr, per_step);
-            } else {
-                double *ps = psi->ptr();
-                const double *p0 = autocorr ? psi0->ptr() : ps;
-                if (norm2) launch_overlap(s, ps, ps, n, S, part, o);
-                if (autocorr) launch_overlap(s, ps, p0, n, S, part, o + 2 * S);
-                gspo_run_fused<double>(p, ps, p0, first_step, nsteps, want ? obs : nullptr, per_step);
+                launch_convert_c128_to_c64(s, psi->ptr(), p->psi32.as<float>(), (long)S * n);
+                if (autocorr) {
+                    if (p->psi0_32.bytes != (size_t)S * n * 2 * sizeof(float))
+                        p->psi0_32.alloc((size_t)S * n * 2 * sizeof(float));
+                    launch_convert_c128_to_c64(s, psi0->ptr(), p->psi0_32.as<float>(), (long)S * n);
+                }
             }
+            if (m > 0 && !p->backward && (orders || self || !grid_on(p)) && gspo_fusable(p).ok) {
+                // observables before step i0 here; those before the later steps
+                // from the row passes between the steps (psi0: autocorrelation)
+                double *o = obs + i0 * per_step;
+                if (g32) {
+                    float *ps = p->psi32.as<float>();
+                    const float *p0 = autocorr ? p->psi0_32.as<float>() : ps;
+                    if (norm2) launch_overlap_c64(s, ps, ps, n, S, part, o);
+                    if (autocorr) launch_overlap_c64(s, ps, p0, n, S, part, o + 2 * S);
+                    gspo_run_fused<float>(p, ps, p0, first_step + i0, m, want ? o : nullptr, per_step);
+                } else {
+                    double *ps = psi->ptr();
+                    const double *p0 = autocorr ? psi0->ptr() : ps;
+                    if (norm2) launch_overlap(s, ps, ps, n, S, part, o);
+                    if (autocorr) launch_overlap(s, ps, p0, n, S, part, o + 2 * S);
+                    gspo_run_fused<double>(p, ps, p0, first_step + i0, m, want ? o : nullptr, per_step);
+                }
+                m = 0;
+            }
+            for (int64_t i = i0; i < i0 + m; ++i) {
+                double *o = obs + i * per_step;
+                if (norm2) {
+                    if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi32.as<float>(), n, S, part, o);
+                    else launch_overlap(s, psi->ptr(), psi->ptr(), n, S, part, o);
+                }
+                if (autocorr) {
+                    if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi0_32.as<float>(), n, S, part, o + 2 * S);
+                    else launch_overlap(s, psi->ptr(), psi0->ptr(), n, S, part, o + 2 * S);
+                }
+                prop_step(p, psi, first_step + i, g32, orders);
+                if (p->kind == qdx_prop::CHEBY)
+                    HIPCHK(hipMemcpyAsync(orders_d + i, &p->ctl.as<ChebyCtl>()->last_order, sizeof(int),
+                                          hipMemcpyDeviceToDevice, s));
+                if (p->kind == qdx_prop::SIL || p->kind == qdx_prop::ARNOLDI) sil_counts.push_back(p->sil_napply);
+            }
+            if (g32) launch_convert_c64_to_c128(s, p->psi32.as<float>(), psi->ptr(), (long)S * n);
+        };
+        StreamKeep keep{s, {}};
+        const double *z = autocorr ? psi0->ptr() : nullptr;
+        int *ord = p->kind == qdx_prop::CHEBY ? orders_d : nullptr;
+        if (whole && dense_on(p)) {
+            dense_run(p, psi, first_step, nsteps, z, want ? obs : nullptr, ord, keep);
+        } else if (whole && grid_on(p)) {
+            for (int64_t done = 0; done < nsteps;) {
+                int64_t m = p->gskip;   // after launches that gave up
+                if (m == 0) {
+                    done += grid_run(p, psi, first_step + done, nsteps - done, z,
+                                     want ? obs + done * per_step : nullptr, ord ? ord + done : nullptr, keep);
+                    if (done == nsteps) break;
+                    m = grid_launch_steps(p);   // that launch gave up
+                }
+                m = std::min<int64_t>(m, nsteps - done);
+                step_by_step(done, m, true);
+                done += m;
+                p->gskip = std::max<int64_t>(0, p->gskip - m);
+            }
+        } else {
+            step_by_step(0, nsteps, false);
         }
-        if (fused) done = nsteps;
-        for (int64_t i = done; i < nsteps; ++i) {
-            double *o = obs + i * per_step;
-            if (norm2) {
-                if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi32.as<float>(), n, S, part, o);
-                else launch_overlap(s, psi->ptr(), psi->ptr(), n, S, part, o);
-            }
-            if (autocorr) {
-                if (g32) launch_overlap_c64(s, p->psi32.as<float>(), p->psi0_32.as<float>(), n, S, part, o + 2 * S);
-                else launch_overlap(s, psi->ptr(), psi0->ptr(), n, S, part, o + 2 * S);
-            }
-            prop_step(p, psi, first_step + i, g32);
-            if (p->kind == qdx_prop::CHEBY)
-                HIPCHK(hipMemcpyAsync(orders + i, &p->ctl.as<ChebyCtl>()->last_order, sizeof(int),
-                                      hipMemcpyDeviceToDevice, s));
-            if (p->kind == qdx_prop::SIL || p->kind == qdx_prop::ARNOLDI) sil_counts.push_back(p->sil_napply);
-        }
-        if (g32) launch_convert_c64_to_c128(s, p->psi32.as<float>(), psi->ptr(), (long)S * n);
         std::vector<double> host((size_t)nsteps * per_step + nsteps);
         if (nsteps > 0)
             HIPCHK(hipMemcpyAsync(host.data(), obs, host.size() * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -2326,6 +2393,10 @@ bool sil_grid_basis(qdx_prop *p, qdx_wf *psi, long step, std::vector<double> &al
                     int &convorder, int &napply) {
     qdx_ctx *ctx = p->ctx;
     if (!p->sil_grid || ctx->line_ppt != 0) return false;
+    if (p->gskip > 0) {
+        --p->gskip;
+        return false;
+    }
     const int order = p->sil_order;
     hipStream_t s = ctx->stream;
     p->ham->finalize();
@@ -2345,11 +2416,10 @@ bool sil_grid_basis(qdx_prop *p, qdx_wf *psi, long step, std::vector<double> &al
         HIPCHK(hipStreamSynchronize(s));
     }
     if (*p->greport) {
-        HIPCHK(hipMemsetAsync(p->gflags.p, 0, p->gflags.bytes, s));
-        p->gepoch = 0;
-        p->sil_grid = false;
+        grid_missed(p);
         return false;
     }
+    p->gmiss = 0;
     const int it = (int)res[1];
     if (!std::isfinite(res[0])) fail(QDX_ERR_OVERFLOW, "Norm is not a number");
     for (int i = 0; i < order; ++i) {

@@ -341,6 +341,11 @@ struct qdx_ctx {
     // points per thread of the single propagator's Chebyshev line kernels:
     // 0 chooses (4 on grids that give fewer than two waves per SIMD at 8)
     int line_ppt = 0;
+    // persistent launches (qdx_grid.hip) so far and those that gave up waiting;
+    // qdx_ctx_set_wait_limit: the launches that take wait_us instead of the
+    // usual bound, from number wait_first on
+    int64_t grid_launches = 0, grid_missed = 0;
+    int64_t wait_us = 0, wait_first = 0, wait_count = 0;
     LinePlan plan(int L, bool fp32, const std::vector<int> &r) {
         auto &tab = fp32 ? tw32 : tw64;
         auto it = tab.find(L);
@@ -969,12 +974,16 @@ struct qdx_prop {
     // tables (GSPO: real part, then imaginary part)
     bool dense = false;
     DevBuf dtab, dfields;
-    // 2D grids that fit the chip's registers (Chebyshev): whole runs in one
-    // launch (qdx_grid.hip); gepoch: the flags' values so far
+    // 2D grids that fit the chip's registers (Chebyshev, split operator): whole
+    // runs in one launch (qdx_grid.hip); gepoch: the flags' values so far
     bool grid2d = false;
     GridShape gs;
     DevBuf gflags, gobs;
     unsigned gepoch = 0;
+    // launches that gave up in a row, and the steps that go by the per-order
+    // kernels before the next try
+    int gmiss = 0;
+    long gskip = 0;
     bool sil_grid = false;    // the Lanczos basis by the persistent kernel
     int *greport = nullptr;   // host memory: status of the last launch
     int last_nb = 0, nb_init = 0;   // partial counts of the last Chebyshev step

@@ -202,3 +202,86 @@ def test_lanczos(N0, N1, S, order, imag):
         return p, Q.SIL(H, 2.0 / (hi - lo), order=order, imag=imag)
     check(both(make, 3, True), 1e-10)
     check(both(make, 2, False), 1e-10)
+
+
+def propagator(c, kind, precision="fp64", nt=12):
+    """(problem, propagator) on 40 x 24 points, a few orders per step"""
+    import qdng_amd as Q
+    laser = kind not in ("imag", "gspo2")
+    p = box(40, 24, 2 if kind == "gspo2" else 1, laser, nt=nt)
+    if kind.startswith("gspo"):
+        ops = [p.gpu_split_op(c, [k]) for k in (("kin", "pot", "dip") if laser else ("kin", "pot"))]
+        return p, Q.GSPO(ops, 0.5, precision=precision)
+    H = p.gpu_ham(c)
+    lo, hi = H.bounds()
+    if kind == "sil":
+        return p, Q.SIL(H, 2.0 / (hi - lo))
+    return p, Q.Cheby(H, 3.0 / (hi - lo), prec=1e-12, precision=precision, imag=kind == "imag")
+
+
+# The steps of a launch that gave up are those of the per-order kernels: the
+# bounds of the comparisons above.  FP32 split operator: each step rounds psi to
+# 2^-24 about five times, 3e-7, which adds up like a random walk over 2100 steps
+# to 1.4e-5; 1e-4 leaves a factor of seven.
+@pytest.mark.parametrize("skip", [0, 1])
+@pytest.mark.parametrize("kind,precision,steps,tol", [
+    ("cheby", "fp64", 300, 1e-11), ("cheby", "fp32", 300, 1e-4), ("cheby", "compact", 300, 5e-7),
+    ("gspo", "fp64", 2100, 1e-11), ("gspo", "fp32", 2100, 1e-4), ("gspo2", "fp64", 2100, 1e-11),
+    ("gspo2", "fp32", 2100, 1e-4), ("sil", "fp64", 3, 1e-10)])
+def test_launch_that_gives_up_in_a_run(kind, precision, steps, tol, skip):
+    """A launch of a run of several gives up (the first or the second): its
+    steps go by the per-order kernels, the launches behind it are persistent
+    again, and the report is whole."""
+    import qdng_amd as Q
+    print("[gpu case] grid give-up", kind, precision, steps, skip, flush=True)
+    out = []
+    for points in (0, 8):
+        c = Q.Context(0)
+        try:
+            c.set_line_points(points)
+            p, U = propagator(c, kind, precision, steps + 2)
+            w, w0 = p.gpu_wf(c), p.gpu_wf(c)
+            c.set_wait_limit(0, skip, 1)
+            n2, ac, nh, _ = U.run(w, 1, steps, w0)
+            out.append((w.download(), np.array(n2), np.array(ac), list(nh)))
+            launches, missed = c.persistent_stats()
+            assert (missed == 1 and launches >= 2) if points == 0 else launches == 0
+            del U, w, w0
+        finally:
+            c.close()
+    check(out, tol)
+
+
+@pytest.mark.parametrize("kind,precision,tol", [("cheby", "fp64", 1e-11), ("cheby", "compact", 5e-8),
+                                                ("cheby", "fp32", 1e-5), ("imag", "fp64", 1e-11)])
+def test_single_steps_that_give_up(kind, precision, tol):
+    """Three misses in a row: 64 steps go by the per-order kernels, then the
+    launches are tried again."""
+    import qdng_amd as Q
+    print("[gpu case] grid give-up, single steps", kind, precision, flush=True)
+    c, d = Q.Context(0), Q.Context(0)
+    try:
+        d.set_line_points(8)
+        p, U = propagator(c, kind, precision, 80)
+        _, V = propagator(d, kind, precision, 80)
+        w, v = p.gpu_wf(c), p.gpu_wf(d)
+        c.set_wait_limit(0, 0, 3)
+        want = [1, 2, 3] + [3] * 64 + [4, 5]
+        for i, n in enumerate(want):
+            assert U.apply(w, i).n_hpsi == V.apply(v, i).n_hpsi
+            assert c.persistent_stats() == (n, min(n, 3))
+            if i in (0, 3, 68):
+                assert rel(w.download(), v.download()) < tol * (i + 1)
+            w.normalize()
+            v.normalize()
+        del U, V, w, v
+    finally:
+        c.close()
+        d.close()
+
+
+def test_wait_limit_arguments(ctx):
+    import qdng_amd as Q
+    for bad in [(-1, 0, 1), (1000001, 0, 1), (0, -1, 1), (0, 0, -1)]:
+        with pytest.raises(Q.QdxError):
+            ctx.set_wait_limit(*bad)
