@@ -490,7 +490,10 @@ int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points);
  * trace in psi, its steps run by the per-order kernels and the next launch tries
  * again, after three misses in a row only every 64 steps, then more rarely.
  * Results are those of the per-order kernels for the steps concerned (equal
- * up to rounding).  set_wait_limit: after `skip` further launches on this context
+ * up to rounding).  Persistent launches of several threads of a process go side
+ * by side as long as their blocks (one per line, at least 512 points each)
+ * together are no more than the device's CUs, else one after the other.
+ * set_wait_limit: after `skip` further launches on this context
  * the next `count` bound their waits by `us` microseconds instead (at most 10^6;
  * 0: they give up at the first wait, which serves to test callers).
  * persistent_stats: launches so far and those that gave up (either may be

@@ -27,8 +27,8 @@
 // epochs that grow over all launches of a propagator.
 //
 // All blocks have to be on the chip together: there are at most as many as
-// CUs, each fits a CU by itself, and the host lets one such launch run per
-// device and process at a time.  (Cooperative launches would say so to the
+// CUs, each fits a CU by itself, and the host lets no more such launches run at a
+// time, per device and process, than their blocks have CUs.  (Cooperative launches would say so to the
 // runtime, but they cost 20 us more, and once a process has made one its other
 // streams run slower: a batch of jobs 34 -> 45 ms.)  Other processes on the
 // GPU can still hold CUs, so every wait is bounded (GridRun::wait): a block that

@@ -978,6 +978,7 @@ struct qdx_prop {
     // runs in one launch (qdx_grid.hip); gepoch: the flags' values so far
     bool grid2d = false;
     GridShape gs;
+    int cus = 0;              // CUs of the device
     DevBuf gflags, gobs;
     unsigned gepoch = 0;
     // launches that gave up in a row, and the steps that go by the per-order

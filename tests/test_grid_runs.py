@@ -285,3 +285,50 @@ def test_wait_limit_arguments(ctx):
     for bad in [(-1, 0, 1), (1000001, 0, 1), (0, -1, 1), (0, 0, -1)]:
         with pytest.raises(Q.QdxError):
             ctx.set_wait_limit(*bad)
+
+
+def test_threads():
+    """Four contexts in four threads, two grids that share the chip and two
+    that need all of it: the bits of runs one after the other, no launch gives
+    up."""
+    import threading
+
+    import qdng_amd as Q
+    print("[gpu case] grid threads", flush=True)
+    shapes = [(64, 64, 1, "cheby"), (256, 64, 1, "gspo"), (512, 512, 2, "cheby"), (256, 256, 1, "sil")]
+
+    def start(N0, N1, S, kind):
+        c = Q.Context(0)
+        p = box(N0, N1, S)
+        H = p.gpu_ham(c)
+        lo, hi = H.bounds()
+        if kind == "gspo":
+            U = Q.GSPO([p.gpu_split_op(c, [k]) for k in ("kin", "pot")], 0.5)
+        else:
+            U = Q.SIL(H, 2.0 / (hi - lo)) if kind == "sil" else Q.Cheby(H, 20.0 / (hi - lo), prec=1e-10)
+        return c, U, p.gpu_wf(c), p.gpu_wf(c)
+
+    def work(prog, out):
+        c, U, w, w0 = prog
+        w.copy_from(w0)
+        for i in range(6):
+            U.run(w, i * 20, 20, w0)
+        out.append(w.download())
+
+    progs = [start(*s) for s in shapes]
+    try:
+        alone, together = [[] for _ in shapes], [[] for _ in shapes]
+        for g, o in zip(progs, alone):
+            work(g, o)
+        threads = [threading.Thread(target=work, args=a) for a in zip(progs, together)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert all(np.array_equal(a, b) for a, b in zip(alone, together))
+        assert all(g[0].persistent_stats()[1] == 0 for g in progs)
+    finally:
+        ctxs = [g[0] for g in progs]
+        progs.clear()
+        for c in ctxs:
+            c.close()
