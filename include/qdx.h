@@ -460,7 +460,11 @@ int qdx_batch_graph_stats(qdx_batch *b, int64_t *captured, int64_t *replayed);
  * middle 8, 4, 3, 2 or a prime 5 .. 31; at most 16).  A plan set here is used by the
  * propagators and Hamiltonians created and the batch jobs submitted
  * afterwards on this context (a batch job keeps the plans it was submitted
- * with).  Different plans give the same transform up to rounding. */
+ * with).  Propagators with a side of that length then run the kernels that
+ * transform by plans instead of those with a factorisation of their own (see
+ * qdx_ctx_set_line_points); plans that the batch's autotuner or a tuning file
+ * installs do not change that choice.  Different plans give the same transform
+ * up to rounding. */
 int qdx_ctx_set_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, const int32_t *radix, int32_t nst);
 /* the plan in use for length L (radix: room for 16) */
 int qdx_ctx_get_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, int32_t *radix, int32_t *nst);
@@ -479,7 +483,9 @@ int qdx_ctx_get_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, int32_t *
  * states; split operator up to 384) and 2D grids of up to 2^19 points and
  * states (Chebyshev, split operator, short iterative Lanczos; one or two
  * states) run whole propagations in one kernel instead; 4 or 8 selects the
- * kernels above for them too.  No
+ * kernels above for them too, and the context's plans in the kinetic pass along
+ * dimension 1, which 0 runs with a factorisation of its own where the line has
+ * one.  No
  * QDng counterpart: FFTW lays out its own threads (src/fft/fft.cpp:95-110). */
 int qdx_ctx_set_line_points(qdx_ctx *ctx, int32_t points);
 int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points);

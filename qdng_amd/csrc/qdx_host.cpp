@@ -97,7 +97,8 @@ void cheby_step(qdx_prop *p, qdx_wf *psi, long step) {
     auto cols = [&](const R *pm1, const ConvCheck &c) {
         for (int d = 1; d < p->grid.nd; ++d) {
             KTimer t(ctx, QDX_K_LINE_PASS);
-            Launch<R>::kin_pass(s, g, S, d, d > 1, plans[d], h, pm1, X, ctl, c, p->cmp);
+            Launch<R>::kin_pass(s, g, S, d, d > 1, plans[d], h, pm1, X, ctl, c, p->cmp,
+                                ctx->line_ppt == 0 && !p->own_plan);
         }
     };
     // exp(exponent * offset), exponent -i dt (real time) or -dt (imaginary);
@@ -778,7 +779,7 @@ void grid_buffers(qdx_prop *p, size_t es) {
 // the block shape of a 2D grid on this device; false: it takes the per-order
 // kernels
 bool grid_fits(qdx_prop *p) {
-    if (p->grid.nd != 2) return false;
+    if (p->grid.nd != 2 || p->own_plan) return false;
     HIPCHK(hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, p->ctx->device));
     return grid_shape(p->grid.N[0], p->grid.N[1], p->S, p->cus, p->kind == qdx_prop::GSPO, p->gs);
 }
@@ -944,6 +945,7 @@ int qdx_ctx_set_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, const int
         std::vector<int> r(radix, radix + nst);
         if (!radix_ok(L, r)) fail(QDX_ERR_PARAM, "radix plan does not fit the line length");
         ctx->radix[{L, precision == QDX_FP32_BULK}] = r;
+        ctx->own_plans.insert({L, precision == QDX_FP32_BULK});
     });
 }
 
@@ -1493,6 +1495,7 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
         if (precision == QDX_FP32_BULK) h->ensure32();
         // element bytes of the term buffers (compact: 8 hi + 2 lo)
         const size_t es = p->cmp ? 10 : precision == QDX_FP32_BULK ? 2 * sizeof(float) : 2 * sizeof(double);
+        p->own_plan = p->ctx->plan_set(p->grid, precision == QDX_FP32_BULK);
         p->grid2d = grid_fits(p.get());
         if (p->grid2d) {
             grid_buffers(p.get(), p->cmp ? 16 : es);   // compact terms are exchanged as complex128
@@ -1516,7 +1519,7 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
         p->line_step = !imag && p->grid.nd == 1 && p->S == 1 &&
                        p->grid.N[0] <= (precision == QDX_FP32_BULK ? kMaxLine : 2048) &&
                        line_lds <= 160 * 1024;
-        p->dense = p->grid.nd == 1 && dense_blocks(p->grid.N[0], p->S, false) > 0;
+        p->dense = p->grid.nd == 1 && !p->own_plan && dense_blocks(p->grid.N[0], p->S, false) > 0;
         if (p->dense) {
             const std::vector<double> t = circulant_tables(kinetic_values(h), p->grid.N[0],
                                                            [](double T) { return (long double)T; });
@@ -1639,7 +1642,8 @@ static void gspo_create_impl(qdx_ham *const *ops, int32_t nops, double dt, int32
             else ++nx;
             if (o->time_dependent()) ++nfield;
         }
-        p->dense = !imag && p->grid.nd == 1 && nkin == 1 && p->ops[0]->terms[0].kind == T_KIN && nx <= kMaxXOps &&
+        p->own_plan = p->ctx->plan_set(p->grid, precision == QDX_FP32_BULK);
+        p->dense = !imag && p->grid.nd == 1 && !p->own_plan && nkin == 1 && p->ops[0]->terms[0].kind == T_KIN && nx <= kMaxXOps &&
                    nfield <= 1 && dense_blocks(p->grid.N[0], p->S, true) > 0;
         if (p->dense) {
             const auto T = kinetic_values(p->ops[0]);
@@ -2359,6 +2363,7 @@ static void krylov_create(qdx_ham *h, double dt, int32_t order, double err, int3
         }
         // reduction partials of qdx_prop_run's observables
         p->partials.alloc(kMaxPartials * sizeof(double));
+        p->own_plan = p->ctx->plan_set(p->grid, false);
         p->sil_grid = !arnoldi && order <= kSilMost && grid_fits(p.get());
         if (p->sil_grid) {
             grid_buffers(p.get(), 16);

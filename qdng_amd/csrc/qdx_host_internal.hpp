@@ -14,6 +14,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <set>
 #include <tuple>
 #include <memory>
 #include <stdexcept>
@@ -285,6 +286,15 @@ struct qdx_ctx {
     std::map<int, std::unique_ptr<DevBuf>> tw64, tw32;
     // radix plans set (or tuned) per line length and precision (fp32 flag)
     std::map<std::pair<int, bool>, std::vector<int>> radix;
+    // those set by the caller: propagators created afterwards run them, in place
+    // of kernels with a factorisation of their own (qdx_dense.hip, qdx_grid.hip,
+    // the line filter)
+    std::set<std::pair<int, bool>> own_plans;
+    bool plan_set(const Grid &g, bool fp32) const {
+        for (int d = 0; d < g.nd; ++d)
+            if (own_plans.count({g.N[d], fp32})) return true;
+        return false;
+    }
     DevBuf partials;   // reduction scratch
     DevBuf scal;       // small device result area
     DevBuf wfx, ktab;  // scratch of the momentum expectation (a transformed copy, k table)
@@ -957,6 +967,7 @@ struct qdx_prop {
     double dt = 0;
     Grid grid;
     int S = 1;
+    bool own_plan = false;   // the caller had set a radix plan for one of its lengths
     // Chebyshev
     qdx_ham *ham = nullptr;
     ChebyParams cp;

@@ -283,9 +283,10 @@ struct Launch {
     // first pass of an order also evaluates the break test of the previous
     // order and records its outcome in ctl (done, accnorm), which the row
     // kernel of the order then only reads
+    // filter: the in-place line filter where it suits, else the plan's stages.
     static void kin_pass(hipStream_t s, const GridDev &g, int S, int dim, bool accumulate,
                          const LinePlan &p, const HamDev<R> &h, const R *src, R *Y,
-                         ChebyCtl *ctl, const ConvCheck &cc, bool cmp = false);
+                         ChebyCtl *ctl, const ConvCheck &cc, bool cmp, bool filter);
     // dst = H src (both complex128) through the same kernels; X scratch
     static void ham_apply(hipStream_t s, const GridDev &g, const HamDev<R> &h,
                           const LinePlan *plans, const double *src, double *dst, R *X);

@@ -285,7 +285,8 @@ void Launch<R>::col_pass(hipStream_t s, const GridDev &g, int S, int dim, int mo
 // share a CU.  128^3 points: FP64 (67 MB) 32.7 -> 24.0 us, compact terms (42
 // MB) 20.5 -> 17.6.  Mode 5 stays with k_col: its larger stride and third
 // stream bound it elsewhere (36.5 against 37.6 us here, compact 24.6 against
-// 28.6).
+// 28.6).  FP32: the same on 128^3 points (14.5 against 14.6 us), ahead on others (a
+// whole step on 64^3 points 1.03 -> 0.98 ms).
 template <class R, bool CMP>
 __global__ void __launch_bounds__(256, 3) k_kin_filter(GridDev g, int S, int dim, int W, LinePlan p, int R2, int R3,
                                                        HamDev<R> h, cx<R> *__restrict__ Y,
@@ -406,8 +407,9 @@ static void kin_pass_P(hipStream_t s, const GridDev &g, int S, int dim, bool acc
 
 template <class R>
 void Launch<R>::kin_pass(hipStream_t s, const GridDev &g, int S, int dim, bool accumulate, const LinePlan &plan,
-                         const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp) {
-    if (!accumulate && kin_filter<R>(s, g, S, dim, plan, h, src, Y, ctl, cc, cmp)) return;
+                         const HamDev<R> &h, const R *src, R *Y, ChebyCtl *ctl, const ConvCheck &cc, bool cmp,
+                         bool filter) {
+    if (filter && !accumulate && kin_filter<R>(s, g, S, dim, plan, h, src, Y, ctl, cc, cmp)) return;
     const bool gen = plan.odd_prime();
     if (plan.ppt == 4 && gen) kin_pass_P<R, 4, true>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
     else if (plan.ppt == 4) kin_pass_P<R, 4, false>(s, g, S, dim, accumulate, plan, h, src, Y, ctl, cc, cmp);
@@ -475,7 +477,8 @@ void Launch<R>::line_fft(hipStream_t s, const GridDev &g, int S, int dim, const 
                                       const HamDev<R> &, double, R *, ChebyCtl *, const ConvCheck &, int,           \
                                       const double *);                                                              \
     template void Launch<R>::kin_pass(hipStream_t, const GridDev &, int, int, bool, const LinePlan &,              \
-                                      const HamDev<R> &, const R *, R *, ChebyCtl *, const ConvCheck &, bool);      \
+                                      const HamDev<R> &, const R *, R *, ChebyCtl *, const ConvCheck &, bool,       \
+                                      bool);                                                                       \
     template void Launch<R>::ham_apply(hipStream_t, const GridDev &, const HamDev<R> &, const LinePlan *,          \
                                        const double *, double *, R *);                                              \
     template void Launch<R>::line_fft(hipStream_t, const GridDev &, int, int, const LinePlan &, const double *, R *);

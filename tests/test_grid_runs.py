@@ -204,6 +204,55 @@ def test_lanczos(N0, N1, S, order, imag):
     check(both(make, 2, False), 1e-10)
 
 
+@pytest.mark.parametrize("N,kind,precision", [(N, k, q) for N, k in [
+    ([64, 24], "cheby"), ([64, 24], "gspo"), ([64, 24], "sil"), ([128], "cheby"), ([128], "gspo"), ([16, 64, 16], "cheby")]
+    for q in (("fp64",) if k == "sil" else ("fp64", "fp32"))])
+def test_a_set_plan_is_used(N, kind, precision):
+    """A radix plan that the caller set for a side selects the kernels that
+    transform by plans, as 4 or 8 line points do: here the same kernels, so the
+    same bits.  One the batch's tuning installs does not."""
+    import qdng_amd as Q
+    print("[gpu case] set plan", N, kind, precision, flush=True)
+
+    def run(plan, points):
+        c = Q.Context(0)
+        try:
+            c.set_line_points(points)
+            if plan:
+                c.set_radix_plan(64 if 64 in N else 128, plan, precision)
+            p = cases.Problem(N, [-6.0] * len(N), [6.0] * len(N))
+            x = p.axes()
+            r2 = sum(a ** 2 for a in x)
+            p.kinetic(0, [1500.0] * len(N))
+            p.potential(0, 0, np.minimum(0.03 * r2, 1.0))
+            p.psi0 = cases.normalized(p, np.exp(-r2 + 0.5j * x[0]))
+            if kind == "gspo":
+                U = Q.GSPO([p.gpu_split_op(c, [k]) for k in ("kin", "pot")], 1.0, precision=precision)
+            else:
+                H = p.gpu_ham(c)
+                lo, hi = H.bounds()
+                U = Q.SIL(H, 2.0 / (hi - lo)) if kind == "sil" else \
+                    Q.Cheby(H, 20.0 / (hi - lo), prec=1e-10, precision=precision)
+            w = p.gpu_wf(c)
+            U.run(w, 0, 2)
+            launches = c.persistent_stats()[0]
+            out = w.download()
+            del U, w
+            return out, launches
+        finally:
+            c.close()
+
+    plan = [4, 4, 4] if 64 in N else [4, 8, 4]
+    points = 8 if len(N) == 1 and kind == "gspo" else 4
+    a, na = run(plan, 0)
+    b, nb = run(plan, points)
+    d, nd = run(None, 0)
+    assert na == nb == 0
+    assert nd > 0 or len(N) != 2
+    assert np.array_equal(a, b)
+    assert not np.array_equal(a, d) and rel(a, d) < (1e-11 if precision == "fp64" else 1e-5)
+
+
 def propagator(c, kind, precision="fp64", nt=12):
     """(problem, propagator) on 40 x 24 points, a few orders per step"""
     import qdng_amd as Q
