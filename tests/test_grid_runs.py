@@ -204,6 +204,41 @@ def test_lanczos(N0, N1, S, order, imag):
     check(both(make, 2, False), 1e-10)
 
 
+# every radix of the line filter's two stages that the shapes above leave out
+# (R2 5, 7, 9, 13 to 17, 19, 23; R3 9, 14, 15), along either dimension
+RADICES = [(160, 72), (168, 112), (144, 120), (336, 16), (600, 16), (16, 1024), (136, 184), (152, 208)]
+
+
+@pytest.mark.parametrize("N0,N1", [s for n in RADICES for s in (n, n[::-1])])
+@pytest.mark.parametrize("kind", ["cheby", "gspo"])
+def test_against_the_oracle(N0, N1, kind):
+    """The oracle's bounds of the other propagator tests."""
+    import qdng_amd as Q
+    from oracle import oracle as O
+    print("[gpu case] grid oracle", N0, N1, kind, flush=True)
+    c = Q.Context(0)
+    try:
+        p = box(N0, N1, 1, True)
+        w, psi = p.gpu_wf(c), p.psi0.copy()
+        if kind == "cheby":
+            lo, hi = p.gpu_ham(c).bounds()
+            dt = 20.0 / (hi - lo)
+            _, _, nh, _ = Q.Cheby(p.gpu_ham(c), dt, prec=1e-12).run(w, 0, 3)
+            U = O.Cheby(p.oracle_ham(), dt, prec=1e-12)
+            assert list(nh) == [U.step(psi, i) for i in range(3)]
+        else:
+            kinds = ("kin", "pot", "dip")
+            Q.GSPO([p.gpu_split_op(c, [k]) for k in kinds], 2.0).run(w, 0, 3)
+            U = O.GSPO([p.oracle_split_op([k]) for k in kinds], 2.0, 1)
+            for i in range(3):
+                U.step(psi, i)
+        assert c.persistent_stats() == (1, 0)
+        assert rel(w.download(), psi) < (1e-10 if kind == "cheby" else 1e-12)
+        del w
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("N,kind,precision", [(N, k, q) for N, k in [
     ([64, 24], "cheby"), ([64, 24], "gspo"), ([64, 24], "sil"), ([128], "cheby"), ([128], "gspo"), ([16, 64, 16], "cheby")]
     for q in (("fp64",) if k == "sil" else ("fp64", "fp32"))])
