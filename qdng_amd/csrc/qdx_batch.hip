@@ -66,7 +66,15 @@ __global__ void __launch_bounds__(NT) k_brow(const BJob<R> *__restrict__ jobs, c
     const BJob<R> J = jobs[t.job];
     const int step = *tick_p - J.start_tick;
     if (step < 0 || step >= J.nsteps || J.ctl->failed) return;
-    if (PHASE == 2 && (k >= J.order || J.ctl->done)) return;
+    if (PHASE == 2) {
+        // done: the order whose launch found the series converged.  This one may
+        // be finding it now: block 0 records it while others start, and a block
+        // of which some waves left here would go on with a sum that nobody
+        // formed.  So only earlier orders end it here; this one's blocks all
+        // reach the test below.
+        const int dn = J.ctl->done;
+        if (k >= J.order || (dn > 0 && dn < k)) return;
+    }
     extern __shared__ __align__(16) char smem_raw[];
     __shared__ double red[16];
     BRowTile<R, LB> B(J, t.first, reinterpret_cast<cx<R> *>(smem_raw));
@@ -128,7 +136,7 @@ __global__ void __launch_bounds__(NT) k_brow(const BJob<R> *__restrict__ jobs, c
         double acc_prev;
         if (prev_converged(cc, red, &acc_prev)) {
             if (t.first == 0 && threadIdx.x == 0) {
-                J.ctl->done = 1;
+                J.ctl->done = k;
                 J.ctl->accnorm = acc_prev;
             }
             return;

@@ -432,3 +432,23 @@ def test_restart_from_snapshot_is_bit_identical(ctx, precision):
         assert np.array_equal(C.fetch(j), a)
     with pytest.raises(Q.QdxError):
         C.submit(jobs[0].gpu_ham(None), 1.0, steps, jobs[0].psi0, first_step=steps)   # beyond the laser
+
+
+def test_converged_orders_end_for_whole_blocks(ctx):
+    """The same jobs give the same bits in every batch: the launch that finds a
+    series converged ends it for all waves of a block (some of them went on,
+    in about 1 % of the largest jobs)."""
+    import qdng_amd as Q
+    note("64 jobs of 384 x 384 points, five batches")
+    rng = np.random.default_rng(91)
+    jobs = [cases.driven_job([384, 384], rng, 4) for _ in range(64)]
+    ref = None
+    for _ in range(5):
+        B = Q.Batch(ctx, "fp64", 2 << 30)
+        ids = [B.submit(p.gpu_ham(None), 1.0, 4, p.psi0) for p in jobs]
+        B.run(2)
+        got = [B.fetch(j) for j in ids]
+        del B
+        if ref is None:
+            ref = got
+        assert [i for i in range(64) if not np.array_equal(got[i], ref[i])] == []
