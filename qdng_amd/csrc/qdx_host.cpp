@@ -74,7 +74,7 @@ void cheby_step(qdx_prop *p, qdx_wf *psi, long step) {
         const int N0 = p->grid.N[0];
         const int lp = (ctx->line_ppt == 8 || N0 > 1024) ? 8 : 4;
         const LinePlan lplan = lp == 8 ? plans[0] : ctx->plan_ppt(N0, fp32, 4);
-        Launch<R>::cheby_line(s, g, h, lplan, p->coefd.as<double>(), p->k_launch, p->cp.offset, p->cp.offset_i,
+        Launch<R>::cheby_line(s, g, h, lplan, p->coef(), p->k_launch, p->cp.offset, p->cp.offset_i,
                               1.0 / p->cp.scaling, p->cp.prec, psi->ptr(), ctl, p->partials.as<double>());
         p->last_nb = 1;
         p->nb_init = 1;
@@ -181,7 +181,7 @@ std::vector<SplitOp> gspo_sequence(qdx_prop *p) {
 
 // exp(-i tau T_d(k)) for every state and dimension of a kinetic split
 // operator (layout of k_col's ek: state-major, dimensions in order, (re, im)
-// pairs), from the operator's own device tables T_d; a state without a
+// pairs), from the operator's own tables T_d; a state without a
 // kinetic term gets 1.  Built once per (operator, tau).
 const double *kinetic_exp_table(qdx_prop *p, qdx_ham *op, double tau) {
     const auto key = std::make_pair((const qdx_ham *)op, tau);
@@ -191,16 +191,13 @@ const double *kinetic_exp_table(qdx_prop *p, qdx_ham *op, double tau) {
     long tot = 0;
     for (int d = 0; d < g.nd; ++d) tot += g.N[d];
     std::vector<double> e(2 * (size_t)op->S * tot);
-    const HamDev<double> &h = op->dev.h64;
-    std::vector<double> t;
     for (int s = 0; s < op->S; ++s) {
         long off = 0;
         for (int d = 0; d < g.nd; ++d) {
-            t.assign(g.N[d], 0.0);
-            if (h.tk[s][0]) HIPCHK(hipMemcpy(t.data(), h.tk[s][d], g.N[d] * sizeof(double), hipMemcpyDeviceToHost));
+            const double *t = op->kin_table(s, d);
             for (int k = 0; k < g.N[d]; ++k) {
-                e[2 * (s * tot + off + k)] = std::cos(tau * t[k]);
-                e[2 * (s * tot + off + k) + 1] = -std::sin(tau * t[k]);
+                e[2 * (s * tot + off + k)] = t ? std::cos(tau * t[k]) : 1.0;
+                e[2 * (s * tot + off + k) + 1] = t ? -std::sin(tau * t[k]) : 0.0;
             }
             off += g.N[d];
         }
@@ -411,44 +408,75 @@ void gspo_run_fused(qdx_prop *p, R *psi, const R *psi0, long first, long nsteps,
 // qdx_ctx_set_line_points 4 or 8 asks for the line-transform kernels
 bool dense_on(const qdx_prop *p) { return p->dense && p->ctx->line_ppt == 0; }
 
-// The circulant matrix t(i - j) = 1/N sum_k f(T_k) cos(2 pi k (i - j) / N) of
-// f(T) for every state (T_k = T_{N-k}, f real), as the dense kernels read it:
-// per state and parity (t(d) +- t(d + N/2)) / 2 for d < N.  Summed in
-// extended precision; a state without a kinetic term has f(0).
-std::vector<double> circulant_tables(const std::vector<std::vector<double>> &Tk, int N,
-                                     const std::function<long double(double)> &f) {
-    std::vector<long double> cs(N), w(N / 2 + 1), t(N);
-    for (int q = 0; q < N; ++q) cs[q] = cosl(2.0L * 3.14159265358979323846264338327950288L * q / N);
-    std::vector<double> tab;
-    for (const std::vector<double> &T : Tk) {
-        for (int k = 0; k <= N / 2; ++k) w[k] = f(T[k]) * (k == 0 || k == N / 2 ? 1.0L : 2.0L) / N;
-        for (int d = 0; d <= N / 2; ++d) {
-            long double a = 0;
-            for (int k = 0, q = 0; k <= N / 2; ++k) {
-                a += w[k] * cs[q];
-                q += d;
-                if (q >= N) q -= N;
+// Sums over k <= N/2 of w_k cos(2 pi k d / N): the even k's part e and the odd
+// k's part o for d <= N/2.  cs: cos(2 pi q / (N stride)) at q.  The even part is
+// the same sum of half the length, and o(N/2 - d) = -o(d) leaves N/4 values of
+// it, whose terms k and N/2 - k differ by (-1)^d: N^2 / 24 products in all (512
+// points: 242 -> 73 us to create a propagator, against N^2 / 4 of them).
+void cosine_sums(const std::vector<long double> &w, int N, const std::vector<long double> &cs, int stride,
+                 std::vector<long double> &e, std::vector<long double> &o) {
+    const int M = N / 2, Q = N / 4, all = (int)cs.size();
+    e.assign(M + 1, 0.0L);
+    o.assign(M + 1, 0.0L);
+    if (N % 4) {
+        for (int d = 0; d <= M; ++d)
+            for (int k = 0, q = 0; k <= M; ++k) {
+                (k % 2 ? o : e)[d] += w[k] * cs[q];
+                q += d * stride;
+                if (q >= all) q -= all;
             }
-            t[d] = a;
-            if (d > 0) t[N - d] = a;
-        }
-        for (int par = 0; par < 2; ++par)
-            for (int d = 0; d < N; ++d) {
-                const long double u = t[(d + N / 2) % N];
-                tab.push_back((double)(0.5L * (par ? t[d] - u : t[d] + u)));
-            }
+        return;
     }
-    return tab;
+    std::vector<long double> w2(Q + 1), e2, o2, pair[2];
+    for (int j = 0; j <= Q; ++j) w2[j] = w[2 * j];
+    cosine_sums(w2, M, cs, 2 * stride, e2, o2);
+    for (int d = 0; d <= M; ++d) e[d] = d <= Q ? e2[d] + o2[d] : e2[M - d] + o2[M - d];
+    for (int k = 1; k <= Q; k += 2)
+        for (int s : {0, 1}) pair[s].push_back(k == M - k ? (s ? 0.0L : w[k]) : s ? w[k] - w[M - k] : w[k] + w[M - k]);
+    for (int d = 0; d <= Q; ++d) {
+        const std::vector<long double> &a = pair[d % 2];
+        const int step = 2 * d * stride % all;
+        long double t = 0;
+        int q = d * stride;
+        for (long double v : a) {
+            t += v * cs[q];
+            q += step;
+            if (q >= all) q -= all;
+        }
+        o[d] = t;
+        o[M - d] = -t;
+    }
 }
 
-// the per-state kinetic tables T_k of a 1D operator
-std::vector<std::vector<double>> kinetic_values(const qdx_ham *op) {
-    const int N = op->grid.N[0];
-    std::vector<std::vector<double>> T(op->S, std::vector<double>(N, 0.0));
-    for (int s = 0; s < op->S; ++s)
-        if (op->dev.h64.tk[s][0])
-            HIPCHK(hipMemcpy(T[s].data(), op->dev.h64.tk[s][0], N * sizeof(double), hipMemcpyDeviceToHost));
-    return T;
+// The circulant matrices t(i - j) = 1/N sum_k f(T_k) cos(2 pi k (i - j) / N) of
+// f(T) for every state (T_k = T_{N-k}; 0 without a kinetic term) of a 1D operator,
+// as the dense kernels read them, appended to tab: per state and parity (t(d) +-
+// t(d + N/2)) / 2 for d < N.  Summed in extended precision.
+void circulant_tables(const qdx_ham *op, const std::function<long double(double)> &f, std::vector<double> &tab) {
+    const int N = op->grid.N[0], M = N / 2;   // N: a multiple of 8
+    std::vector<long double> cs(N), w(M + 1), e, o;
+    for (int q = 0; q <= N / 8; ++q) {
+        const long double a = 2.0L * 3.14159265358979323846264338327950288L * q / N;
+        const long double c = cosl(a), s = sinl(a);
+        for (int p : {q, N - q}) cs[p % N] = c;
+        for (int p : {M - q, M + q}) cs[p] = -c;
+        for (int p : {N / 4 - q, 3 * N / 4 + q}) cs[p] = s;
+        for (int p : {N / 4 + q, 3 * N / 4 - q}) cs[p] = -s;
+    }
+    const std::vector<double> none(N, 0.0);
+    auto T = [&](int s) { return op->kin_table(s, 0) ? op->kin_table(s, 0) : none.data(); };
+    for (int s = 0; s < op->S; ++s) {
+        if (s > 0 && std::equal(T(s), T(s) + M + 1, T(s - 1))) {   // states often share their masses
+            const size_t at = tab.size();
+            tab.resize(at + 2 * N);
+            std::copy_n(tab.data() + at - 2 * N, 2 * N, tab.data() + at);
+            continue;
+        }
+        for (int k = 0; k <= M; ++k) w[k] = f(T(s)[k]) * (k == 0 || k == M ? 1.0L : 2.0L) / N;
+        cosine_sums(w, N, cs, 1, e, o);
+        for (int d = 0; d < N; ++d) tab.push_back((double)e[d <= M ? d : N - d]);
+        for (int d = 0; d < N; ++d) tab.push_back((double)o[d <= M ? d : N - d]);
+    }
 }
 
 // host arrays that copies in flight on a stream still read
@@ -551,7 +579,7 @@ void dense_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *
         a.nsteps = (int)n;
         if (cheby) {
             KTimer t(ctx, QDX_K_CHEBY_ROW);
-            launch_dense_cheby(ctx->stream, S, p->ham->dev.h64, a, p->dtab.as<double>(), p->coefd.as<double>(),
+            launch_dense_cheby(ctx->stream, S, p->ham->dev.h64, a, p->dtab.as<double>(), p->coef(),
                                p->k_launch, p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec, p->imag,
                                psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
             p->last_nb = 1;
@@ -624,9 +652,9 @@ GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const doubl
 // blocks (psi is unchanged then).
 bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, double *obs) {
     hipStream_t s = p->ctx->stream;
-    launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->greport);
+    launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->ctx->report());
     HIPCHK(hipStreamSynchronize(s));
-    if (*p->greport) {
+    if (*p->ctx->report()) {
         grid_missed(p);
         return false;
     }
@@ -741,7 +769,7 @@ long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *p
         const GridCus cus(p);
         if (cheby) {
             KTimer t(ctx, QDX_K_CHEBY_ROW);
-            launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), p->gs, a, p0, p1, p->coefd.as<double>(),
+            launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), p->gs, a, p0, p1, p->coef(),
                                        p->k_launch, p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec,
                                        p->imag, psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
         } else {
@@ -773,7 +801,6 @@ void grid_buffers(qdx_prop *p, size_t es) {
     p->X.alloc(nval * 16);
     p->gflags.alloc(kGridSyncBytes + sizeof(int));
     HIPCHK(hipMemset(p->gflags.p, 0, p->gflags.bytes));
-    HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&p->greport), sizeof(int), hipHostMallocDefault));
 }
 
 // the block shape of a 2D grid on this device; false: it takes the per-order
@@ -908,7 +935,7 @@ int qdx_ctx_create(int device, qdx_ctx **out) {
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         c->partials.alloc(kMaxPartials * sizeof(double));
         c->scal.alloc(4096 * sizeof(double));
-        HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&c->pinned), 4096 * sizeof(double), hipHostMallocDefault));
+        HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&c->pinned), qdx_ctx::kPinned * sizeof(double), hipHostMallocDefault));
         *out = c.release();
     });
 }
@@ -1520,25 +1547,22 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
                        p->grid.N[0] <= (precision == QDX_FP32_BULK ? kMaxLine : 2048) &&
                        line_lds <= 160 * 1024;
         p->dense = p->grid.nd == 1 && !p->own_plan && dense_blocks(p->grid.N[0], p->S, false) > 0;
-        if (p->dense) {
-            const std::vector<double> t = circulant_tables(kinetic_values(h), p->grid.N[0],
-                                                           [](double T) { return (long double)T; });
-            p->dtab.alloc(t.size() * sizeof(double));
-            HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-        }
+        std::vector<double> up;   // the dense tables, then the coefficients
+        if (p->dense) circulant_tables(h, [](double T) { return (long double)T; }, up);
         if (p->line_step || p->dense || p->grid2d) {
             // the same products as the per-order scalars of cheby_step
             const std::complex<double> ph =
                 imag ? std::complex<double>(std::exp(-dt * p->cp.offset), 0.0)
                      : std::exp(std::complex<double>(0, -1) * dt * std::complex<double>(p->cp.offset, p->cp.offset_i));
-            std::vector<double> c(2 * (size_t)std::max(p->k_launch, 1));
+            p->ncoef0 = up.size();
+            up.resize(up.size() + 2 * (size_t)std::max(p->k_launch, 1));
             for (int k = 0; k < p->k_launch; ++k) {
                 const std::complex<double> v = p->cp.coeff[k] * ph;
-                c[2 * k] = v.real();
-                c[2 * k + 1] = v.imag();
+                up[p->ncoef0 + 2 * k] = v.real();
+                up[p->ncoef0 + 2 * k + 1] = v.imag();
             }
-            p->coefd.alloc(c.size() * sizeof(double));
-            HIPCHK(hipMemcpy(p->coefd.p, c.data(), c.size() * sizeof(double), hipMemcpyHostToDevice));
+            p->dtab.alloc(up.size() * sizeof(double));
+            HIPCHK(hipMemcpy(p->dtab.p, up.data(), up.size() * sizeof(double), hipMemcpyHostToDevice));
         }
         HIPCHK(hipDeviceSynchronize());
         ctx_acquire(p->ctx);
@@ -1646,11 +1670,12 @@ static void gspo_create_impl(qdx_ham *const *ops, int32_t nops, double dt, int32
         p->dense = !imag && p->grid.nd == 1 && !p->own_plan && nkin == 1 && p->ops[0]->terms[0].kind == T_KIN && nx <= kMaxXOps &&
                    nfield <= 1 && dense_blocks(p->grid.N[0], p->S, true) > 0;
         if (p->dense) {
-            const auto T = kinetic_values(p->ops[0]);
-            const int N = p->grid.N[0];
-            std::vector<double> t = circulant_tables(T, N, [&](double v) { return cosl((long double)dt * v); });
-            const std::vector<double> ti = circulant_tables(T, N, [&](double v) { return -sinl((long double)dt * v); });
-            t.insert(t.end(), ti.begin(), ti.end());
+            // (the factors in extended precision as well: runs of 300 steps on 128
+            // points end 0.8 to 1.7e-14 from the exact product, with factors
+            // rounded to FP64 1.3 to 3.2e-14)
+            std::vector<double> t;
+            circulant_tables(p->ops[0], [&](double v) { return cosl((long double)dt * v); }, t);
+            circulant_tables(p->ops[0], [&](double v) { return -sinl((long double)dt * v); }, t);
             p->dtab.alloc(t.size() * sizeof(double));
             HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         }
@@ -2448,11 +2473,11 @@ bool sil_grid_basis(qdx_prop *p, qdx_wf *psi, long step, std::vector<double> &al
         const GridCus cus(p);
         launch_sil_grid(s, p->S, h, p->gs, a, ctx->plan_ppt(p->grid.N[0], false, 4),
                         ctx->plan_ppt(p->grid.N[1], false, 4), qv, order, p->dt, p->sil_err, psi->grid.weight(),
-                        psi->ptr(), p->partials.as<double>(), p->greport);
+                        psi->ptr(), p->partials.as<double>(), p->ctx->report());
         HIPCHK(hipMemcpyAsync(res.data(), p->partials.p, nres * sizeof(double), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
     }
-    if (*p->greport) {
+    if (*p->ctx->report()) {
         grid_missed(p);
         return false;
     }

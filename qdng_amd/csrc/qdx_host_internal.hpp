@@ -298,7 +298,10 @@ struct qdx_ctx {
     DevBuf partials;   // reduction scratch
     DevBuf scal;       // small device result area
     DevBuf wfx, ktab;  // scratch of the momentum expectation (a transformed copy, k table)
-    double *pinned = nullptr;
+    double *pinned = nullptr;   // kPinned values
+    static constexpr int kPinned = 4096;
+    // status of the last persistent launch: the last of them
+    int *report() const { return reinterpret_cast<int *>(pinned + kPinned - 1); }
 
     // per-launch HIP-event timing (qdx_ctx_profile): a fixed pool of events;
     // when it is used up the recorded spans are folded into the totals
@@ -651,6 +654,12 @@ struct qdx_ham {
     // upload the applied matrix: W_ij = sum of potentials, mu_ij one dipole,
     // kinetic tables per state and dimension (Kspace.cpp:22-50)
     std::vector<std::vector<double>> hostW, hostMu, hostWi;
+    std::vector<double> host_tk;
+    std::vector<long> tk_off;   // of [state][dimension] in host_tk, -1: none
+    // T_d(k) of a state, null without a kinetic term
+    const double *kin_table(int s, int d) const {
+        return dev.h64.tk[s][0] ? host_tk.data() + tk_off[s * kMaxDims + d] : nullptr;
+    }
     void upload() {
         if (!ctx) return;
         const long n = grid.size();
@@ -661,8 +670,9 @@ struct qdx_ham {
         hostW.assign(S * S, {});
         hostMu.assign(S * S, {});
         hostWi.assign(S, {});
-        std::vector<double> tkh;
-        std::vector<long> tk_off(S * kMaxDims, -1);
+        std::vector<double> &tkh = host_tk;
+        tkh.clear();
+        tk_off.assign(S * kMaxDims, -1);
         for (int i = 0; i < S; ++i) {
             h.unity[i] = 0;
             for (int j = 0; j < S; ++j) {
@@ -979,12 +989,13 @@ struct qdx_prop {
     // single-state 1D lines: the whole step in one block (k_cheby_line) with
     // the phased coefficients coeff[k] exp(-i offset dt) on the device
     bool line_step = false;
-    DevBuf coefd;
     // short 1D lines (any states): whole runs in one block with the kinetic
     // operator as a dense circulant matrix (qdx_dense.hip); dtab holds its
-    // tables (GSPO: real part, then imaginary part)
+    // tables (GSPO: real part, then imaginary part), then the coefficients
     bool dense = false;
     DevBuf dtab, dfields;
+    size_t ncoef0 = 0;
+    const double *coef() const { return dtab.as<double>() + ncoef0; }
     // 2D grids that fit the chip's registers (Chebyshev, split operator): whole
     // runs in one launch (qdx_grid.hip); gepoch: the flags' values so far
     bool grid2d = false;
@@ -997,7 +1008,6 @@ struct qdx_prop {
     int gmiss = 0;
     long gskip = 0;
     bool sil_grid = false;    // the Lanczos basis by the persistent kernel
-    int *greport = nullptr;   // host memory: status of the last launch
     int last_nb = 0, nb_init = 0;   // partial counts of the last Chebyshev step
     // SIL (Lanczos vectors and a buffer as device wave functions; `imag`
     // above selects imaginary time)
@@ -1019,7 +1029,5 @@ struct qdx_prop {
     DevBuf psi32, psi0_32;
     DevBuf obs;   // device observables of qdx_prop_run
 
-    virtual ~qdx_prop() {
-        if (greport) (void)hipHostFree(greport);
-    }
+    virtual ~qdx_prop() = default;
 };
