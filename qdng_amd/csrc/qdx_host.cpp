@@ -2225,7 +2225,7 @@ int qdx_eigen_imag(qdx_prop *U, qdx_ham *Hin, const qdx_wf *psi0, int32_t nef, i
             double dff = 1;
             while (s < max_steps && dff > conv) {
                 chk(qdx_wf_copy(psi_old, psi));
-                prop_step(U, psi, s, psi_in_fp32(U));
+                prop_step(U, psi, s, false);
                 if (i > 0) {   // OProjection::Apply (OProjection.cpp:133-149), psi -= P psi
                     std::vector<std::complex<double>> c(i);
                     for (int j = 0; j < i; ++j) ovl(ef[j], psi, c[j]);
@@ -2279,7 +2279,7 @@ int qdx_eigen_ac(qdx_prop *U, qdx_ham *Hin, const qdx_wf *psi0, int32_t nsteps, 
         qdx_wf *psi = tmp.make(p0);
         chk(qdx_wf_copy(psi, p0));
         for (int i = 1; i < N; ++i) {
-            prop_step(U, psi, i - 1, psi_in_fp32(U));
+            prop_step(U, psi, i - 1, false);
             ovl(psi, p0, ac[i]);
             if (std::isnan(ac[i].real())) fail(QDX_ERR_OVERFLOW, "Correlation is not a number");
         }
@@ -2315,7 +2315,7 @@ int qdx_eigen_ac(qdx_prop *U, qdx_ham *Hin, const qdx_wf *psi0, int32_t nsteps, 
         U->arn_order = arn_order0;
         chk(qdx_wf_copy(psi, p0));
         for (int s = 1; s < N; ++s) {
-            prop_step(U, psi, s - 1, psi_in_fp32(U));
+            prop_step(U, psi, s - 1, false);
             for (int k = 0; k < n_ef; ++k) {
                 const double ph = ek[k] * double(s) * dt;
                 chk(qdx_wf_axpy(ef[k], std::cos(ph), std::sin(ph), psi));

@@ -12,6 +12,7 @@ oracle on the same input: the same peaks and autocorrelation and energies to
 import numpy as np
 import pytest
 
+import cases
 from oracle import oracle as O
 import test_imag_time as T
 
@@ -124,3 +125,25 @@ def test_device_ac_variants_match_oracle(ctx, nsteps, win, width, tol):
     assert len(efs) == len(pk), (len(efs), pk)
     assert np.allclose(ac, ac_o, rtol=0, atol=1e-10)
     assert np.allclose(er, e_o, rtol=1e-10, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [[128], [512], [40, 24], [16, 24, 16]])
+def test_fp32_split_operator_record(ctx, N):
+    """The record of an FP32 split-operator propagation is the run's
+    autocorrelation, whichever kernels it takes: both round psi to 2^-24 a few
+    times per step, 1e-5 bounds 24 steps."""
+    import qdng_amd as Q
+    print("[gpu case] eigen ac FP32 split operator", N, flush=True)
+    p = cases.Problem(N, [-6.0] * len(N), [6.0] * len(N))
+    x = p.axes()
+    r2 = sum(a ** 2 for a in x)
+    p.kinetic(0, [1500.0] * len(N))
+    p.potential(0, 0, np.minimum(0.03 * r2, 1.0))
+    p.psi0 = cases.normalized(p, np.exp(-r2 + 1.5j * x[0]))
+    G = Q.GSPO([p.gpu_split_op(ctx, [k]) for k in ("kin", "pot")], 10.0, precision="fp32")
+    w, w0 = p.gpu_wf(ctx), p.gpu_wf(ctx)
+    _, want, _, _ = G.run(w, 0, 24, w0)
+    assert np.min(np.abs(want)) < 0.9
+    _, _, _, ac = Q.eigen_ac(G, w0, 24, win=False, H=p.gpu_ham(ctx))
+    assert np.max(np.abs(ac - want)) < 1e-5
