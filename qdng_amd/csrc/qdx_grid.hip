@@ -525,6 +525,39 @@ __global__ void __launch_bounds__(256) k_gspo_grid(GridRun a, GridShape g, XGrou
             }
             return;
         }
+        if constexpr (MU && !PRIMES) {
+            // a field and tables, operator by operator for the same reason (a
+            // single step on 512 x 512 points 59 -> 54 us, 64 x 64 49 -> 43; with
+            // PRIMES the registers do not suffice, 240 x 176 points 18 -> 22)
+            for (int o = 0; o < pre.n; ++o) {
+                XSplitDev<R> op = pre.op[o];
+                if (op.mu[0][0]) {
+                    R m[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) m[q] = op.mu[0][0][gi(q)];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) L.mu[q] = op.tau * (double)m[q];
+                    op.mu[0][0] = nullptr;   // the field part is formed per step
+                    if (!op.V[0][0]) continue;
+                }
+                if (op.U) {
+                    const cx<double> *U = reinterpret_cast<const cx<double> *>(op.U);
+                    cx<double> t[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) t[q] = U[gi(q)];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) L.u[q] = cmul(L.u[q], t[q]);
+                    continue;
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    cx<double> v[1] = {L.u[q]};
+                    xsplit_point<R, 1>(op, gi(q), v);
+                    L.u[q] = v[0];
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const long i = gi(q);
