@@ -47,8 +47,11 @@ HBM_PEAK_GBS = 8000.0
 B_ROW = {"fp64": (16 + 16 + 16 + 32 + 8 + 8), "fp32": (8 + 8 + 8 + 32 + 4 + 4),
          "compact": (10 + 10 + 10 + 32 + 8 + 8)}
 B_ROW_PRO = {"fp64": B_ROW["fp64"] - 16, "fp32": B_ROW["fp32"] - 8, "compact": B_ROW["compact"] - 10}
-# GSPO per step and grid point of one state: psi read and write + V
-B_GSPO = {"fp64": 32 + 8, "fp32": 16 + 4}
+# what the persistent 2D kernels exchange between CUs per grid point and state:
+# a term and its filtered line written and read per order (compact terms travel
+# as complex128), psi written and read once per split-operator step
+B_X_CHEBY = {"fp64": 64, "fp32": 32, "compact": 64}
+B_X_GSPO = {"fp64": 32, "fp32": 16}
 PRECISIONS = ("fp64", "compact", "fp32")
 
 
@@ -482,6 +485,7 @@ def precision_3d(ctx, steps=5):
         ref = None
         for prec in PRECISIONS:
             U = Q.Cheby(p.gpu_ham(ctx), dt, prec=1e-10, precision=prec)
+            U.run(p.gpu_wf(ctx), 0, 1, observables=False)   # loads the kernels
             w = p.gpu_wf(ctx)
             sync(ctx)
             t0 = time.perf_counter()
@@ -502,7 +506,7 @@ def precision_3d(ctx, steps=5):
             ach = rb / (msrow * 1e-3) / 1e9 if msrow > 0 else 0.0
             rec[prec] = {"value": npts * hpsi / t, "unit": UNIT, "ms_per_step": t * 1e3 / steps,
                          "hpsi_per_step": [int(nh.min()), int(nh.max())], "order": U.order,
-                         "roofline": {"bound": "hbm", "kernel": "k_cheby_grid", "achieved": ach,
+                         "roofline": {"bound": "hbm", "kernel": "k_cheby_row", "achieved": ach,
                                       "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                                       "avg_launch_us": msrow / max(nrow, 1) * 1e3}}
             if prec == "fp64":
@@ -567,6 +571,43 @@ def cheby_1d_small(ctx, steps=1000):
                     "holds the line): not judged on the roofline"}
 
 
+def grid_roofline(p, prec, kernel_ms, hpsi, launches):
+    """The persistent 2D Chebyshev kernel holds psi, the terms and the surfaces
+    in registers: what it moves is phi to the owners of the columns and the
+    filtered lines back, each written and read once per order.  It is bound by
+    the latency of the filters (LDS) and of that exchange."""
+    gbs = B_X_CHEBY[prec] * p.size * p.S * hpsi / (kernel_ms * 1e-3) / 1e9
+    return {"bound": "latency", "kernel": "k_cheby_grid", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": gbs / HBM_PEAK_GBS, "us_per_order": kernel_ms / hpsi * 1e3, "launches": launches,
+            # the rate a kernel per order would need, which reads and writes its operands in memory
+            "hbm_equivalent_frac": B_ROW[prec] * p.size * p.S * hpsi / (kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+            "bytes_model": f"{B_X_CHEBY[prec]} B per grid point and state exchanged per order"}
+
+
+def summary(out):
+    """The printed record: one short line.  --record writes the whole one."""
+    def short(x):
+        if isinstance(x, float):
+            return float(f"{x:.5g}")
+        return {k: short(v) for k, v in x.items()} if isinstance(x, dict) else x
+    line = {k: out[k] for k in out if k not in ("extra", "cpu_baseline")}
+    if "cpu_baseline" in out:
+        line["cpu_baseline"] = {k: out["cpu_baseline"].get(k) for k in ("value", "value_1_thread", "cores", "fft")}
+    ex = out.get("extra", {})
+    if "l2_fp64_vs_oracle" in ex:
+        line["l2_vs_oracle"] = ex["l2_fp64_vs_oracle"]
+    values = {}
+    for name, c in ex.get("configs", {}).items():
+        if name == "serving":   # [p50, p99] latency in s per arrival rate
+            values[name] = {lam: {p: [short(r["p50_latency_s"]), short(r["p99_latency_s"])] for p, r in recs.items()}
+                            for lam, recs in c["rates"].items()}
+            continue
+        values[name] = {p: r["value"] for p, r in c["precisions"].items()} if "precisions" in c else c.get("value")
+    if values:
+        line["values"] = values
+    return short(line)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -588,6 +629,8 @@ def main():
     ap.add_argument("--precision-3d-only", action="store_true",
                     help="only run the 3D 128^3 precision workload (FP64, compact, FP32 at dt 3.5 and 37) and print "
                          "its record: a short program for traces")
+    ap.add_argument("--record", metavar="FILE", help="write the whole record (every configuration, rooflines, "
+                    "schedules) to FILE; the printed line holds the headline and one value per configuration")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported (every box here has one GPU)",
@@ -634,10 +677,8 @@ def main():
     rp = run_cheby(ctx, p, "fp64", args.steps, args.warmup, profile=True)
     assert int(rp["n_hpsi"].sum()) == hpsi
     launches, row_ms = rp["row"]
-    row_bytes = p.size * p.S * (B_ROW["fp64"] * (hpsi - args.steps) + B_ROW_PRO["fp64"] * args.steps)
-    achieved = row_bytes / (row_ms * 1e-3) / 1e9
     log(f"fp64: {value:.4g} grid-pt*Hpsi/s, {r['seconds'] * 1e3 / args.steps:.3f} ms/step, "
-        f"orders/step {nh.min()}-{nh.max()}, row kernel {launches} launches avg {row_ms / launches * 1e3:.2f} us")
+        f"orders/step {nh.min()}-{nh.max()}, {launches} launches, {row_ms / hpsi * 1e3:.2f} us per order")
 
     out = {
         "metric": METRIC,
@@ -658,28 +699,7 @@ def main():
             "dt": 5.0, "prec": 1e-10, "order": r["order"],
             "hpsi_per_step": [int(nh.min()), int(nh.max())],
         },
-        "roofline": {
-            "bound": "hbm",
-            "achieved": achieved,
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS,
-            "traffic": None,
-            "traffic_note": "the kernel keeps psi, the terms and the surfaces in registers: what it moves is the "
-                            "exchange of phi and of the filtered lines, 64 B per point and state and order",
-            "kernel": "qdx::k_cheby_grid<double, 2, false, false, false>",
-            "points_per_thread": 8,
-            "launches": launches,
-            "avg_launch_us": row_ms / launches * 1e3,
-            "algorithmic_bytes_per_launch": row_bytes / launches,
-            "bytes_model": "96 B per grid point and state per executed order (80 B for order 1), the operands of "
-                           "an order that is a kernel of its own",
-            "measured": "HIP events attached to every launch (hipExtLaunchKernelGGL; one launch runs many steps) "
-                        "over a second timed pass of the same steps",
-            "ms_per_step_profiled_pass": rp["seconds"] * 1e3 / args.steps,
-            "step_frac": B_ROW["fp64"] * value / 1e9 / HBM_PEAK_GBS,
-            "step_frac_note": "the whole step at the same 96 B per grid point and state per executed order",
-        },
+        "roofline": grid_roofline(p, "fp64", row_ms, hpsi, launches),
     }
 
     # ---- parity against the oracle (its own FFT: the checker) over the first
@@ -727,16 +747,12 @@ def main():
             hh = int(rr["n_hpsi"].sum())
             rq = run_cheby(ctx, p, prec, args.steps, args.warmup, profile=True)
             ln, lms = rq["row"]
-            bb = p.size * p.S * (B_ROW[prec] * (hh - args.steps) + B_ROW_PRO[prec] * args.steps)
             v = npts * hh / rr["seconds"]
             rec2d["precisions"][prec] = {
                 "value": v, "unit": UNIT, "ms_per_step": rr["seconds"] * 1e3 / args.steps,
                 "hpsi_per_step": [int(rr["n_hpsi"].min()), int(rr["n_hpsi"].max())], "vs_fp64": v / value,
                 "l2_vs_oracle": ex.get("parity", {}).get(prec, {}).get("l2_vs_oracle"),
-                "roofline": {"bound": "hbm", "kernel": "k_cheby_grid", "achieved": bb / (lms * 1e-3) / 1e9,
-                             "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                             "frac": bb / (lms * 1e-3) / 1e9 / HBM_PEAK_GBS, "avg_launch_us": lms / ln * 1e3,
-                             "bytes_model": f"{B_ROW[prec]} B per grid point and state per executed order"}}
+                "roofline": grid_roofline(p, prec, lms, hh, ln)}
             log(f"{prec}: {v:.4g} grid-pt*Hpsi/s")
         configs["cheby_2d_512x512_2state"] = rec2d
         # GSPO on the same workload: at least 100 timed steps
@@ -746,12 +762,12 @@ def main():
         for prec in ("fp64", "fp32"):
             t, rowk, colk = run_gspo(ctx, p, prec, gsteps, min(args.warmup, 10), profile=True)
             v = npts * gsteps / t
-            eff = B_GSPO[prec] * v / 1e9
+            eff = B_X_GSPO[prec] * v / 1e9
             gs["precisions"][prec] = {
                 "value": v, "unit": "grid-pt*step/s", "ms_per_step": t * 1e3 / gsteps, "steps": gsteps,
-                "roofline": {"bound": "hbm", "kernel": "k_gspo_grid (whole runs)", "achieved": eff,
+                "roofline": {"bound": "latency", "kernel": "k_gspo_grid (whole runs)", "achieved": eff,
                              "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": eff / HBM_PEAK_GBS,
-                             "bytes_model": f"{B_GSPO[prec]} B per grid point and state per step"},
+                             "bytes_model": f"{B_X_GSPO[prec]} B per grid point and state exchanged per step"},
                 "kernel_us_per_step": (rowk[1] + colk[1]) / gsteps * 1e3, "launches": rowk[0] + colk[0]}
             log(f"gspo {prec}: {v:.4g} grid-pt*step/s, {t * 1e3 / gsteps:.4f} ms/step")
         gs["value"] = gs["precisions"]["fp64"]["value"]
@@ -765,7 +781,10 @@ def main():
             configs["serving"] = serving_extra(ctx, [float(x) for x in args.serve_rates.split(",")], args.serve_jobs)
         ex["configs"] = configs
         ex["cheby_1d_256_latency"] = cheby_1d_small(ctx)
-    print(json.dumps(out), flush=True)
+    if args.record:
+        with open(args.record, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(summary(out)), flush=True)
     ctx.close()
 
 
