@@ -499,12 +499,12 @@ int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points);
  * up to rounding).  Persistent launches of several threads of a process go side
  * by side as long as their blocks (one per line, at least 512 points each)
  * together are no more than the device's CUs, else one after the other.
- * set_wait_limit: after `skip` further launches on this context
- * the next `count` bound their waits by `us` microseconds instead (at most 10^6;
- * 0: they give up at the first wait, which serves to test callers).
+ * set_short_launches: after `skip` further launches on this context the next
+ * `count` come without their last block, as if other work held its CU, and give
+ * up after the bound (to test callers).
  * persistent_stats: launches so far and those that gave up (either may be
  * NULL).  No QDng counterpart (its propagators run on the host). */
-int qdx_ctx_set_wait_limit(qdx_ctx *ctx, int64_t us, int64_t skip, int64_t count);
+int qdx_ctx_set_short_launches(qdx_ctx *ctx, int64_t skip, int64_t count);
 int qdx_ctx_persistent_stats(qdx_ctx *ctx, int64_t *launches, int64_t *given_up);
 
 /* Tile shape of the batched kernels for 2D Chebyshev jobs of one grid

@@ -62,7 +62,7 @@ EXPORTS = [
     "qdx_ctx_set_radix_plan", "qdx_ctx_get_radix_plan", "qdx_batch_get_tiling", "qdx_batch_set_tiling",
     "qdx_batch_autotune", "qdx_batch_set_autotune", "qdx_batch_tuning_save", "qdx_batch_tuning_load",
     "qdx_batch_set_lds_schedule", "qdx_batch_get_lds_schedule", "qdx_batch_autotune_lds",
-    "qdx_ctx_set_line_points", "qdx_ctx_get_line_points", "qdx_ctx_set_wait_limit", "qdx_ctx_persistent_stats", "qdx_cheby_create_imag", "qdx_bessel_i0",
+    "qdx_ctx_set_line_points", "qdx_ctx_get_line_points", "qdx_ctx_set_short_launches", "qdx_ctx_persistent_stats", "qdx_cheby_create_imag", "qdx_bessel_i0",
     "qdx_wf_axpy", "qdx_wf_expec_position", "qdx_wf_expec_momentum", "qdx_eigen_imag", "qdx_eigen_ac", "qdx_sil_create", "qdx_gspo_create_imag", "qdx_arnoldi_create",
     # include/qdx_io.h
     "qdx_meta_create", "qdx_meta_read", "qdx_meta_write", "qdx_meta_size", "qdx_meta_key", "qdx_meta_get",
@@ -202,7 +202,7 @@ def lib():
         "qdx_eigen_imag": [vp, vp, vp, i32, i32, C.c_double, i32, C.POINTER(vp), dp, dp, C.POINTER(i32)],
         "qdx_eigen_ac": [vp, vp, vp, i32, i32, C.c_double, i32, i32, i32, C.POINTER(vp), dp, dp, C.POINTER(i32), dp],
         "qdx_ctx_get_line_points": [vp, C.POINTER(i32)],
-        "qdx_ctx_set_wait_limit": [vp, C.c_int64, C.c_int64, C.c_int64],
+        "qdx_ctx_set_short_launches": [vp, C.c_int64, C.c_int64],
         "qdx_ctx_persistent_stats": [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64)],
         "qdx_batch_get_tiling": [vp, i32, i32, C.POINTER(Tiling)],
         "qdx_batch_set_tiling": [vp, i32, i32, C.POINTER(Tiling)],
@@ -471,10 +471,10 @@ class Context:
         _chk(lib().qdx_ctx_get_line_points(self.h, C.byref(n)))
         return n.value
 
-    def set_wait_limit(self, us: int, skip: int = 0, count: int = 1) -> None:
-        """bound of the waits of `count` persistent launches, after `skip` others
-        (qdx_ctx_set_wait_limit)"""
-        _chk(lib().qdx_ctx_set_wait_limit(self.h, int(us), int(skip), int(count)))
+    def set_short_launches(self, skip: int = 0, count: int = 1) -> None:
+        """`count` persistent launches, after `skip` others, without their last
+        block: they give up (qdx_ctx_set_short_launches)"""
+        _chk(lib().qdx_ctx_set_short_launches(self.h, int(skip), int(count)))
 
     def persistent_stats(self):
         """(persistent launches, those that gave up waiting) so far"""

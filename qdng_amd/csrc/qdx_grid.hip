@@ -28,16 +28,20 @@
 //
 // All blocks have to be on the chip together: there are at most as many as
 // CUs, each fits a CU by itself, and the host lets no more such launches run at a
-// time, per device and process, than their blocks have CUs.  (Cooperative launches would say so to the
-// runtime, but they cost 20 us more, and once a process has made one its other
-// streams run slower: a batch of jobs 34 -> 45 ms.)  Other processes on the
-// GPU can still hold CUs, so every wait is bounded (GridRun::wait): a block that
+// time, per device and process, than their blocks have CUs.  (Cooperative
+// launches would say so to the runtime, but they cost 20 us more, and once a
+// process has made one its other streams run slower: a batch of jobs 34 -> 45
+// ms.)  Other processes on the
+// GPU can still hold CUs, so every wait is bounded (kGridWait): a block that
 // gives up leaves, the others follow, and the host, which keeps psi until the
 // launch is known to be complete, runs its steps again order by order.
 #include "qdx_gridfft.hpp"
 #include "qdx_xsplit.hpp"
 
 namespace qdx {
+
+// bound of one wait in ticks of the 100 MHz wall clock: 0.1 s
+constexpr unsigned long long kGridWait = 10000000ull;
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -100,11 +104,9 @@ __device__ __forceinline__ void grid_put(char *sync, int slot, double v, double 
 }
 
 // by wave 0: waits until the first n blocks' flags have reached epoch; false
-// after a.wait ticks of the 100 MHz wall clock, or at once when that is 0.  n <=
-// kGridBlocks.
-__device__ __forceinline__ bool grid_wait(const GridRun &a, int n, unsigned epoch) {
-    if (!a.wait) return false;
-    const unsigned *flags = grid_flags(a.sync, blockIdx.x % kGridCopies);
+// after kGridWait.  n <= kGridBlocks.
+__device__ __forceinline__ bool grid_wait(char *sync, int n, unsigned epoch) {
+    const unsigned *flags = grid_flags(sync, blockIdx.x % kGridCopies);
     const int lane = threadIdx.x & 63;
     unsigned long long t0 = 0;
     for (bool first = true;; first = false) {
@@ -119,7 +121,7 @@ __device__ __forceinline__ bool grid_wait(const GridRun &a, int n, unsigned epoc
         for (int i = 0; i < kGridBlocks / 64; ++i) good = good && (int)(f[i] - epoch) >= 0;
         if (__all(good)) break;
         if (first) t0 = wall_clock64();
-        else if (wall_clock64() - t0 > a.wait) return false;
+        else if (wall_clock64() - t0 > kGridWait) return false;
     }
     asm volatile("" ::: "memory");   // loads of the exchanged data stay behind
     return true;
@@ -351,7 +353,7 @@ __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamD
                 if (ph) break;
 #pragma unroll
                 for (int q = 0; q < 8; ++q) v[q] = x[q];
-                if (wave == 0 && !grid_wait(a, B.nrb, epoch) && tid == 0) bad = 1;
+                if (wave == 0 && !grid_wait(a.sync, B.nrb, epoch) && tid == 0) bad = 1;
                 lds_barrier();
                 if (bad) break;
 #pragma unroll
@@ -386,7 +388,7 @@ __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamD
             ++epoch;
             if (wave == 0) {
                 if (B.col) grid_signal(a.sync, epoch);
-                if (B.row && !grid_wait(a, B.ncb, epoch) && tid == 0) bad = 1;
+                if (B.row && !grid_wait(a.sync, B.ncb, epoch) && tid == 0) bad = 1;
             }
             lds_barrier();
             if (bad) {
@@ -666,7 +668,7 @@ __global__ void __launch_bounds__(256) k_gspo_grid(GridRun a, GridShape g, XGrou
         ++epoch;
         if (wave == 0) {
             if (cols ? B.col : B.row) grid_signal(a.sync, epoch);
-            if ((cols ? B.row : B.col) && !grid_wait(a, cols ? B.ncb : B.nrb, epoch) && tid == 0) bad = 1;
+            if ((cols ? B.row : B.col) && !grid_wait(a.sync, cols ? B.ncb : B.nrb, epoch) && tid == 0) bad = 1;
         }
         lds_barrier();
         if (bad) {
@@ -752,7 +754,7 @@ __global__ void __launch_bounds__(256) k_sil_grid(GridRun a, GridShape g, HamDev
                 grid_drain();
                 grid_signal(a.sync, epoch);
             }
-            if (!grid_wait(a, B.nrb, epoch)) {
+            if (!grid_wait(a.sync, B.nrb, epoch)) {
                 if (tid == 0) bad = 1;
             } else {
                 const double r = grid_sum(a.sync, slot, B.nrb);
@@ -794,7 +796,7 @@ __global__ void __launch_bounds__(256) k_sil_grid(GridRun a, GridShape g, HamDev
             if (ph) break;
 #pragma unroll
             for (int q = 0; q < 8; ++q) v[q] = x[q];
-            if (wave == 0 && !grid_wait(a, B.nrb, epoch) && tid == 0) bad = 1;
+            if (wave == 0 && !grid_wait(a.sync, B.nrb, epoch) && tid == 0) bad = 1;
             lds_barrier();
             if (bad) break;
 #pragma unroll
@@ -810,7 +812,7 @@ __global__ void __launch_bounds__(256) k_sil_grid(GridRun a, GridShape g, HamDev
         ++epoch;
         if (wave == 0) {
             if (B.col) grid_signal(a.sync, epoch);
-            if (B.row && !grid_wait(a, B.ncb, epoch) && tid == 0) bad = 1;
+            if (B.row && !grid_wait(a.sync, B.ncb, epoch) && tid == 0) bad = 1;
         }
         lds_barrier();
         if (bad) break;

@@ -527,7 +527,7 @@ long run_fields(qdx_prop *p, qdx_ham *fop, int nf, long first, long n, long most
 
 // Steps of one dense launch.  It holds a CU that a persistent launch of another
 // context may need all the while, so it ends well within that one's wait
-// (kGridWaitUs, 0.1 s): about 10 ms by the time an order or a split-operator step
+// (0.1 s): about 10 ms by the time an order or a split-operator step
 // takes (orders: 128 points 0.9 us, 512 points 3.6, 256 points and two states
 // 2.4; steps: 128 points 1.7 us, 384 points 4.0, 256 points and two coupled
 // states 6.1), a thousand times a launch's own cost.
@@ -601,15 +601,16 @@ bool grid_on(const qdx_prop *p) { return p->grid2d && p->ctx->line_ppt == 0; }
 // ... and so do launches that gave up again and again (grid_missed)
 bool grid_ready(const qdx_prop *p) { return grid_on(p) && p->gskip == 0; }
 
-// Usual bound of a wait: a launch whose blocks are all on the chip waits for
-// microseconds, one that shares the GPU for as long as the others' kernels run.
-constexpr int64_t kGridWaitUs = 100000;
-
-// the bound of the waits of the next persistent launch, in ticks of 10 ns
-unsigned grid_wait_ticks(qdx_ctx *c) {
-    const int64_t i = c->grid_launches++ - c->wait_first;
-    const bool set = i >= 0 && i < c->wait_count;
-    return (unsigned)(100 * (set ? c->wait_us : kGridWaitUs));
+// The blocks of the next persistent launch: all, or all but the last where the
+// caller wants launches that give up (*forced; also a launch that ends before
+// anyone would wait for that block counts as one).
+GridShape grid_launch_shape(qdx_prop *p, bool *forced) {
+    qdx_ctx *c = p->ctx;
+    const int64_t i = c->grid_launches++ - c->short_first;
+    GridShape g = p->gs;
+    *forced = i >= 0 && i < c->short_count && g.blocks > 1;
+    if (*forced) --g.blocks;
+    return g;
 }
 
 // A launch gave up waiting for its blocks.  Its steps go by the per-order
@@ -634,7 +635,6 @@ GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const doubl
     }
     a.epoch = p->gepoch;
     p->gepoch += signals;
-    if (signals) a.wait = grid_wait_ticks(p->ctx);
     a.sync = p->gflags.as<char>();
     a.status = reinterpret_cast<int *>(a.sync + kGridSyncBytes);
     a.A = p->phiA.p;
@@ -649,12 +649,12 @@ GridRun grid_args(qdx_prop *p, long first, long n, unsigned signals, const doubl
 }
 
 // After a launch: psi and the observables; false when it gave up waiting for its
-// blocks (psi is unchanged then).
-bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, double *obs) {
+// blocks or was made to (psi is unchanged then).
+bool grid_end(qdx_prop *p, qdx_wf *psi, const GridRun &a, double *obs, bool forced) {
     hipStream_t s = p->ctx->stream;
-    launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->ctx->report());
+    if (!forced) launch_grid_finish(s, p->S, psi->n(), p->gs, a, psi->ptr(), obs, p->ctx->report());
     HIPCHK(hipStreamSynchronize(s));
-    if (*p->ctx->report()) {
+    if (forced || *p->ctx->report()) {
         grid_missed(p);
         return false;
     }
@@ -767,18 +767,20 @@ long grid_run(qdx_prop *p, qdx_wf *psi, long first, long nsteps, const double *p
         std::copy(field0, field0 + kMaxStates * kMaxStates, a.field0);
         a.observe = obs != nullptr;
         const GridCus cus(p);
+        bool forced;
+        const GridShape g = grid_launch_shape(p, &forced);
         if (cheby) {
             KTimer t(ctx, QDX_K_CHEBY_ROW);
-            launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), p->gs, a, p0, p1, p->coef(),
+            launch_cheby_grid<R>(ctx->stream, S, dev(p->ham), g, a, p0, p1, p->coef(),
                                        p->k_launch, p->cp.offset, p->cp.offset_i, 1.0 / p->cp.scaling, p->cp.prec,
                                        p->imag, psi->ptr(), p->ctl.as<ChebyCtl>(), p->partials.as<double>());
         } else {
             KTimer t(ctx, QDX_K_GSPO_ROW);
             const HamDev<R> &h = dev(p->ops[0]);
-            launch_gspo_grid<R>(ctx->stream, S, p->gs, a, pre, fop != nullptr, coupled, p0, p1, ek, h.inv_nd[0],
+            launch_gspo_grid<R>(ctx->stream, S, g, a, pre, fop != nullptr, coupled, p0, p1, ek, h.inv_nd[0],
                                       h.inv_nd[1], psi->ptr());
         }
-        if (!grid_end(p, psi, a, obs ? obs + (size_t)i * 4 * S : nullptr)) return i;
+        if (!grid_end(p, psi, a, obs ? obs + (size_t)i * 4 * S : nullptr, forced)) return i;
         p->last_nb = p->gs.nrb;
         p->nb_init = p->gs.nrb;
         if (late) late();
@@ -1002,14 +1004,12 @@ int qdx_ctx_get_line_points(qdx_ctx *ctx, int32_t *points) {
     });
 }
 
-int qdx_ctx_set_wait_limit(qdx_ctx *ctx, int64_t us, int64_t skip, int64_t count) {
+int qdx_ctx_set_short_launches(qdx_ctx *ctx, int64_t skip, int64_t count) {
     return guarded([&] {
         if (!ctx) fail(QDX_ERR_PARAM, "ctx is NULL");
-        if (us < 0 || us > 1000000) fail(QDX_ERR_PARAM, "wait limit: 0 to 1000000 us");
         if (skip < 0 || count < 0) fail(QDX_ERR_PARAM, "negative launch count");
-        ctx->wait_us = us;
-        ctx->wait_first = ctx->grid_launches + skip;
-        ctx->wait_count = count;
+        ctx->short_first = ctx->grid_launches + skip;
+        ctx->short_count = count;
     });
 }
 
@@ -2469,15 +2469,16 @@ bool sil_grid_basis(qdx_prop *p, qdx_wf *psi, long step, std::vector<double> &al
     GridRun a = grid_args(p, step, 1, 4u * (unsigned)order + 8, nullptr, nullptr);
     const size_t nres = 2 + 2 * (size_t)order;
     std::vector<double> res(nres);
+    bool forced;
     {
         const GridCus cus(p);
-        launch_sil_grid(s, p->S, h, p->gs, a, ctx->plan_ppt(p->grid.N[0], false, 4),
+        launch_sil_grid(s, p->S, h, grid_launch_shape(p, &forced), a, ctx->plan_ppt(p->grid.N[0], false, 4),
                         ctx->plan_ppt(p->grid.N[1], false, 4), qv, order, p->dt, p->sil_err, psi->grid.weight(),
                         psi->ptr(), p->partials.as<double>(), p->ctx->report());
         HIPCHK(hipMemcpyAsync(res.data(), p->partials.p, nres * sizeof(double), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
     }
-    if (*p->ctx->report()) {
+    if (forced || *p->ctx->report()) {
         grid_missed(p);
         return false;
     }

@@ -355,10 +355,10 @@ struct qdx_ctx {
     // 0 chooses (4 on grids that give fewer than two waves per SIMD at 8)
     int line_ppt = 0;
     // persistent launches (qdx_grid.hip) so far and those that gave up waiting;
-    // qdx_ctx_set_wait_limit: the launches that take wait_us instead of the
-    // usual bound, from number wait_first on
+    // short_count of them from number short_first on come without their last
+    // block (qdx_ctx_set_short_launches)
     int64_t grid_launches = 0, grid_missed = 0;
-    int64_t wait_us = 0, wait_first = 0, wait_count = 0;
+    int64_t short_first = 0, short_count = 0;
     LinePlan plan(int L, bool fp32, const std::vector<int> &r) {
         auto &tab = fp32 ? tw32 : tw64;
         auto it = tab.find(L);

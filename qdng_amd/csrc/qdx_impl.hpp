@@ -215,7 +215,6 @@ struct GridRun {
     int part = 0;                     // GSPO: 1, 2 the parts of a single step, 0 a whole run
     bool observe = false;             // partial sums of the observables are wanted (GSPO)
     unsigned epoch = 0;               // flags reach at most epoch + 2 orders nsteps
-    unsigned wait = 0;                // bound of one wait, ticks of the 100 MHz clock (0: gives up at the first)
     char *sync = nullptr;             // flags and partial sums (kGridSyncBytes)
     int *status = nullptr;            // set by a run that gave up waiting
     void *A = nullptr, *B = nullptr;  // exchange buffers (grid_exchange_len values of the kernel precision)

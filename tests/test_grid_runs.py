@@ -289,7 +289,7 @@ def test_a_set_plan_is_used(N, kind, precision):
 
 
 def propagator(c, kind, precision="fp64", nt=12):
-    """(problem, propagator) on 40 x 24 points, a few orders per step"""
+    """(problem, propagator) on 40 x 24 points (two blocks), a few orders per step"""
     import qdng_amd as Q
     laser = kind not in ("imag", "gspo2")
     p = box(40, 24, 2 if kind == "gspo2" else 1, laser, nt=nt)
@@ -325,7 +325,7 @@ def test_launch_that_gives_up_in_a_run(kind, precision, steps, tol, skip):
             c.set_line_points(points)
             p, U = propagator(c, kind, precision, steps + 2)
             w, w0 = p.gpu_wf(c), p.gpu_wf(c)
-            c.set_wait_limit(0, skip, 1)
+            c.set_short_launches(skip, 1)
             n2, ac, nh, _ = U.run(w, 1, steps, w0)
             out.append((w.download(), np.array(n2), np.array(ac), list(nh)))
             launches, missed = c.persistent_stats()
@@ -349,7 +349,7 @@ def test_single_steps_that_give_up(kind, precision, tol):
         p, U = propagator(c, kind, precision, 80)
         _, V = propagator(d, kind, precision, 80)
         w, v = p.gpu_wf(c), p.gpu_wf(d)
-        c.set_wait_limit(0, 0, 3)
+        c.set_short_launches(0, 3)
         want = [1, 2, 3] + [3] * 64 + [4, 5]
         for i, n in enumerate(want):
             assert U.apply(w, i).n_hpsi == V.apply(v, i).n_hpsi
@@ -364,11 +364,11 @@ def test_single_steps_that_give_up(kind, precision, tol):
         d.close()
 
 
-def test_wait_limit_arguments(ctx):
+def test_short_launch_arguments(ctx):
     import qdng_amd as Q
-    for bad in [(-1, 0, 1), (1000001, 0, 1), (0, -1, 1), (0, 0, -1)]:
+    for bad in [(-1, 1), (0, -1)]:
         with pytest.raises(Q.QdxError):
-            ctx.set_wait_limit(*bad)
+            ctx.set_short_launches(*bad)
 
 
 def test_threads():
