@@ -480,9 +480,12 @@ int qdx_ctx_get_radix_plan(qdx_ctx *ctx, int32_t precision, int32_t L, int32_t *
  * transform up to rounding.  Single-state 1D lines run a whole step in one
  * block, with 4 points per thread up to 1024 points and 8 above, unless 8
  * is set.  With 0, short 1D lines (Chebyshev up to 512 points, 256 for two
- * states; split operator up to 384) and 2D grids of up to 2^19 points and
- * states (Chebyshev, split operator, short iterative Lanczos; one or two
- * states) run whole propagations in one kernel instead; 4 or 8 selects the
+ * states, 128 for three and four; split operator up to 384) and 2D grids whose
+ * rows and columns fit the CUs (Chebyshev, split operator, short iterative
+ * Lanczos; one or two states; S N0 <= 2048 and ceil(N1 / floor(2048 / (S N0)))
+ * <= the number of CUs, 256, and the same with N0 and N1 exchanged: up to 2^19
+ * values, as 512 x 512 with two states) run whole propagations in one kernel
+ * instead; 4 or 8 selects the
  * kernels above for them too, and the context's plans in the kinetic pass along
  * dimension 1, which 0 runs with a factorisation of its own where the line has
  * one.  No

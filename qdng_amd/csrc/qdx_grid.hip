@@ -1,7 +1,7 @@
 // gfx950 persistent kernels of 2D grids that fit the chip's registers: whole
 // Chebyshev and split-operator runs in one launch.
 //
-// A 2D grid of up to 2^19 points and states is bound by latency when every
+// A 2D grid of up to 2^19 points times states is bound by latency when every
 // order is two launches (row kernel and column pass): each of them reads its
 // operands back from memory, fills the chip with only two waves per SIMD and
 // drains (512 x 512 points, two states: 36 us per order in FP64, 25 in FP32;
@@ -251,6 +251,11 @@ __device__ __forceinline__ void grid_observe(const GridRun &a, int step, int st,
 // imag_time_step, OCheby.cpp:92-297): the operands, break tests and orders of
 // the per-order kernels.  partials: slots of the per-order kernels, one value
 // per row block.  NIP: negative imaginary potential (one state).
+// PRIMES: radices of primes above 7.  One instance holds the butterflies of all of
+// them, so it spills (116 to 212 bytes of scratch per lane here, 0.8 to 1.1 kB in
+// k_gspo_grid with two states); it is ahead of the per-order kernels all the same
+// (240 x 176 points: a Chebyshev order 40 -> 14 us, a split-operator step of two
+// coupled states 53 -> 23; 232 x 248: 297 -> 28 and 394 -> 38).
 template <class R, int S, bool IMAG, bool NIP, bool PRIMES>
 __global__ void __launch_bounds__(256) k_cheby_grid(GridRun a, GridShape g, HamDev<R> h, LinePlan p0, LinePlan p1,
                                                     const double *__restrict__ coef, int order, double offset,

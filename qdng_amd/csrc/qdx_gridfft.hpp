@@ -11,7 +11,9 @@
 // f are applied in registers between the two middle stages.  The inverse runs
 // on swapped real and imaginary parts, which makes it the same forward
 // butterflies.  Bound by LDS latency (one wave per SIMD: 8 reads of 16 bytes
-// take 470 cycles, the butterfly behind them 330).  Against the Stockham
+// take 470 cycles, the butterfly behind them 330; in a run on 512 x 512 points
+// vector instructions issue in 22 % of the wave cycles, and bank conflicts take
+// 0.3 cycles per LDS instruction).  Against the Stockham
 // stages of fft_line (4 points per thread, two buffers, run-time strides) the
 // filter of four 512-point lines per block went from 5.7 to 4.4 us; an order
 // of a Chebyshev series on 240 x 176 points from 29.2 to 16.5 us.

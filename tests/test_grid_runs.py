@@ -245,7 +245,7 @@ def test_against_the_oracle(N0, N1, kind):
 def test_a_set_plan_is_used(N, kind, precision):
     """A radix plan that the caller set for a side selects the kernels that
     transform by plans, as 4 or 8 line points do: here the same kernels, so the
-    same bits.  One the batch's tuning installs does not."""
+    same bits."""
     import qdng_amd as Q
     print("[gpu case] set plan", N, kind, precision, flush=True)
 
