@@ -411,8 +411,8 @@ bool dense_on(const qdx_prop *p) { return p->dense && p->ctx->line_ppt == 0; }
 // Sums over k <= N/2 of w_k cos(2 pi k d / N): the even k's part e and the odd
 // k's part o for d <= N/2.  cs: cos(2 pi q / (N stride)) at q.  The even part is
 // the same sum of half the length, and o(N/2 - d) = -o(d) leaves N/4 values of
-// it, whose terms k and N/2 - k differ by (-1)^d: N^2 / 24 products in all (512
-// points: 242 -> 73 us to create a propagator, against N^2 / 4 of them).
+// it, whose terms k and N/2 - k differ by (-1)^d: N^2 / 24 products in all (384
+// points: 335 -> 132 us to create a split operator, against N^2 / 4 of them).
 void cosine_sums(const std::vector<long double> &w, int N, const std::vector<long double> &cs, int stride,
                  std::vector<long double> &e, std::vector<long double> &o) {
     const int M = N / 2, Q = N / 4, all = (int)cs.size();
@@ -451,18 +451,15 @@ void cosine_sums(const std::vector<long double> &w, int N, const std::vector<lon
 // The circulant matrices t(i - j) = 1/N sum_k f(T_k) cos(2 pi k (i - j) / N) of
 // f(T) for every state (T_k = T_{N-k}; 0 without a kinetic term) of a 1D operator,
 // as the dense kernels read them, appended to tab: per state and parity (t(d) +-
-// t(d + N/2)) / 2 for d < N.  Summed in extended precision.
-void circulant_tables(const qdx_ham *op, const std::function<long double(double)> &f, std::vector<double> &tab) {
+// t(d + N/2)) / 2 for d < N.  Summed in extended precision, term by term (in_order)
+// or by cosine_sums; the two differ in the last bits.  The Chebyshev series are
+// summed in order: their break tests can fall within rounding of prec, and other
+// bits then end a series one order apart.
+void circulant_tables(const qdx_ham *op, const std::function<long double(double)> &f, bool in_order,
+                      std::vector<double> &tab) {
     const int N = op->grid.N[0], M = N / 2;   // N: a multiple of 8
-    std::vector<long double> cs(N), w(M + 1), e, o;
-    for (int q = 0; q <= N / 8; ++q) {
-        const long double a = 2.0L * 3.14159265358979323846264338327950288L * q / N;
-        const long double c = cosl(a), s = sinl(a);
-        for (int p : {q, N - q}) cs[p % N] = c;
-        for (int p : {M - q, M + q}) cs[p] = -c;
-        for (int p : {N / 4 - q, 3 * N / 4 + q}) cs[p] = s;
-        for (int p : {N / 4 + q, 3 * N / 4 - q}) cs[p] = -s;
-    }
+    const std::vector<long double> &cs = op->ctx->cosines(N);
+    std::vector<long double> w(M + 1), t(M + 1), e, o;
     const std::vector<double> none(N, 0.0);
     auto T = [&](int s) { return op->kin_table(s, 0) ? op->kin_table(s, 0) : none.data(); };
     for (int s = 0; s < op->S; ++s) {
@@ -473,7 +470,25 @@ void circulant_tables(const qdx_ham *op, const std::function<long double(double)
             continue;
         }
         for (int k = 0; k <= M; ++k) w[k] = f(T(s)[k]) * (k == 0 || k == M ? 1.0L : 2.0L) / N;
-        cosine_sums(w, N, cs, 1, e, o);
+        if (in_order) {
+            for (int d = 0; d <= M; ++d) {
+                long double a = 0;
+                for (int k = 0, q = 0; k <= M; ++k) {
+                    a += w[k] * cs[q];
+                    q += d;
+                    if (q >= N) q -= N;
+                }
+                t[d] = a;
+            }
+            e.resize(M + 1);
+            o.resize(M + 1);
+            for (int d = 0; d <= M; ++d) {   // t(N - d) = t(d)
+                e[d] = 0.5L * (t[d] + t[M - d]);
+                o[d] = 0.5L * (t[d] - t[M - d]);
+            }
+        } else {
+            cosine_sums(w, N, cs, 1, e, o);
+        }
         for (int d = 0; d < N; ++d) tab.push_back((double)e[d <= M ? d : N - d]);
         for (int d = 0; d < N; ++d) tab.push_back((double)o[d <= M ? d : N - d]);
     }
@@ -1548,7 +1563,7 @@ static void cheby_create_impl(qdx_ham *h, double dt, int32_t order, double prec,
                        line_lds <= 160 * 1024;
         p->dense = p->grid.nd == 1 && !p->own_plan && dense_blocks(p->grid.N[0], p->S, false) > 0;
         std::vector<double> up;   // the dense tables, then the coefficients
-        if (p->dense) circulant_tables(h, [](double T) { return (long double)T; }, up);
+        if (p->dense) circulant_tables(h, [](double T) { return (long double)T; }, true, up);
         if (p->line_step || p->dense || p->grid2d) {
             // the same products as the per-order scalars of cheby_step
             const std::complex<double> ph =
@@ -1674,8 +1689,8 @@ static void gspo_create_impl(qdx_ham *const *ops, int32_t nops, double dt, int32
             // points end 0.8 to 1.7e-14 from the exact product, with factors
             // rounded to FP64 1.3 to 3.2e-14)
             std::vector<double> t;
-            circulant_tables(p->ops[0], [&](double v) { return cosl((long double)dt * v); }, t);
-            circulant_tables(p->ops[0], [&](double v) { return -sinl((long double)dt * v); }, t);
+            circulant_tables(p->ops[0], [&](double v) { return cosl((long double)dt * v); }, false, t);
+            circulant_tables(p->ops[0], [&](double v) { return -sinl((long double)dt * v); }, false, t);
             p->dtab.alloc(t.size() * sizeof(double));
             HIPCHK(hipMemcpy(p->dtab.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         }

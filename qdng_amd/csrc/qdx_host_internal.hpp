@@ -351,6 +351,15 @@ struct qdx_ctx {
         p.ppt = 4;
         return p;
     }
+    // cos(2 pi q / N) of the dense kernels' tables, per line length (at most 512
+    // points)
+    std::map<int, std::vector<long double>> cos_tab;
+    const std::vector<long double> &cosines(int N) {
+        std::vector<long double> &c = cos_tab[N];
+        for (int q = (int)c.size(); q < N; ++q)
+            c.push_back(cosl(2.0L * 3.14159265358979323846264338327950288L * q / N));
+        return c;
+    }
     // points per thread of the single propagator's Chebyshev line kernels:
     // 0 chooses (4 on grids that give fewer than two waves per SIMD at 8)
     int line_ppt = 0;
